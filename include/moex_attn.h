@@ -23,7 +23,7 @@
  * combine instead, with a workspace of T * H * ns * 1032 bytes for their partials (ns = moex_gqa_splits(T, KV,
  * moex_decode_splits(max_t), turbo)). moex_attn_decode with ns == 1 and T <= 2 (the reference's one-split call) runs
  * the split-K kernels too, with its partials in a workspace of T * H * n2 * 1032 bytes (n2 = moex_gqa_splits(T, KV,
- * moex_decode_splits(max_t), turbo); none when n2 == 1). The dense GEMM (moex_dense.h) keeps two more. Each is one per (device, stream), allocated on first use with hipMalloc and grown
+ * moex_decode_splits(max_t), turbo); none when n2 == 1). The dense GEMM (moex_dense.h) keeps one more. Each is one per (device, stream), allocated on first use with hipMalloc and grown
  * when a larger call comes. An outgrown buffer is not freed before the process ends, because a HIP graph captured
  * earlier may still replay into it. No workspace is allocated while the stream is being captured: a call that would
  * need to grow one reports hipErrorStreamCaptureUnsupported. So after one eager call of a given max_t and T on a

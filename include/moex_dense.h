@@ -8,10 +8,10 @@
  * matrix in any of the reference's forms (int8, int4 gs64, int6 gs64, fp16). Every entry point replaces one function
  * of src/kernels.cuh, cited on its declaration, with the reference's argument order. All pointers are device pointers;
  * stream is an opaque hipStream_t (NULL = the default stream). Nothing allocates or synchronizes, except the MFMA
- * GEMM (moex_gemm_i8 with S > 8, moex_gemm when it takes the GEMM): it rounds X to fp16 into a per-(device, stream)
- * workspace of S * I * 2 bytes and, when its tile grid is short of one workgroup per CU, splits K and keeps the fp32
- * partial sums in a second one (nks * S * O * 4 bytes, nks <= 512 / tiles). Both are allocated on first use and
- * grown (after waiting for the stream) for larger sizes, kept until the process ends. Errors are reported as in
+ * GEMM (moex_gemm_i8 with S > 8, moex_gemm when it takes the GEMM): for calls whose tiles fill the chip (from some 400
+ * rows on at the attention's shapes) it rounds X to fp16 into a per-(device, stream) workspace of S * I * 2 bytes,
+ * allocated on first use, grown for larger sizes and kept until the process ends; while it cannot be had (the stream
+ * is being captured before an eager call of that size) the call runs without it, slower. Errors are reported as in
  * moex_attn.h (print and exit(1), or the soft-error slot).
  */
 #ifndef MOEX_DENSE_H

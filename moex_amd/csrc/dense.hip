@@ -11,19 +11,15 @@
 //                          sum across the wavefront, and the KS parts of a row are added in LDS. KS and the sum order
 //                          depend on O and I only, so any row of a multi-row call is bit-identical to the same row
 //                          alone.
-//   gemm_kernel            S > 8 rows (prefill): Y = X . W^T * s on v_mfma_f32_32x32x16_f16. Weights are widened to
+//   gemm_tile_kernel       S > 8 rows (prefill): Y = X . W^T * s on v_mfma_f32_16x16x32_f16. Weights are widened to
 //                          fp16 exactly (integers), activations rounded to fp16 as the reference does
-//                          (kernels.cuh:306-307), fp32 accumulation, the row scale applied last. Workgroup tile 128
-//                          weight rows x 128 tokens, 4 wavefronts of 64 x 64, K steps of 32 double-buffered in LDS,
-//                          up to three workgroups per CU; the blocks of a token tile run on one XCD (its activations
-//                          are read into one L2).
-//   gemm_ws_kernel         The same product and sum order with split roles: 4 wavefronts widen the next K step into
-//                          LDS while 4 run the MFMAs of this one. Used when the grid fits the chip in one pass.
+//                          (kernels.cuh:306-307), fp32 accumulation, the row scale applied last. One workgroup per
+//                          tile, 16 x 16 to 288 x 256 outputs, chosen so that the call's tiles fill the chip.
 //   quantize_gs64_kernel   fp16 rows -> int4 / int6 codes + a scale per 64-input group (bit-exact).
 //   gemv_mat_kernel        the GEMV of the int4 / int6 / fp16 forms: a lane per 16-weight unit of R rows, each unit
 //                          summed in order and scaled, wavefront and part sums as gemv_kernel.
-//   gemm_kernel<form>      the same tiled MFMA GEMM for every form: the staging widens int4 / int6 weights times
-//                          their group scale to fp16 (or copies fp16 weights) where int8 is widened exactly.
+//   gemm_tile_kernel<form> the same GEMM for every form: the staging widens int4 / int6 weights times their group
+//                          scale to fp16 (or copies fp16 weights) where int8 is widened exactly.
 #include <algorithm>
 #include <cstdlib>
 #include "common.hpp"
@@ -231,9 +227,6 @@ __global__ void __launch_bounds__(64 * GV_WAVES) gemv1_kernel(const int8_t* __re
 }
 
 // ---- prefill GEMM ----
-constexpr int GM_BM = 128, GM_BN = 128, GM_BK = 32;
-constexpr int GM_LD = GM_BK + 8;  // halves per LDS row (80 B: conflict-free 16-byte operand reads)
-
 // The weight forms of a dense matrix (struct Mat, kernels.cuh:186-196): int8 with a row scale, int4 and int6 with a
 // scale per 64 inputs (gs64), fp16.
 enum { MF_I8 = 0, MF_Q4 = 1, MF_Q6 = 2, MF_F16 = 3 };
@@ -253,20 +246,21 @@ struct WStage {
     uint32_t h;   // int6: the 16 high 2-bit fields
     float sc;     // int4 / int6: the group scale
 };
-template <int FMT>
-__device__ __forceinline__ void wstage_load(WStage& w, const void* W, const uint8_t* Wh, const float* s, size_t row,
-                                            int I, int k) {
+// loaded from element offset off (row * I + k) past a uniform element base, the tile's first row and K step
+template <int FMT, class off_t>
+__device__ __forceinline__ void wstage_load_at(WStage& w, const void* W, const uint8_t* Wh, const float* s, size_t base,
+                                               off_t off) {
     if constexpr (FMT == MF_I8) {
-        w.a = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(W) + row * I + k);
+        w.a = *reinterpret_cast<const uint4*>(reinterpret_cast<const int8_t*>(W) + base + off);
     } else if constexpr (FMT == MF_F16) {
-        const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(W) + row * I + k);
+        const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const uint8_t*>(W) + 2 * base + (size_t)(2 * off));
         w.a = p[0];
         w.b = p[1];
     } else {
-        const uint2 lo = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(W) + row * (I / 2) + k / 2);
+        const uint2 lo = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(W) + base / 2 + off / 2);
         w.a = make_uint4(lo.x, lo.y, 0u, 0u);
-        if constexpr (FMT == MF_Q6) w.h = *reinterpret_cast<const uint32_t*>(Wh + row * (I / 4) + k / 4);
-        w.sc = s[row * (I / 64) + k / 64];
+        if constexpr (FMT == MF_Q6) w.h = *reinterpret_cast<const uint32_t*>(Wh + base / 4 + off / 4);
+        w.sc = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(s + base / 64) + off / 64 * 4);
     }
 }
 template <int FMT>
@@ -283,10 +277,10 @@ __device__ __forceinline__ void wstage_widen(const WStage& w, bool ok, uint32_t 
         float v[16];
 #pragma unroll
         for (int e = 0; e < 16; e++) {
-            const uint32_t nib = ((e < 8 ? w.a.x : w.a.y) >> (4 * (e & 7))) & 15u;
+            const uint32_t dw = e < 8 ? w.a.x : w.a.y;
             int q;
-            if constexpr (FMT == MF_Q4) q = (int)nib - (int)((nib & 8u) << 1);       // two's complement nibble
-            else q = (int)(nib | (((w.h >> (2 * e)) & 3u) << 4)) - 32;               // 6-bit code, offset 32
+            if constexpr (FMT == MF_Q4) q = (int)__builtin_amdgcn_sbfe(dw, 4 * (e & 7), 4);  // two's complement nibble
+            else q = (int)(((dw >> (4 * (e & 7))) & 15u) | (((w.h >> (2 * e)) & 3u) << 4)) - 32;  // 6-bit code, offset 32
             v[e] = r32((float)q * w.sc);
         }
 #pragma unroll
@@ -294,99 +288,281 @@ __device__ __forceinline__ void wstage_widen(const WStage& w, bool ok, uint32_t 
     }
 }
 
-template <int FMT>
-__global__ void __launch_bounds__(256, 3) gemm_kernel(const void* __restrict__ W, const uint8_t* __restrict__ Wh,
-                                                   const float* __restrict__ s, const _Float16* __restrict__ X,
-                                                   float* __restrict__ Y, int S, int I, int O) {
-    __shared__ __align__(16) _Float16 lds[2][2][GM_BM * GM_LD];  // [buffer][W, X][row][k]
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 31, h32 = lane >> 5;
-    // XCD-aware order (block b runs on XCD b % 8): with the token tiles a multiple of 8, XCD x takes token tiles
-    // x * spx .. x * spx + spx - 1 against every weight tile, so each token tile is read into one L2 only
-    const int nO = (O + GM_BM - 1) / GM_BM, nS = (S + GM_BN - 1) / GM_BN, bid = blockIdx.x;
-    int ot, stl;
-    if (nS % 8 == 0) {
-        const int spx = nS / 8, i = bid >> 3;
-        ot = i / spx;
-        stl = (bid & 7) * spx + i % spx;
-    } else {
-        ot = bid % nO;
-        stl = bid / nO;
-    }
-    const int o0 = ot * GM_BM, s0 = stl * GM_BN;
-    const int wo = (wv >> 1) * 64, ws = (wv & 1) * 64;  // this wavefront's 64 x 64 block of the tile
-    // staging: thread tid owns 16 weights (row tid/2, k 16*(tid%2)) and 16 activations (token tid/2, same k)
-    const int sr = tid >> 1, sk = (tid & 1) * 16;
-    const bool wok = o0 + sr < O, xok = s0 + sr < S;
-    const size_t wrow = (size_t)min(o0 + sr, O - 1);
-    const _Float16* xp = X + (size_t)min(s0 + sr, S - 1) * I + sk;
-    WStage wreg;
-    uint4 xreg[2];
-    auto load = [&](int k0) {
-        wstage_load<FMT>(wreg, W, Wh, s, wrow, I, k0 + sk);
+// gemm_tile_kernel: Y = X . W^T (* s) on v_mfma_f32_16x16x32_f16, one workgroup of 8 wavefronts per tile of BM weight
+// rows x BN tokens. Wavefronts form a GM x GN x KW grid: each computes 16 WM x 16 WN outputs over the KW-th part of
+// every K step of 32 KW BKU inputs; the KW partial sums of an output are added through LDS at the end, in part order.
+// Weights go through registers, PD steps ahead, and are widened on their way into LDS (two buffers); activations the
+// same way from fp32, or (XH) rounded to fp16 once before the kernel and moved into LDS by DMA.
+//
+// What bounds it. The large tiles: LDS traffic (a 144 x 64 wavefront tile reads 13 KB per 36 MFMAs of 16 cycles, ~90 B
+// a cycle of the CU's 128, besides the staging's writes) beside the MFMAs, and the clock under MFMA load. 288 x 256
+// outputs are what 256 VGPRs and 160 KB of LDS hold, and at 2048 tokens the qkv matrix is 256 such tiles, one a CU.
+// The small tiles: the latency of a K step's loads; a tile that one CU runs alone has all of its K parts inside one
+// workgroup, so no partial sum goes through memory and no second launch adds them.
+// Measured (graph-replayed calls over rotating weights, us; before: 128 x 128 tiles on 4 wavefronts or 4 + 4 split
+// roles, an fp16 rounding launch for every call, K split over workgroups with a reduction launch), int8:
+//   tokens              9          64         300        512        1024       2048
+//   qkv  9216 x 2048    19.2->9.0  31.0->13.6 46.7->29.1 48.4->42.7 74.8->58.0 142.9->92.0 (842 TFLOPS)
+//   o    2048 x 4096    17.2->8.5  24.1->10.5 33.8->21.9 38.8->22.7 52.9->34.5  74.3->52.3 (657 TFLOPS)
+// int4 at 300 tokens: qkv 45.9 -> 31.1, o 31.7 -> 25.3; fp16 at 2048: 142.0 -> 88.1, 82.3 -> 59.9.
+template <int WM_, int WN_, int GM_, int GN_, int KW_, int BKU_, int PD_, bool XH_ = false, int WPE_ = 2>
+struct GemmTile {
+    static constexpr int WM = WM_, WN = WN_, GM = GM_, GN = GN_, KW = KW_, BKU = BKU_, PD = PD_;
+    static constexpr bool XH = XH_;
+    static constexpr int WPE = WPE_;  // wavefronts per SIMD the registers allow
+    using off_t = std::conditional_t<(16 * WM * GM * 16 * WN * GN > 256), uint32_t, size_t>;  // offsets inside a tile
+    static constexpr int BM = 16 * WM * GM, BN = 16 * WN * GN, BK = 32 * KW * BKU, LD = BK + 8, XLD = XH ? BK : LD;
+    static constexpr int STAGE = BM * LD + BN * XLD;                   // halves of a K step's operands
+    static constexpr int RED = KW > 1 ? KW * BN * (BM + 4) * 4 : 0;    // bytes of the partial sums
+    static constexpr int LDS = 2 * STAGE * 2 > RED ? 2 * STAGE * 2 : RED;
+    static constexpr int NW = (BM * (BK / 16) + 511) / 512;            // 16-weight units a thread stages
+    static constexpr int NX = XH ? 1 : (BN * (BK / 4) + 511) / 512;    // 4-activation units a thread stages
+    static constexpr int ND = BN * BK * 2 / 8192;                      // 1 KB transfers a wavefront issues (XH)
+    static_assert(GM * GN * KW == 8 && LDS <= 160 * 1024, "tile");
+    static_assert(!XH || BK <= 512, "a transfer holds whole rows of a K step");
+};
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16x(const void* base, uint32_t off, const unsigned char* lds) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
+template <int N> __device__ __forceinline__ void gemm_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+template <int FMT, class C>
+__global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(const void* __restrict__ W, const uint8_t* __restrict__ Wh,
+                                                           const float* __restrict__ s, const void* __restrict__ Xv,
+                                                           float* __restrict__ Y, int S, int I, int O, int vec) {
+    extern __shared__ __align__(16) _Float16 gl[];
+    const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nO = (O + C::BM - 1) / C::BM, nt = gridDim.x;
+    // XCD-aware order (block b runs on XCD b % 8): each XCD takes a run of tiles, weight tiles fastest, so that a token
+    // tile's activations are read into as few L2s as possible
+    const int q8 = nt >> 3, r8 = nt & 7, xc = blockIdx.x & 7, xi = blockIdx.x >> 3;
+    const int tile = (xc < r8 ? xc * (q8 + 1) : r8 * (q8 + 1) + (xc - r8) * q8) + xi;
+    const int o0 = (tile % nO) * C::BM, s0 = (tile / nO) * C::BN;
+    const int nk = I / C::BK;  // whole K steps; a ragged one follows them
+    WStage wst[C::PD][C::NW];
+    float4 xst[C::PD][C::NX];
+    constexpr int WU = C::BK / 16, XU = C::BK / 4;  // units of a row
+    // XH: transfer d of wavefront wv covers rows of the tile in 1 KB runs; lane l moves 16-byte piece sl of a row into
+    // slot l % PC (piece = slot ^ row % 8), so that the 16 rows of an operand read hit different banks
+    constexpr int PC = C::BK / 8, RPI = 64 / PC;
+    uint32_t xd[C::XH ? C::ND : 1];
+    if constexpr (C::XH) {
 #pragma unroll
-        for (int j = 0; j < 2; j++) xreg[j] = reinterpret_cast<const uint4*>(xp + k0)[j];
-    };
-    auto store = [&](int b) {
-        uint32_t h[8];
-        wstage_widen<FMT>(wreg, wok, h);
-        uint4* wd = reinterpret_cast<uint4*>(&lds[b][0][sr * GM_LD + sk]);
-        wd[0] = make_uint4(h[0], h[1], h[2], h[3]);
-        wd[1] = make_uint4(h[4], h[5], h[6], h[7]);
-        uint4* xd = reinterpret_cast<uint4*>(&lds[b][1][sr * GM_LD + sk]);
-        xd[0] = xok ? xreg[0] : make_uint4(0u, 0u, 0u, 0u);
-        xd[1] = xok ? xreg[1] : make_uint4(0u, 0u, 0u, 0u);
-    };
-    float16_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-    const int nk = I / GM_BK;
-    load(0);
-    store(0);
-    if (nk > 1) load(GM_BK);
-    __syncthreads();
-    for (int kt = 0; kt < nk; kt++) {
-        const int b = kt & 1;
-        if (kt + 1 < nk) {
-            store(b ^ 1);                                  // tile kt + 1, loaded during the previous step
-            if (kt + 2 < nk) load((kt + 2) * GM_BK);
+        for (int d = 0; d < C::ND; d++) {
+            const int r = (wv * C::ND + d) * RPI + lane / PC, sl = lane % PC;
+            xd[d] = ((uint32_t)min(r, S - 1 - s0) * I + 8 * (sl ^ (r & 7))) * 2;
         }
-        // D^T (tokens x rows per 32x32 block) = X . W^T: A = activation rows, B = weight rows, both [row][k]
-#pragma unroll
-        for (int kk = 0; kk < GM_BK; kk += 16) {
-            half8_t a[2], bw[2];
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                a[j] = *reinterpret_cast<const half8_t*>(&lds[b][1][(ws + 32 * j + r) * GM_LD + kk + 8 * h32]);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                bw[i] = *reinterpret_cast<const half8_t*>(&lds[b][0][(wo + 32 * i + r) * GM_LD + kk + 8 * h32]);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], bw[i], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
     }
-    // acc[i][j] element e: weight row wo + 32i + r (the lane's column), token ws + 32j + 8*(e/4) + 4*h32 + e%4
+    auto dma = [&](int kt, int buf) {
+        if constexpr (C::XH) {
+            const _Float16* base = reinterpret_cast<const _Float16*>(Xv) + (size_t)s0 * I + kt * C::BK;
+            const unsigned char* dst = reinterpret_cast<const unsigned char*>(gl + buf * C::STAGE + C::BM * C::LD);
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int o = o0 + wo + 32 * i + r;
-        if (o >= O) continue;
-        const float so = FMT == MF_I8 ? s[o] : 1.f;  // the group scales are in the widened weights
+            for (int d = 0; d < C::ND; d++) dma16x(base, xd[d], dst + (wv * C::ND + d) * 1024);
+        }
+    };
+    // a thread's units: offsets from the tile's first row (rows past the matrix repeat the last one: their outputs are
+    // not stored), the K step added to the uniform bases
+    typename C::off_t wro[C::NW], xro[C::NX];
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+    for (int u = 0; u < C::NW; u++) {
+        const int e = tid + 512 * u;
+        wro[u] = (typename C::off_t)min(e / WU, O - 1 - o0) * I + 16 * (e % WU);
+    }
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int t = s0 + ws + 32 * j + 8 * (e >> 2) + 4 * h32 + (e & 3);
-                if (t < S) Y[(size_t)t * O + o] = FMT == MF_I8 ? acc[i][j][e] * so : acc[i][j][e];
+    for (int u = 0; u < C::NX; u++) {
+        const int e = tid + 512 * u;
+        xro[u] = ((typename C::off_t)min(e / XU, S - 1 - s0) * I + 4 * (e % XU)) * 4;
+    }
+    auto load = [&](WStage(&w)[C::NW], float4(&x)[C::NX], int kt, auto rag) {
+        constexpr bool RAG = decltype(rag)::value;
+        const size_t wbase = (size_t)o0 * I + (size_t)kt * C::BK;
+        const char* xb = reinterpret_cast<const char*>(Xv) + ((size_t)s0 * I + (size_t)kt * C::BK) * 4;
+#pragma unroll
+        for (int u = 0; u < C::NW; u++) {
+            typename C::off_t off = wro[u];  // RAG: inputs past the row's end are read inside it, zeroed when stored
+            if (RAG) off -= max(0, kt * C::BK + 16 * ((tid + 512 * u) % WU) - (I - 16));
+            wstage_load_at<FMT>(w[u], W, Wh, s, wbase, off);
+        }
+        if constexpr (C::XH) return;
+#pragma unroll
+        for (int u = 0; u < C::NX; u++) {
+            if ((C::BN * XU) % 512 != 0 && tid + 512 * u >= C::BN * XU) break;
+            typename C::off_t off = xro[u];
+            if (RAG) off -= 4 * max(0, kt * C::BK + 4 * ((tid + 512 * u) % XU) - (I - 4));
+            x[u] = *reinterpret_cast<const float4*>(xb + off);
+        }
+    };
+    auto store = [&](const WStage(&w)[C::NW], const float4(&x)[C::NX], int kt, auto rag) {
+        constexpr bool RAG = decltype(rag)::value;
+        _Float16* b = gl + (kt & 1) * C::STAGE;
+#pragma unroll
+        for (int u = 0; u < C::NW; u++) {
+            const int e = tid + 512 * u, r = e / WU, k = 16 * (e % WU);
+            if ((C::BM * WU) % 512 != 0 && e >= C::BM * WU) break;
+            uint32_t h[8];
+            wstage_widen<FMT>(w[u], !RAG || kt * C::BK + k < I, h);
+            uint4* d = reinterpret_cast<uint4*>(b + r * C::LD + k);
+            d[0] = make_uint4(h[0], h[1], h[2], h[3]);
+            d[1] = make_uint4(h[4], h[5], h[6], h[7]);
+        }
+        if constexpr (C::XH) return;
+        b += C::BM * C::LD;
+#pragma unroll
+        for (int u = 0; u < C::NX; u++) {
+            const int e = tid + 512 * u, r = e / XU, k = 4 * (e % XU);
+            if ((C::BN * XU) % 512 != 0 && e >= C::BN * XU) break;
+            const bool ok = !RAG || kt * C::BK + k < I;
+            const float4 v = x[u];
+            *reinterpret_cast<uint2*>(b + r * C::LD + k) =
+                make_uint2(ok ? h22u(half2_t{(_Float16)v.x, (_Float16)v.y}) : 0u, ok ? h22u(half2_t{(_Float16)v.z, (_Float16)v.w}) : 0u);
+        }
+    };
+    const int kg = wv / (C::GM * C::GN), wg = wv % (C::GM * C::GN), wr = (wg / C::GN) * 16 * C::WM, wt = (wg % C::GN) * 16 * C::WN;
+    float4_t acc[C::WM][C::WN];
+#pragma unroll
+    for (int i = 0; i < C::WM; i++)
+#pragma unroll
+        for (int j = 0; j < C::WN; j++) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    auto bar = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    const _Float16* ws0 = gl + (wr + m16) * C::LD + kg * 32 * C::BKU + 8 * g;
+    const _Float16* xs0 = gl + C::BM * C::LD + (wt + m16) * C::XLD + (C::XH ? 0 : kg * 32 * C::BKU + 8 * g);
+    int xu[C::BKU];  // halves from xs0 to the operand of sub-step u
+#pragma unroll
+    for (int u = 0; u < C::BKU; u++) xu[u] = C::XH ? 8 * ((4 * (kg * C::BKU + u) + g) ^ (m16 & 7)) : 32 * u;
+    auto compute = [&](int kt) {
+        const _Float16* wb = ws0 + (kt & 1) * C::STAGE;
+        const _Float16* xb = xs0 + (kt & 1) * C::STAGE;
+#pragma unroll
+        for (int u = 0; u < C::BKU; u++) {
+            half8_t b[C::WN];
+#pragma unroll
+            for (int j = 0; j < C::WN; j++) b[j] = *reinterpret_cast<const half8_t*>(xb + 16 * j * C::XLD + xu[u]);
+#pragma unroll
+            for (int i = 0; i < C::WM; i++) {
+                const half8_t a = *reinterpret_cast<const half8_t*>(wb + 16 * i * C::LD + 32 * u);
+#pragma unroll
+                for (int j = 0; j < C::WN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[j], acc[i][j], 0, 0, 0);
             }
+        }
+    };
+    constexpr int LPU = FMT == MF_I8 ? 1 : FMT == MF_Q6 ? 3 : 2;  // loads of a weight unit
+    constexpr std::false_type whole{};
+    if (nk > 0) {
+        dma(0, 0);
+#pragma unroll
+        for (int p = 0; p < C::PD; p++) load(wst[p], xst[p], min(p, nk - 1), whole);
+        store(wst[0], xst[0], 0, whole);
+        load(wst[0], xst[0], min(C::PD, nk - 1), whole);
+        if constexpr (C::XH) gemm_vm_wait<C::NW * LPU>();
+        bar();
+    }
+    // Step kt: its operands are in buffer kt % 2; the next step's weights and activations, loaded PD steps ago, are
+    // widened into the other buffer and the registers refilled. The two wavefronts of a SIMD stage at opposite ends
+    // of the step, so that one's MFMAs run beside the other's loads and LDS writes. No condition inside: past the
+    // last step the last one is loaded and stored again, into a buffer that nobody reads.
+    auto steps = [&](auto first) {
+        for (int k0 = 0; k0 < nk; k0 += C::PD) {
+#pragma unroll
+            for (int p = 0; p < C::PD; p++) {
+                const int kt = k0 + p;
+                if (C::PD > 1 && kt >= nk) break;
+                WStage(&w)[C::NW] = wst[(p + 1) % C::PD];
+                float4(&x)[C::NX] = xst[(p + 1) % C::PD];
+                if constexpr (decltype(first)::value) {
+                    store(w, x, kt + 1, whole);
+                    dma(min(kt + 1, nk - 1), (kt + 1) & 1);
+                    load(w, x, min(kt + 1 + C::PD, nk - 1), whole);
+                    compute(kt);
+                } else {
+                    dma(min(kt + 1, nk - 1), (kt + 1) & 1);
+                    compute(kt);
+                    store(w, x, kt + 1, whole);
+                    load(w, x, min(kt + 1 + C::PD, nk - 1), whole);
+                }
+                if constexpr (C::XH) gemm_vm_wait<C::NW * LPU>();  // the step's transfers; the weight loads after them fly on
+                bar();
+            }
+        }
+    };
+    if (wv < 4) steps(std::true_type{});
+    else steps(std::false_type{});
+    if constexpr (!C::XH) {
+        if (nk * C::BK < I) {  // the ragged last step: inputs past I are zero in both operands
+            load(wst[0], xst[0], nk, std::true_type{});
+            store(wst[0], xst[0], nk, std::true_type{});
+            bar();
+            compute(nk);
+            bar();
+        }
+    }
+    // acc[i][j] element e: weight row wr + 16 i + 4 g + e, token wt + 16 j + m16
+    if constexpr (C::KW == 1) {
+#pragma unroll
+        for (int i = 0; i < C::WM; i++) {
+            const int o = o0 + wr + 16 * i + 4 * g;
+            if (o >= O) continue;
+            float sc[4] = {1.f, 1.f, 1.f, 1.f};
+            if constexpr (FMT == MF_I8) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) sc[e] = s[min(o + e, O - 1)];
+            }
+#pragma unroll
+            for (int j = 0; j < C::WN; j++) {
+                const int t = s0 + wt + 16 * j + m16;
+                if (t >= S) continue;
+                float* y = Y + (size_t)t * O + o;
+                const float4_t v = acc[i][j];
+                if (vec) {
+                    *reinterpret_cast<float4*>(y) = make_float4(v[0] * sc[0], v[1] * sc[1], v[2] * sc[2], v[3] * sc[3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (o + e < O) y[e] = v[e] * sc[e];
+                }
+            }
+        }
+    } else {
+        float* red = reinterpret_cast<float*>(gl);  // [part][token][row], rows padded by 4
+        constexpr int RL = C::BM + 4;
+#pragma unroll
+        for (int i = 0; i < C::WM; i++)
+#pragma unroll
+            for (int j = 0; j < C::WN; j++) {
+                const float4_t v = acc[i][j];
+                *reinterpret_cast<float4*>(red + ((size_t)kg * C::BN + wt + 16 * j + m16) * RL + wr + 16 * i + 4 * g) =
+                    make_float4(v[0], v[1], v[2], v[3]);
+            }
+        bar();
+        for (int e = tid; e < C::BN * (C::BM / 4); e += 512) {
+            const int tl = e / (C::BM / 4), rl = 4 * (e % (C::BM / 4)), t = s0 + tl, o = o0 + rl;
+            if (t >= S || o >= O) continue;
+            float4 a = *reinterpret_cast<const float4*>(red + (size_t)tl * RL + rl);
+#pragma unroll
+            for (int p = 1; p < C::KW; p++) {
+                const float4 b = *reinterpret_cast<const float4*>(red + ((size_t)p * C::BN + tl) * RL + rl);
+                a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+            }
+            float v[4] = {a.x, a.y, a.z, a.w};
+            if constexpr (FMT == MF_I8) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[i] *= s[min(o + i, O - 1)];
+            }
+            float* y = Y + (size_t)t * O + o;
+            if (vec) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
+            else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (o + i < O) y[i] = v[i];
+            }
+        }
     }
 }
-
 // Activations rounded to fp16 once (round to nearest even, as kernels.cuh:306-307 rounds them inside gemm_i8_k): the
 // GEMM tiles re-read them once per weight tile, so fp16 halves that traffic and takes the rounding off the staging.
 __global__ void __launch_bounds__(256) round_f16_kernel(const float4* __restrict__ X, uint2* __restrict__ Xh, size_t n4) {
@@ -395,123 +571,6 @@ __global__ void __launch_bounds__(256) round_f16_kernel(const float4* __restrict
         Xh[i] = make_uint2(h22u(half2_t{(_Float16)v.x, (_Float16)v.y}), h22u(half2_t{(_Float16)v.z, (_Float16)v.w}));
     }
 }
-
-constexpr int GEMM_WS_MAX_BLOCKS = 512;  // 2 workgroups x 256 CUs
-constexpr int GEMM_MIN_KSTEPS = 16;        // K steps of a split, at least
-
-// Sum of the K splits of gemm_ws_kernel, in split order (deterministic), times the row scale (int8; s = nullptr: none).
-__global__ void __launch_bounds__(256) gemm_reduce_kernel(const float* __restrict__ part, const float* __restrict__ s,
-                                                          float* __restrict__ Y, int S, int O, int nks) {
-    const size_t n = (size_t)S * O;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        float a = 0.f;
-        for (int k = 0; k < nks; k++) a += part[k * n + i];
-        Y[i] = s ? a * s[i % O] : a;  // no row scale for the group-scaled forms
-    }
-}
-
-// Warp-specialised variant: wavefronts 4-7 load and widen the next K step into the other LDS buffer while
-// wavefronts 0-3 run the MFMAs of this one (one barrier per K step), so the staging VALU work runs beside the MFMAs.
-template <int FMT>
-__global__ void __launch_bounds__(512, 2) gemm_ws_kernel(const void* __restrict__ W, const uint8_t* __restrict__ Wh,
-                                                         const float* __restrict__ s, const _Float16* __restrict__ X,
-                                                         float* __restrict__ Y, int S, int I, int O, int nks,
-                                                         float* __restrict__ part) {
-    __shared__ __align__(16) _Float16 lds[2][2][GM_BM * GM_LD];  // [buffer][W, X][row][k]
-    const int nO = (O + GM_BM - 1) / GM_BM, nS = (S + GM_BN - 1) / GM_BN, tiles = nO * nS;
-    const int ks = blockIdx.x / tiles, bid = blockIdx.x % tiles;  // K split ks of tile bid (nks = 1: no split)
-    const int kb = ks * (I / GM_BK) / nks, nk = (ks + 1) * (I / GM_BK) / nks - kb;
-    int ot, stl;
-    if (nS % 8 == 0) {
-        const int spx = nS / 8, i = bid >> 3;
-        ot = i / spx;
-        stl = (bid & 7) * spx + i % spx;
-    } else {
-        ot = bid % nO;
-        stl = bid / nO;
-    }
-    const int o0 = ot * GM_BM, s0 = stl * GM_BN;
-    if (threadIdx.x >= 256) {
-        // ---- staging: thread t owns 16 weights (row t/2, k 16*(t%2)) and 16 activations (token t/2, same k) ----
-        const int tid = threadIdx.x - 256, sr = tid >> 1, sk = (tid & 1) * 16;
-        const bool wok = o0 + sr < O, xok = s0 + sr < S;
-        const size_t wrow = (size_t)min(o0 + sr, O - 1);
-        const _Float16* xp = X + (size_t)min(s0 + sr, S - 1) * I + kb * GM_BK + sk;
-        WStage wreg;
-        uint4 xreg[2];
-        auto load = [&](int k0) {
-            wstage_load<FMT>(wreg, W, Wh, s, wrow, I, kb * GM_BK + k0 + sk);
-#pragma unroll
-            for (int j = 0; j < 2; j++) xreg[j] = reinterpret_cast<const uint4*>(xp + k0)[j];
-        };
-        auto store = [&](int b) {
-            uint32_t h[8];
-            wstage_widen<FMT>(wreg, wok, h);
-            uint4* wd = reinterpret_cast<uint4*>(&lds[b][0][sr * GM_LD + sk]);
-            wd[0] = make_uint4(h[0], h[1], h[2], h[3]);
-            wd[1] = make_uint4(h[4], h[5], h[6], h[7]);
-            uint4* xd = reinterpret_cast<uint4*>(&lds[b][1][sr * GM_LD + sk]);
-            xd[0] = xok ? xreg[0] : make_uint4(0u, 0u, 0u, 0u);
-            xd[1] = xok ? xreg[1] : make_uint4(0u, 0u, 0u, 0u);
-        };
-        load(0);
-        store(0);
-        if (nk > 1) load(GM_BK);
-        __syncthreads();
-        for (int kt = 0; kt < nk; kt++) {
-            if (kt + 1 < nk) {
-                store((kt + 1) & 1);  // the buffer the computing wavefronts finished at the last barrier
-                if (kt + 2 < nk) load((kt + 2) * GM_BK);
-            }
-            __syncthreads();
-        }
-        return;
-    }
-    // ---- computing wavefronts ----
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r = lane & 31, h32 = lane >> 5;
-    const int wo = (wv >> 1) * 64, ws = (wv & 1) * 64;  // this wavefront's 64 x 64 block of the tile
-    float16_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-    __syncthreads();
-    for (int kt = 0; kt < nk; kt++) {
-        const int b = kt & 1;
-#pragma unroll
-        for (int kk = 0; kk < GM_BK; kk += 16) {
-            half8_t a[2], bw[2];
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                a[j] = *reinterpret_cast<const half8_t*>(&lds[b][1][(ws + 32 * j + r) * GM_LD + kk + 8 * h32]);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-                bw[i] = *reinterpret_cast<const half8_t*>(&lds[b][0][(wo + 32 * i + r) * GM_LD + kk + 8 * h32]);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[j], bw[i], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const int o = o0 + wo + 32 * i + r;
-        if (o >= O) continue;
-        const float so = nks > 1 || FMT != MF_I8 ? 1.f : s[o];  // a K split leaves the scale to the reduction
-        float* Yo = nks > 1 ? part + (size_t)ks * S * O : Y;
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const int t = s0 + ws + 32 * j + 8 * (e >> 2) + 4 * h32 + (e & 3);
-                if (t < S) Yo[(size_t)t * O + o] = acc[i][j][e] * so;
-            }
-    }
-}
-
 
 template <int NT>
 void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, int I, int O, hipStream_t st) {
@@ -732,6 +791,101 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
     MOEX_LAUNCHED();
 }
 
+// ---- the GEMM's choice of tile ----
+// A call runs ceil(tiles / CUs) rounds of one tile per CU (the smallest tiles share a CU, at the same cost), and us0 +
+// us1 * I / 1024 is a tile's time, fitted over the qkv and o_proj shapes at 9 to 2048 tokens (int8; the other forms are
+// within 25 % of it, tile against tile closer). The XH tiles' rounding launch costs 8 us + 1.5 us per million
+// activations, so they pay where a call runs several rounds or the tile is large: qkv at 777 tokens 48.0 us with
+// 128 x 128 XH, 59.5 with the fp32-reading 128 x 128, 55.3 with 144 x 256; at 300 tokens (one round) 32.4 against 29.1.
+// The tile with the smallest estimate runs. Against every tile at 13 token counts on both shapes it was the fastest or
+// within 4 %.
+struct GemmCost { int BM, BN; bool xh; int BK; float us0, us1; };
+using GemmA = GemmTile<9, 4, 2, 4, 1, 2, 1, true>;  // 288 x 256
+using GemmB = GemmTile<9, 2, 1, 8, 1, 2, 1, true>;  // 144 x 256
+using GemmC = GemmTile<9, 2, 1, 4, 2, 1, 2>;        // 144 x 128
+using GemmD = GemmTile<4, 2, 2, 4, 1, 2, 3>;        // 128 x 128
+using GemmE = GemmTile<4, 2, 2, 4, 1, 2, 2, true>;  // 128 x 128
+using GemmF = GemmTile<4, 2, 2, 2, 2, 1, 3>;        // 128 x 64
+using GemmG = GemmTile<4, 2, 1, 2, 4, 1, 2>;        // 64 x 64
+using GemmH = GemmTile<4, 2, 1, 1, 8, 1, 2>;        // 64 x 32
+using GemmI = GemmTile<2, 2, 1, 1, 8, 1, 1, false, 4>;       // 32 x 32
+using GemmJ = GemmTile<2, 1, 1, 1, 8, 1, 2, false, 4>;       // 32 x 16
+using GemmK = GemmTile<1, 1, 1, 1, 8, 1, 2, false, 4>;       // 16 x 16
+template <class C> constexpr GemmCost gemm_cost(float us0, float us1) { return {C::BM, C::BN, C::XH, C::BK, us0, us1}; }
+constexpr GemmCost GEMM_COST[] = {
+    gemm_cost<GemmA>(10.f, 33.f), gemm_cost<GemmB>(13.f, 17.f), gemm_cost<GemmC>(17.f, 10.8f), gemm_cost<GemmD>(5.5f, 11.f),
+    gemm_cost<GemmE>(2.f, 9.f),   gemm_cost<GemmF>(3.f, 7.f),   gemm_cost<GemmG>(1.2f, 4.25f), gemm_cost<GemmH>(1.5f, 2.5f),
+    gemm_cost<GemmI>(1.f, 1.75f), gemm_cost<GemmJ>(.7f, 1.15f), gemm_cost<GemmK>(.2f, 1.f)};
+
+template <int FMT, class C>
+void launch_gemm_t(const void* W, const uint8_t* Wh, const float* s, const void* X, float* Y, int S, int I, int O,
+                   hipStream_t st) {
+    static bool once = [] {
+        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tile_kernel<FMT, C>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return true;
+    }();
+    (void)once;
+    const int tiles = ((O + C::BM - 1) / C::BM) * ((S + C::BN - 1) / C::BN);
+    const int vec = O % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;  // 16-byte output stores
+    hipLaunchKernelGGL((gemm_tile_kernel<FMT, C>), dim3(tiles), dim3(512), C::LDS, st, W, Wh, s, X, Y, S, I, O, vec);
+    MOEX_LAUNCHED();
+}
+
+int gemm_pick(int S, int I, int O, bool xh) {
+    const int cus = dense_cus();
+    int best = -1;
+    float us = 0.f;
+    for (int c = 0; c < (int)(sizeof(GEMM_COST) / sizeof(GEMM_COST[0])); c++) {
+        const GemmCost& t = GEMM_COST[c];
+        if (t.xh && (!xh || I % t.BK != 0)) continue;  // whole K steps only
+        // a tile's offsets stay within 32 bits (the smallest tile's are 64-bit)
+        if (t.BM * t.BN > 256 && (size_t)std::max(t.BM, t.BN) * I * 4 >= (size_t)1 << 32) continue;
+        const size_t tiles = (size_t)((O + t.BM - 1) / t.BM) * ((S + t.BN - 1) / t.BN);
+        const float e = (float)((tiles + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f)) +
+                        (t.xh ? 8.f + 1.5e-6f * (float)S * (float)I : 0.f);
+        if (best < 0 || e < us) {
+            best = c;
+            us = e;
+        }
+    }
+    return best;
+}
+
+template <int FMT>
+void launch_gemm(const void* W, const uint8_t* Wh, const float* s, const float* X, float* Y, int S, int I, int O,
+                 hipStream_t st) {
+    int c = gemm_pick(S, I, O, true);
+    const void* Xg = X;
+    if (GEMM_COST[c].xh) {
+        // quiet: while the workspace cannot be had (a capture before an eager call of this size, or no memory) a tile
+        // that rounds the activations itself runs
+        const size_t n4 = (size_t)S * I / 4;
+        uint2* Xh = reinterpret_cast<uint2*>(stream_workspace(n4 * 8, st, 2, true));
+        if (Xh) {
+            hipLaunchKernelGGL(round_f16_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, st,
+                               reinterpret_cast<const float4*>(X), Xh, n4);
+            MOEX_LAUNCHED();
+            Xg = Xh;
+        } else {
+            c = gemm_pick(S, I, O, false);
+        }
+    }
+    switch (c) {
+        case 0: launch_gemm_t<FMT, GemmA>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 1: launch_gemm_t<FMT, GemmB>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 2: launch_gemm_t<FMT, GemmC>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 3: launch_gemm_t<FMT, GemmD>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 4: launch_gemm_t<FMT, GemmE>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 5: launch_gemm_t<FMT, GemmF>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 6: launch_gemm_t<FMT, GemmG>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 7: launch_gemm_t<FMT, GemmH>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 8: launch_gemm_t<FMT, GemmI>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 9: launch_gemm_t<FMT, GemmJ>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        default: launch_gemm_t<FMT, GemmK>(W, Wh, s, Xg, Y, S, I, O, st); break;
+    }
+}
+
 }  // namespace
 
 void launch_quantize_rows_i8(const uint16_t* W, int8_t* q, float* s, int O, int I, hipStream_t st) {
@@ -750,40 +904,6 @@ void launch_gemv_i8(const int8_t* q, const float* s, const float* x, float* y, i
         case 7: launch_gemv_t<7>(q, s, x, y, I, O, st); break;
         default: launch_gemv_t<8>(q, s, x, y, I, O, st); break;
     }
-}
-
-void launch_gemm_i8(const int8_t* q, const float* s, const float* X, float* Y, int S, int I, int O, hipStream_t st) {
-    // Both kernels sum in the same order (identical results). A grid that fits the chip in one pass of two
-    // workgroups per CU runs the warp-specialised kernel; a larger one the 4-wavefront kernel, whose extra
-    // workgroups in flight hide the staging better than the split roles do (measured on the qkv/o_proj shapes).
-    const size_t n4 = (size_t)S * I / 4;  // I % 32 == 0
-    _Float16* Xh = reinterpret_cast<_Float16*>(stream_workspace(n4 * 8, st, 2));
-    if (!Xh) {
-        report(hipErrorOutOfMemory, __FILE__, __LINE__);
-        return;
-    }
-    hipLaunchKernelGGL(round_f16_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, st,
-                       reinterpret_cast<const float4*>(X), reinterpret_cast<uint2*>(Xh), n4);
-    MOEX_LAUNCHED();
-    const int blocks = ((O + GM_BM - 1) / GM_BM) * ((S + GM_BN - 1) / GM_BN);
-    if (blocks <= GEMM_WS_MAX_BLOCKS) {
-        // a grid short of one workgroup per CU splits K (each split at least GEMM_MIN_KSTEPS steps), summed by a
-        // second kernel; at one per CU and above, the partials' traffic cost more than the extra workgroups gained
-        int nks = 2 * blocks >= GEMM_WS_MAX_BLOCKS ? 1 : std::max(1, std::min(GEMM_WS_MAX_BLOCKS / blocks, I / GM_BK / GEMM_MIN_KSTEPS));
-        float* part = nullptr;
-        if (nks > 1) {
-            part = reinterpret_cast<float*>(stream_workspace((size_t)nks * S * O * sizeof(float), st, 3));
-            if (!part) nks = 1;
-        }
-        hipLaunchKernelGGL(gemm_ws_kernel<MF_I8>, dim3(blocks * nks), dim3(512), 0, st, q, nullptr, s, Xh, Y, S, I, O, nks,
-                           part);
-        if (nks > 1) {
-            MOEX_LAUNCHED();
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(1024), dim3(256), 0, st, part, s, Y, S, O, nks);
-        }
-    } else
-        hipLaunchKernelGGL(gemm_kernel<MF_I8>, dim3(blocks), dim3(256), 0, st, q, nullptr, s, Xh, Y, S, I, O);
-    MOEX_LAUNCHED();
 }
 
 void launch_quantize_rows_gs64(const uint16_t* W, uint8_t* q, uint8_t* qh, float* s, int O, int I, bool six,
@@ -815,45 +935,14 @@ void launch_gemv_mat(const moex_mat& m, const float* x, float* y, int NT, int I,
     }
 }
 
+void launch_gemm_i8(const int8_t* q, const float* s, const float* X, float* Y, int S, int I, int O, hipStream_t st) {
+    launch_gemm<MF_I8>(q, nullptr, s, X, Y, S, I, O, st);
+}
+
 void launch_gemm_mat(const moex_mat& m, const float* X, float* Y, int S, int I, int O, hipStream_t st) {
-    const size_t n4 = (size_t)S * I / 4;  // I % 32 == 0
-    _Float16* Xh = reinterpret_cast<_Float16*>(stream_workspace(n4 * 8, st, 2));
-    if (!Xh) {
-        report(hipErrorOutOfMemory, __FILE__, __LINE__);
-        return;
-    }
-    hipLaunchKernelGGL(round_f16_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, st,
-                       reinterpret_cast<const float4*>(X), reinterpret_cast<uint2*>(Xh), n4);
-    MOEX_LAUNCHED();
-    // the int8 GEMM's choice of kernel and K split (launch_gemm_i8); the group scales are in the widened weights, so
-    // the split's reduction applies none
-    const int blocks = ((O + GM_BM - 1) / GM_BM) * ((S + GM_BN - 1) / GM_BN);
-    const void* W = m.q4 ? static_cast<const void*>(m.q4) : m.q6 ? static_cast<const void*>(m.q6)
-                                                                 : static_cast<const void*>(m.f16);
-    const uint8_t* Wh = m.q4 ? nullptr : m.q6h;
-    const float* sg = m.q4 || m.q6 ? m.s : nullptr;
-    if (blocks <= GEMM_WS_MAX_BLOCKS) {
-        int nks = 2 * blocks >= GEMM_WS_MAX_BLOCKS ? 1 : std::max(1, std::min(GEMM_WS_MAX_BLOCKS / blocks, I / GM_BK / GEMM_MIN_KSTEPS));
-        float* part = nullptr;
-        if (nks > 1) {
-            part = reinterpret_cast<float*>(stream_workspace((size_t)nks * S * O * sizeof(float), st, 3));
-            if (!part) nks = 1;
-        }
-        if (m.q4) hipLaunchKernelGGL(gemm_ws_kernel<MF_Q4>, dim3(blocks * nks), dim3(512), 0, st, W, Wh, sg, Xh, Y, S, I, O, nks, part);
-        else if (m.q6) hipLaunchKernelGGL(gemm_ws_kernel<MF_Q6>, dim3(blocks * nks), dim3(512), 0, st, W, Wh, sg, Xh, Y, S, I, O, nks, part);
-        else hipLaunchKernelGGL(gemm_ws_kernel<MF_F16>, dim3(blocks * nks), dim3(512), 0, st, W, Wh, sg, Xh, Y, S, I, O, nks, part);
-        if (nks > 1) {
-            MOEX_LAUNCHED();
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(1024), dim3(256), 0, st, part, nullptr, Y, S, O, nks);
-        }
-    } else if (m.q4) {
-        hipLaunchKernelGGL(gemm_kernel<MF_Q4>, dim3(blocks), dim3(256), 0, st, W, Wh, sg, Xh, Y, S, I, O);
-    } else if (m.q6) {
-        hipLaunchKernelGGL(gemm_kernel<MF_Q6>, dim3(blocks), dim3(256), 0, st, W, Wh, sg, Xh, Y, S, I, O);
-    } else {
-        hipLaunchKernelGGL(gemm_kernel<MF_F16>, dim3(blocks), dim3(256), 0, st, W, Wh, sg, Xh, Y, S, I, O);
-    }
-    MOEX_LAUNCHED();
+    if (m.q4) launch_gemm<MF_Q4>(m.q4, nullptr, m.s, X, Y, S, I, O, st);
+    else if (m.q6) launch_gemm<MF_Q6>(m.q6, m.q6h, m.s, X, Y, S, I, O, st);
+    else launch_gemm<MF_F16>(m.f16, nullptr, nullptr, X, Y, S, I, O, st);
 }
 
 }  // namespace moex

@@ -180,3 +180,71 @@ def test_int8_mat_routes_to_gemm_i8():
         M.gemm_i8(q, s, x[:n], b, n, I, O)
         torch.cuda.synchronize()
         assert np.array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+
+@pytest.mark.parametrize("fmt", ["i8", "q4", "q6", "f16"])
+@pytest.mark.parametrize("O,I,S,shift", [
+    (9211, 2048, 2047, 0),   # 288 x 256 tiles, ragged in both directions, O % 4 != 0 (4-byte stores)
+    (9212, 1024, 1021, 0),   # 144 x 256
+    (9217, 512, 509, 0),     # 144 x 128
+    (2049, 4096, 1531, 1),   # 128 x 128, output 4 bytes off a 16-byte boundary
+    (9215, 2048, 770, 0),    # 128 x 128, fp16 activations
+    (2048, 1088, 650, 0),    # 128 x 64; I % 128 != 0
+    (2050, 4096, 400, 0),    # 64 x 64
+    (2048, 4160, 161, 1),    # 64 x 32, a ragged last K step (I % 256 = 64)
+    (2047, 320, 65, 0),      # 32 x 32, K steps 1.25
+    (9216, 192, 17, 0),      # 32 x 16, I below one K step
+    (33, 64, 11, 0),         # 16 x 16, the smallest I of the group-scaled forms
+])
+def test_gemm_tiles(fmt, O, I, S, shift):
+    """Every tile of the GEMM at its edges (the tile is chosen by size; the comments name it): ragged O and S, a last K
+    step shorter than the tile's, outputs that only 4-byte stores can write. Against the precision model of the GEMM;
+    its fp32 sums of up to 4160 products of random sign differ from the exact ones by ~1e-6 of the largest output, and
+    no value outside [S][O] is written."""
+    import torch
+    import moex_amd as M
+    rng = np.random.default_rng(O + I + S)
+    w = (rng.standard_normal((O, I)) * 0.02).astype(np.float16)
+    if fmt == "i8":
+        q = torch.empty((O, I), dtype=torch.int8, device="cuda")
+        s = torch.empty(O, dtype=torch.float32, device="cuda")
+        M.quantize_rows_i8(dev(w.view(np.int16)), q, s, O, I)
+        torch.cuda.synchronize()
+        m, hq, hs, _keep = M.Mat(q=q, s=s), q.cpu().numpy(), s.cpu().numpy(), (q, s)
+    else:
+        m, (hw, hh, hs), F, _keep = _make(fmt, w)
+    x = rng.standard_normal((S, I)).astype(np.float32)
+    buf = torch.full((shift + S * O + 64,), float("nan"), dtype=torch.float32, device="cuda")
+    Y = buf[shift:shift + S * O]
+    M.gemm(m, dev(x), Y, S, I, O)
+    torch.cuda.synchronize()
+    got = Y.cpu().numpy().reshape(S, O)
+    rows = sorted({0, 15, 16, S // 2, S - 2, S - 1} & set(range(S)))
+    cols = np.unique(np.r_[0:O:max(1, O // 128), max(0, O - 20):O])
+    if fmt == "i8":
+        model = orc.dense_i8_fp16x(hq[cols], hs[cols], x[rows])
+    else:
+        model = orc.dense_mat_fp16x(F, hw[cols], None if hh is None else hh[cols], None if hs is None else hs[cols], x[rows])
+    rel = _rel(got[np.ix_(rows, cols)].astype(np.float64), model)
+    report("gemm tiles", fmt=fmt, O=O, I=I, S=S, rel=rel)
+    assert np.all(np.isfinite(got)) and rel < 1e-5
+    assert torch.isnan(buf[shift + S * O:]).all() and torch.isnan(buf[:shift]).all()
+
+
+@pytest.mark.parametrize("I", [32, 96, 2080])
+def test_gemm_odd_inputs(I):
+    """I a multiple of 32 but not of 64 (int8 and fp16 only), below, above and at a K step's remainder."""
+    import torch
+    import moex_amd as M
+    rng = np.random.default_rng(I)
+    for O, S in ((130, 9), (2048, 300), (4608, 1100)):
+        w = (rng.standard_normal((O, I)) * 0.02).astype(np.float16)
+        m, (hw, _, _), F, _keep = _make("f16", w)
+        x = rng.standard_normal((S, I)).astype(np.float32)
+        Y = torch.full((S, O), float("nan"), dtype=torch.float32, device="cuda")
+        M.gemm(m, dev(x), Y, S, I, O)
+        torch.cuda.synchronize()
+        got = Y.cpu().numpy()
+        rows, cols = [0, S // 2, S - 1], np.arange(0, O, max(1, O // 100))
+        assert np.all(np.isfinite(got))
+        assert _rel(got[np.ix_(rows, cols)].astype(np.float64), orc.dense_mat_fp16x(F, hw[cols], None, None, x[rows])) < 1e-5

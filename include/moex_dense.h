@@ -71,7 +71,7 @@ void moex_gemv(const moex_mat* m, const float* x, float* y, int I, int O, void* 
 /* gemm(m, X, Y, S, I, O, st) (kernels.cuh:339-369): Y [S][O] = X [S][I] . W^T with the reference's choice of path:
  *   int8: moex_gemm_i8;
  *   int6 with S <= 8: one GEMV pass for all S rows, each row bit-identical to moex_gemv of that row;
- *   int4 and fp16 with S <= 2: moex_gemv row by row;
+ *   int4 and fp16 with S <= 2: moex_gemv of each row (the same bits; two rows in one pass over the weights);
  *   otherwise the fp16 MFMA GEMM: activations rounded to fp16, int4 / int6 weights times their group scale rounded
  *   to fp16 (fp16 weights as stored), fp32 accumulation (gemm_wmma_k :225-248, gemm_i8_k<true> :250-337).
  * The GEMM takes the per-stream workspaces of moex_gemm_i8 (see the top of this file). */

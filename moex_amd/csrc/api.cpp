@@ -174,7 +174,7 @@ void moex_gemm(const moex_mat* m, const float* X, float* Y, int S_, int I, int O
         launch_gemv_mat(*m, X, Y, S_, I, O, S(stream));
         return;
     }
-    if (S_ <= 2) {  // :358-362: the GEMV row by row
+    if (S_ <= 2) {  // :358-362: the GEMV of each row
         launch_gemv_mat(*m, X, Y, S_, I, O, S(stream));
         return;
     }

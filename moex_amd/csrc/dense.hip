@@ -4,13 +4,12 @@
 // gemv_q4_k / gemv_q6_k / gemv_f16_k, gemm_wmma_k, gemm_i8_k<true>: kernels.cuh:68-93,225-337,486-590).
 //
 //   quantize_rows_kernel   fp16 [O][I] -> int8 [O][I] + scale absmax/127 per row (bit-exact: IEEE divide, rint).
-//   gemv_kernel<NT>        y[t][o] = s[o] * sum_i q[o][i] x[t][i] for NT <= 8 rows of x, fp32 sums. HBM-bound on the
-//                          weights, which are read once for all NT rows. The NT input rows sit in LDS; a wavefront
-//                          takes 8 weight rows over 1/KS of I, its lanes walking it in 16-byte chunks (1 KB contiguous
-//                          per row and instruction, 16 KB per wavefront issued before any product), reduces each
-//                          sum across the wavefront, and the KS parts of a row are added in LDS. KS and the sum order
-//                          depend on O and I only, so any row of a multi-row call is bit-identical to the same row
-//                          alone.
+//   gemv1_kernel<NT, R>    y[t][o] = s[o] * sum_i q[o][i] x[t][i] for NT <= 8 rows of x, fp32 sums. HBM-bound on the
+//                          weights, which are read once for all NT rows. A wavefront takes R weight rows over 1/KS of
+//                          I, a lane 16 weights of each, sums them in order and over the wavefront, and the KS parts
+//                          of a row are added in LDS. KS and the sum order depend on O and I only, so any row of a
+//                          multi-row call is bit-identical to the same row alone.
+//   gemv_kernel<NT>        The same for parts of more than 64 16-weight chunks, which a lane walks in steps.
 //   gemm_tile_kernel       S > 8 rows (prefill): Y = X . W^T * s on v_mfma_f32_16x16x32_f16. Weights are widened to
 //                          fp16 exactly (integers), activations rounded to fp16 as the reference does
 //                          (kernels.cuh:306-307), fp32 accumulation, the row scale applied last. One workgroup per
@@ -28,21 +27,55 @@ namespace moex {
 
 namespace {
 
-// sum over the wavefront, every lane receives it: DPP within each 16-lane row (rotate by 8 and 4, then the quad
-// swaps), then the 16- and 32-lane swaps (v_permlane16/32_swap). All VALU: the ds_bpermute round trips of __shfl_xor
-// were most of a GEMV's time after its loads had landed (o_proj, 2 rows: 9.0 -> 6.2 us without them)
+// sum over the wavefront, every lane receives it: the 32- and 16-lane swaps (v_permlane32/16_swap), then DPP within each
+// 16-lane row (rotate by 8 and 4, then the quad swaps). All VALU: the ds_bpermute round trips of __shfl_xor were most
+// of a GEMV's time after its loads had landed (o_proj, 2 rows: 9.0 -> 6.2 us without them)
 template <int CTRL> __device__ __forceinline__ float dpp_f(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
 }
 __device__ __forceinline__ float wave_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
     v += dpp_f<0x128>(v);  // row_ror:8
     v += dpp_f<0x124>(v);  // row_ror:4
     v += dpp_f<0x4e>(v);   // quad_perm [2, 3, 0, 1]
-    v += dpp_f<0xb1>(v);   // quad_perm [1, 0, 3, 2]
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    return v + dpp_f<0xb1>(v);  // quad_perm [1, 0, 3, 2]
+}
+// N values summed over the wavefront together: the 32- and 16-lane swaps each fold two values into one register (a pair
+// of values costs one swap and one add instead of two of each), then DPP within the 16-lane rows. On return v[k] holds,
+// in all lanes of row q = lane / 16, the sum of value wave_sums_index(k, q). The tree over the lanes is the same for
+// every N and value (lanes 32 apart, 16, 8, 4, 2, 1).
+template <int N> __device__ __forceinline__ void wave_sums(float (&v)[N]) {
+    constexpr int H = (N + 1) / 2, Q = (H + 1) / 2;
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[k]), __float_as_uint(k + H < N ? v[k + H] : v[k]),
+                                                        false, false);
+        v[k] = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < Q; k++) {
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[k]), __float_as_uint(k + Q < H ? v[k + Q] : v[k]),
+                                                        false, false);
+        v[k] = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < Q; k++) {
+        v[k] += dpp_f<0x128>(v[k]);
+        v[k] += dpp_f<0x124>(v[k]);
+        v[k] += dpp_f<0x4e>(v[k]);
+        v[k] += dpp_f<0xb1>(v[k]);
+    }
+}
+// the value whose sum v[k] holds in row q, or N if none (its lanes hold a copy of another)
+template <int N> __device__ __forceinline__ int wave_sums_index(int k, int q) {
+    constexpr int H = (N + 1) / 2, Q = (H + 1) / 2;
+    const int h = k + ((q & 1) ? Q : 0);
+    if ((q & 1) && h >= H) return N;
+    const int i = h + ((q & 2) ? H : 0);
+    return i < N ? i : N;
 }
 
 __global__ void __launch_bounds__(256) quantize_rows_kernel(const uint16_t* __restrict__ W, int8_t* __restrict__ q,
@@ -62,6 +95,17 @@ __global__ void __launch_bounds__(256) quantize_rows_kernel(const uint16_t* __re
     if (threadIdx.x == 0) s[row] = sc;
 }
 
+// A transfer of 16 bytes a lane from base + off (uniform base, 32-bit byte offset) to lds + 16 * lane, in inline asm: the
+// compiler cannot tell which LDS bytes it writes and would make the next LDS read wait for every load in flight. The
+// kernels wait for their own transfers.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16x(const void* base, uint32_t off, const unsigned char* lds) {
+    const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int GV_R = 8;       // weight rows of a row group
 // 16-byte chunks per lane and row loaded before any is used: 16 KB per wavefront in flight, 8 KB from NT = 5 on
@@ -147,82 +191,99 @@ __global__ void __launch_bounds__(64 * GV_WAVES) gemv_kernel(const int8_t* __res
 #undef GV_LOAD
 }
 
-// The same product when every wavefront has at most one row group and one load step (rounds = 1, a part of at most
-// 64 * GV_U chunks: the attention's qkv and o shapes). Without loops every load goes out at the start; each lane reads
-// its inputs straight from L2, so the products wait only for their own rows. Same sum order as gemv_kernel.
+// The same product when a part of a row is at most 64 chunks, one load a lane (the attention's qkv and o shapes): a
+// wavefront takes R rows, sends all of its loads before any product and needs no loop. Same sum order as gemv_kernel.
+// It is bound by the weight stream and the launch for few input rows, by the FMAs (and the widening, once per group of
+// 4 input rows) for many. One or two input rows are read by each lane straight from L2; more are copied into LDS once
+// per workgroup by DMA (float4 e of the rows in slot e ^ (e / 8) % 4: the lanes of a read, 64 bytes apart, then hit
+// different banks), as eight wavefronts each reading 4 or 8 rows from L2 took longer than the weights, and their
+// values left no registers for the weights in flight. Graph-replayed over rotating weights, us, before -> now (before:
+// every input row from L2, 8 rows a wavefront, qkv's rows not split, six cross-lane steps per sum):
+//   input rows          1           2           3            4            6            8
+//   qkv  9216 x 2048    7.0 -> 5.2  8.7 -> 6.0  12.3 -> 6.6  21.0 -> 7.7  16.3 -> 9.2  20.9 -> 10.6
+//   o    2048 x 4096    4.2 -> 3.9  4.8 -> 4.9  5.4 -> 4.8   6.2 -> 5.1   7.7 -> 6.1   9.3 -> 6.7
 template <int NT, int R>
-__global__ void __launch_bounds__(64 * GV_WAVES) gemv1_kernel(const int8_t* __restrict__ q, const float* __restrict__ s,
-                                                              const float* __restrict__ x, float* __restrict__ y, int I,
-                                                              int O, int KS) {
-    constexpr int GV_U = gv_u<NT>();
-    extern __shared__ __align__(16) float red[];  // the partial sums [GV_WAVES][NT][R] (R weight rows a group)
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nb = gridDim.x;
-    const int ngroups = (O + R - 1) / R;
-    const int part = wv % KS, slice = I / 16 / KS, cb = part * slice, ce = cb + slice;
-    const int g = blockIdx.x + nb * (wv / KS);
-    const bool on = g < ngroups;
-    // the lane's 16 inputs of each row of x first (read from L2 by every wavefront of this part; no LDS copy and no
-    // barrier before the products), then the weights, so the products of the first weight rows start while the
-    // later rows are still arriving
-    float4 xv[GV_U][NT][4];
-#pragma unroll
-    for (int u = 0; u < GV_U; u++) {
-        if (cb + 64 * u >= ce) continue;  // a step past the part (wave-uniform): nothing to load
-        const int c = min(cb + 64 * u + lane, I / 16 - 1);
+__global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* __restrict__ q, const float* __restrict__ s,
+                                                                 const float* __restrict__ x, float* __restrict__ y,
+                                                                 int I, int O, int KS) {
+    constexpr bool XL = NT > 2;
+    extern __shared__ __align__(16) float xs[];  // XL: the input rows [NT][I]; then the partial sums [GV_WAVES][NT * R]
+    float* red = xs + (XL ? NT * I : 0);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ngroups = (O + R - 1) / R, gpw = GV_WAVES / KS;
+    const int part = wv % KS, slice = I / 16 / KS, cb = part * slice;
+    const int g = blockIdx.x * gpw + wv / KS;
+    const bool on = lane < slice;
+    const int c = min(cb + lane, I / 16 - 1);
+    constexpr int TB = NT < 4 ? NT : 4;
+    float4 xv[TB][4];
+    if constexpr (XL) {
+        const int n = NT * I / 256;  // 1 KB transfers
+        for (int i = wv; i < n; i += GV_WAVES) {
+            const uint32_t e = 64 * i + lane;
+            dma16x(x, 16 * (e ^ ((e >> 3) & 3)), reinterpret_cast<const unsigned char*>(xs) + 1024 * i);
+        }
+    } else {
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int d = 0; d < 4; d++) xv[u][t][d] = reinterpret_cast<const float4*>(x + (size_t)t * I)[4 * c + d];
+            for (int d = 0; d < 4; d++) xv[t][d] = reinterpret_cast<const float4*>(x + (size_t)t * I)[4 * c + d];
     }
-    u32x4 w[GV_U][R];
+    u32x4 w[R];
 #pragma unroll
-    for (int u = 0; u < GV_U; u++)
+    for (int r = 0; r < R; r++)  // rows past the last repeat it
+        w[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q + (size_t)min(g * R + r, O - 1) * I) + c);
+    // XL: this wavefront's transfers have landed when only its R weight loads are in flight
+    if constexpr (XL) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(R) : "memory");
+    float acc[NT * R];
+#pragma unroll
+    for (int t0 = 0; t0 < NT; t0 += TB) {  // input rows in groups whose values fit the registers
+        if constexpr (XL) {
+#pragma unroll
+            for (int t = t0; t < NT && t < t0 + TB; t++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const uint32_t e = t * (I / 4) + 4 * c + d;
+                    xv[t - t0][d] = reinterpret_cast<const float4*>(xs)[e ^ ((e >> 3) & 3)];
+                }
+        }
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const u32x4* row = reinterpret_cast<const u32x4*>(q + (size_t)min(min(g, ngroups - 1) * R + r, O - 1) * I);
-            const int c = cb + 64 * u + lane;
-            w[u][r] = on && c < ce ? __builtin_nontemporal_load(row + c) : u32x4{0u, 0u, 0u, 0u};
-        }
-    // the row scale of this lane's output, loaded now so that its round trip overlaps the weights'
-    const float so = s[min(min(g, ngroups - 1) * R + lane % R, O - 1)];
-    float acc[NT][R];
+            float a[TB];
 #pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int r = 0; r < R; r++) acc[t][r] = 0.f;
-#pragma unroll
-    for (int u = 0; u < GV_U; u++) {
-        const int c = cb + 64 * u + lane;
-        if (c >= ce) continue;
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
+            for (int t = 0; t < TB; t++) a[t] = 0.f;
 #pragma unroll
             for (int d = 0; d < 4; d++) {
-                const float4 xq = xv[u][t][d];
+                const uint32_t wd = w[r][d];
+                const float w0 = (float)(int8_t)wd, w1 = (float)(int8_t)(wd >> 8), w2 = (float)(int8_t)(wd >> 16),
+                            w3 = (float)(int8_t)(wd >> 24);
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const uint32_t wd = w[u][r][d];
-                    acc[t][r] += (float)(int8_t)(wd) * xq.x;
-                    acc[t][r] += (float)(int8_t)(wd >> 8) * xq.y;
-                    acc[t][r] += (float)(int8_t)(wd >> 16) * xq.z;
-                    acc[t][r] += (float)(int8_t)(wd >> 24) * xq.w;
+                for (int t = 0; t < TB && t0 + t < NT; t++) {
+                    a[t] = fmaf(w0, xv[t][d].x, a[t]);
+                    a[t] = fmaf(w1, xv[t][d].y, a[t]);
+                    a[t] = fmaf(w2, xv[t][d].z, a[t]);
+                    a[t] = fmaf(w3, xv[t][d].w, a[t]);
                 }
             }
+#pragma unroll
+            for (int t = 0; t < TB && t0 + t < NT; t++) acc[(t0 + t) * R + r] = on ? a[t] : 0.f;
         }
+        if constexpr (NT > TB) asm volatile("" ::: "memory");  // the next group's values are read after these are used
     }
+    wave_sums(acc);
 #pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const float v = wave_sum(acc[t][r]);
-            if (lane == 0) red[(wv * NT + t) * R + r] = v;
-        }
+    for (int k = 0; k < ((NT * R + 1) / 2 + 1) / 2; k++) {
+        const int i = wave_sums_index<NT * R>(k, lane >> 4);
+        if ((lane & 15) == 0 && i < NT * R) red[wv * NT * R + i] = acc[k];
+    }
     __syncthreads();
-    if (on && part == 0 && lane < NT * R) {
-        const int t = lane / R, r = lane % R, o = g * R + r;
-        float v = red[(wv * NT + t) * R + r];
-        for (int p = 1; p < KS; p++) v += red[((wv + p) * NT + t) * R + r];
-        if (o < O) y[(size_t)t * O + o] = v * so;
+    const int rows = gpw * R;  // of this workgroup
+    for (int e = tid; e < NT * rows; e += 64 * GV_WAVES) {
+        const int t = e / rows, rr = e % rows, gl = rr / R, r = rr % R, o = (blockIdx.x * gpw + gl) * R + r;
+        if (o >= O) continue;
+        float v = red[gl * KS * NT * R + t * R + r];
+        for (int p = 1; p < KS; p++) v += red[(gl * KS + p) * NT * R + t * R + r];
+        y[(size_t)t * O + o] = v * s[o];
     }
 }
 
@@ -321,14 +382,6 @@ struct GemmTile {
     static_assert(GM * GN * KW == 8 && LDS <= 160 * 1024, "tile");
     static_assert(!XH || BK <= 512, "a transfer holds whole rows of a K step");
 };
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16x(const void* base, uint32_t off, const unsigned char* lds) {
-    const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
 template <int N> __device__ __forceinline__ void gemm_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 template <int FMT, class C>
 __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(const void* __restrict__ W, const uint8_t* __restrict__ Wh,
@@ -572,6 +625,45 @@ __global__ void __launch_bounds__(256) round_f16_kernel(const float4* __restrict
     }
 }
 
+template <int NT, int R>
+bool launch_gemv1_r(const int8_t* q, const float* s, const float* x, float* y, int I, int O, int ks, hipStream_t st) {
+    const size_t lds = (NT > 2 ? (size_t)NT * I * 4 : 0) + (size_t)GV_WAVES * NT * R * 4;
+    if (lds > 160 * 1024 || (NT > 2 && (reinterpret_cast<uintptr_t>(x) & 15))) return false;  // 16-byte transfers
+    static bool once = [] {
+        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv1_kernel<NT, R>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return true;
+    }();
+    (void)once;
+    const int gpw = GV_WAVES / ks, wgs = ((O + R - 1) / R + gpw - 1) / gpw;
+    hipLaunchKernelGGL((gemv1_kernel<NT, R>), dim3(wgs), dim3(64 * GV_WAVES), lds, st, q, s, x, y, I, O, ks);
+    MOEX_LAUNCHED();
+    return true;
+}
+template <int NT>
+bool launch_gemv1(const int8_t* q, const float* s, const float* x, float* y, int I, int O, int ks, int cus,
+                  hipStream_t st) {
+    // the rows per wavefront with the cheapest rounds over the chip: R rows and a fixed part of about two rows' time each.
+    // Of 2, 3, 4, 6, 9 and 12 it was the fastest or within 12 % of it for 1 to 8 input rows on qkv (9) and o_proj (4)
+    int best = 0;
+    long cost = 0;
+    for (int R : {2, 3, 4, 6, 9, 12}) {
+        const long gpw = GV_WAVES / ks, wgs = ((O + R - 1) / R + gpw - 1) / gpw, e = (wgs + cus - 1) / cus * (R + 2);
+        if (!best || e < cost) {
+            best = R;
+            cost = e;
+        }
+    }
+    switch (best) {
+        case 2: return launch_gemv1_r<NT, 2>(q, s, x, y, I, O, ks, st);
+        case 3: return launch_gemv1_r<NT, 3>(q, s, x, y, I, O, ks, st);
+        case 4: return launch_gemv1_r<NT, 4>(q, s, x, y, I, O, ks, st);
+        case 6: return launch_gemv1_r<NT, 6>(q, s, x, y, I, O, ks, st);
+        case 9: return launch_gemv1_r<NT, 9>(q, s, x, y, I, O, ks, st);
+        default: return launch_gemv1_r<NT, 12>(q, s, x, y, I, O, ks, st);
+    }
+}
+
 template <int NT>
 void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, int I, int O, hipStream_t st) {
     static bool once = [] {
@@ -581,8 +673,8 @@ void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, in
     }();
     (void)once;
     const int groups = (O + GV_R - 1) / GV_R;
-    int ks = 1;  // split each row over up to 8 wavefronts until ~4 wavefronts per CU have work
-    while (ks < GV_WAVES && groups * ks < 1024 && (I / 16) % (128 * ks) == 0) ks *= 2;
+    int ks = 1;  // split each row over up to 8 wavefronts until 8 wavefronts per CU have 8 rows each
+    while (ks < GV_WAVES && groups * ks < 2048 && (I / 16) % (128 * ks) == 0) ks *= 2;
     static const int cus = [] {
         int dev = 0, v = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
@@ -590,21 +682,10 @@ void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, in
             return v;
         return 256;
     }();
+    if (I / 16 / ks <= 64 && launch_gemv1<NT>(q, s, x, y, I, O, ks, cus, st)) return;
     const int nb = std::min(cus, groups * ks);
     const size_t lds = (size_t)NT * I * 4 + GV_WAVES * NT * GV_R * 4;
-    const bool one = groups <= nb * (GV_WAVES / ks) && I / 16 / ks <= 64 * gv_u<NT>();
-    if (one) {
-        // groups of 4 rows when groups of 8 would leave half the wavefronts without work (o_proj): every wavefront
-        // then has work, half as much, and the sums are the same (a row's sum order does not depend on the group)
-        if ((O + 3) / 4 * ks <= nb * GV_WAVES && groups * ks * 2 <= nb * GV_WAVES)
-            hipLaunchKernelGGL((gemv1_kernel<NT, 4>), dim3(nb), dim3(64 * GV_WAVES), (size_t)GV_WAVES * NT * 4 * 4, st,
-                               q, s, x, y, I, O, ks);
-        else
-            hipLaunchKernelGGL((gemv1_kernel<NT, GV_R>), dim3(nb), dim3(64 * GV_WAVES), (size_t)GV_WAVES * NT * GV_R * 4,
-                               st, q, s, x, y, I, O, ks);
-    } else {
-        hipLaunchKernelGGL(gemv_kernel<NT>, dim3(nb), dim3(64 * GV_WAVES), lds, st, q, s, x, y, I, O, ks);
-    }
+    hipLaunchKernelGGL(gemv_kernel<NT>, dim3(nb), dim3(64 * GV_WAVES), lds, st, q, s, x, y, I, O, ks);
     MOEX_LAUNCHED();
 }
 
@@ -915,8 +996,8 @@ void launch_quantize_rows_gs64(const uint16_t* W, uint8_t* q, uint8_t* qh, float
 
 void launch_gemv_mat(const moex_mat& m, const float* x, float* y, int NT, int I, int O, hipStream_t st) {
     if (m.q4) {
-        for (int t = 0; t < NT; t++)
-            launch_gemv_mat_t<MF_Q4, 1>(m.q4, nullptr, m.s, x + (size_t)t * I, y + (size_t)t * O, I, O, st);
+        if (NT == 2) launch_gemv_mat_t<MF_Q4, 2>(m.q4, nullptr, m.s, x, y, I, O, st);  // the rows' own bits, one pass
+        else launch_gemv_mat_t<MF_Q4, 1>(m.q4, nullptr, m.s, x, y, I, O, st);
     } else if (m.q6) {
         switch (NT) {
             case 1: launch_gemv_mat_t<MF_Q6, 1>(m.q6, m.q6h, m.s, x, y, I, O, st); break;
@@ -930,8 +1011,8 @@ void launch_gemv_mat(const moex_mat& m, const float* x, float* y, int NT, int I,
         }
     } else {
         const uint8_t* W = reinterpret_cast<const uint8_t*>(m.f16);
-        for (int t = 0; t < NT; t++)
-            launch_gemv_mat_t<MF_F16, 1>(W, nullptr, nullptr, x + (size_t)t * I, y + (size_t)t * O, I, O, st);
+        if (NT == 2) launch_gemv_mat_t<MF_F16, 2>(W, nullptr, nullptr, x, y, I, O, st);
+        else launch_gemv_mat_t<MF_F16, 1>(W, nullptr, nullptr, x, y, I, O, st);
     }
 }
 

@@ -180,3 +180,32 @@ def test_many_row_groups():
     got = Y.cpu().numpy()
     assert _rel(got.astype(np.float64), orc.dense_i8_f64(qh, sh, x)) < 1e-5
     assert np.array_equal(got[1], y1.cpu().numpy())
+
+
+@pytest.mark.parametrize("O,I,shift", [
+    (1001, 512, 0),    # half of a part's lanes idle, O not a multiple of any row group
+    (12301, 2048, 0),  # more row groups than one round of workgroups
+    (700, 1536, 0),    # parts of more than 64 chunks: the looped kernel
+    (9216, 1024, 1),   # input rows 4 bytes off a 16-byte boundary: no transfers into LDS
+    (130, 8192, 0),    # the most parts a row is split in
+])
+def test_gemv_rows_split(O, I, shift):
+    """Every path of the int8 GEMV at 1 to 8 rows: each row the bits of the one-row call, and within 1e-5 of the exact
+    product."""
+    import torch
+    import moex_amd as M
+    rng = np.random.default_rng(O + I)
+    q, s = _quantize((rng.standard_normal((O, I)) * 0.02).astype(np.float16))
+    buf = torch.zeros(8 * I + shift, dtype=torch.float32, device="cuda")
+    x = rng.standard_normal((8, I)).astype(np.float32)
+    xd = buf[shift:]
+    xd.copy_(dev(x).reshape(-1))
+    one = torch.full((8, O), float("nan"), dtype=torch.float32, device="cuda")
+    for t in range(8):
+        M.gemv_i8(q, s, xd[t * I:], one[t], I, O)
+    for S in range(2, 9):
+        Y = torch.full((S, O), float("nan"), dtype=torch.float32, device="cuda")
+        M.gemm_i8(q, s, xd, Y, S, I, O)
+        torch.cuda.synchronize()
+        assert torch.equal(Y, one[:S]), S
+    assert _rel(one.cpu().numpy().astype(np.float64), orc.dense_i8_f64(q.cpu().numpy(), s.cpu().numpy(), x)) < 1e-5

@@ -248,3 +248,21 @@ def test_gemm_odd_inputs(I):
         rows, cols = [0, S // 2, S - 1], np.arange(0, O, max(1, O // 100))
         assert np.all(np.isfinite(got))
         assert _rel(got[np.ix_(rows, cols)].astype(np.float64), orc.dense_mat_fp16x(F, hw[cols], None, None, x[rows])) < 1e-5
+
+
+@pytest.mark.parametrize("fmt", ["q4", "f16"])
+def test_two_rows_equal_gemv(shape, fmt):
+    """int4 and fp16 with two rows (one pass over the weights): each row the bits of the one-row GEMV."""
+    import torch
+    import moex_amd as M
+    O, I = shape
+    rng = np.random.default_rng(O)
+    m, _, _, _keep = _make(fmt, (rng.standard_normal((O, I)) * 0.02).astype(np.float16))
+    xd = dev(rng.standard_normal((2, I)).astype(np.float32))
+    Y = torch.full((2, O), float("nan"), dtype=torch.float32, device="cuda")
+    M.gemm(m, xd, Y, 2, I, O)
+    Yr = torch.full_like(Y, float("nan"))
+    for t in range(2):
+        M.gemv(m, xd[t], Yr[t], I, O)
+    torch.cuda.synchronize()
+    assert torch.equal(Y, Yr)

@@ -158,8 +158,8 @@ constexpr int ring_stage() { return 2 * CH * AHD + 2 * CH * 4; }
 
 // chunk c of the ring into stage c % NS (the producers' transfers of it)
 template <int CH, int NS>
-__device__ __forceinline__ void ring_issue(unsigned char* smem, const moex_kv_cache& kv, size_t rbase, int pw, int lane,
-                                           int lo, int first, int c) {
+__device__ __forceinline__ void ring_issue(unsigned char* smem, const moex_kv_cache& kv, size_t rbase, int max_t, int pw,
+                                           int lane, int lo, int first, int c) {
     static_assert((CH == 64 || CH == 128) && NS >= 2 && NS <= 4, "ring shape");
     constexpr int KB = CH * AHD, STAGE = ring_stage<CH>(), NI = CH / 8;
     constexpr bool SC_ALL = CH == 128;
@@ -170,11 +170,26 @@ __device__ __forceinline__ void ring_issue(unsigned char* smem, const moex_kv_ca
     const int c0 = c == 0 ? lo : lo + first + (c - 1) * CH, ce = c == 0 ? lo + first : lo + first + c * CH;
     unsigned char* st = smem + (c % NS) * STAGE;
     unsigned char* sb = st + (pw < 2 ? 0 : KB);
+    // instruction i covers rows 4i .. 4i+3; row r's piece p in slot p ^ (r % 16) (K) or p ^ 4 ((r / 4) % 4) (V)
+    if (c0 + CH <= max_t) {
+        // every row of a whole chunk lies in the cache: a uniform base and four lane offsets, no address arithmetic a
+        // transfer (it shares the SIMD with a consumer: 2 tokens over 40 000 keys 18.7 -> 17.3 us). Rows past ce (a
+        // short chunk 0) are the rows that follow: their scores are masked, their P is 0 (their scales are not moved)
+        uint32_t off[4];
 #pragma unroll
-    for (int u = 0; u < NI; u++) {
-        const int i = NI * (pw & 1) + u, r = 4 * i + r4;  // instruction i covers rows 4i .. 4i+3
-        const int piece = pw < 2 ? sl ^ (r & 15) : sl ^ (4 * (i & 3));
-        dma16(src + (size_t)min(c0 + r, ce - 1) * AHD + 16 * piece, sb + i * 1024);
+        for (int j = 0; j < 4; j++) off[j] = r4 * AHD + 16 * (pw < 2 ? sl ^ (4 * j + r4) : sl ^ (4 * j));
+#pragma unroll
+        for (int u = 0; u < NI; u++) {
+            const int i = NI * (pw & 1) + u;
+            dma16s(src + (size_t)c0 * AHD + i * 1024, off[u & 3], sb + i * 1024);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < NI; u++) {
+            const int i = NI * (pw & 1) + u, r = 4 * i + r4;
+            const int piece = pw < 2 ? sl ^ (r & 15) : sl ^ (4 * (i & 3));
+            dma16(src + (size_t)min(c0 + r, ce - 1) * AHD + 16 * piece, sb + i * 1024);
+        }
     }
     if (sc) {
         const int k0 = SC_ALL ? 64 * (pw & 1) : 0;
@@ -183,21 +198,21 @@ __device__ __forceinline__ void ring_issue(unsigned char* smem, const moex_kv_ca
 }
 // the first NS - 1 chunks
 template <int CH, int NS>
-__device__ __forceinline__ void ring_first(unsigned char* smem, const moex_kv_cache& kv, size_t rbase, int pw, int lane,
+__device__ __forceinline__ void ring_first(unsigned char* smem, const moex_kv_cache& kv, size_t rbase, int max_t, int pw, int lane,
                                            int lo, int first, int nch) {
-    for (int c = 0; c < NS - 1 && c < nch; c++) ring_issue<CH, NS>(smem, kv, rbase, pw, lane, lo, first, c);
+    for (int c = 0; c < NS - 1 && c < nch; c++) ring_issue<CH, NS>(smem, kv, rbase, max_t, pw, lane, lo, first, c);
 }
 // issued: the first chunks went out already (ring_first). ppos >= 0: the cache row at position ppos was just formed
 // by this workgroup (patch: K row, V row, ks, vs in LDS) and may not have reached memory when its chunk was moved; the
 // producer that moved each part of that row overwrites it in the stage once the chunk has landed.
 template <int CH, int NS>
-__device__ __forceinline__ void ring_producer(unsigned char* smem, const moex_kv_cache& kv, size_t rbase, int pw,
+__device__ __forceinline__ void ring_producer(unsigned char* smem, const moex_kv_cache& kv, size_t rbase, int max_t, int pw,
                                               int lane, int lo, int first, int nch, bool issued = false, int ppos = -1,
                                               const unsigned char* patch = nullptr) {
     constexpr int KB = CH * AHD, STAGE = ring_stage<CH>(), NI = CH / 8;
     constexpr bool SC_ALL = CH == 128;
     const bool sc = SC_ALL || !(pw & 1);
-    if (!issued) ring_first<CH, NS>(smem, kv, rbase, pw, lane, lo, first, nch);
+    if (!issued) ring_first<CH, NS>(smem, kv, rbase, max_t, pw, lane, lo, first, nch);
     for (int c = 0; c < nch; c++) {
         // chunk c has landed when at most the chunks issued after it are in flight (NI or NI + 1 instructions each)
         const int after = min(nch - 1 - c, NS - 2);
@@ -218,7 +233,7 @@ __device__ __forceinline__ void ring_producer(unsigned char* smem, const moex_kv
                     reinterpret_cast<const float*>(patch + 2 * AHD)[pw < 2 ? 0 : 1];
         }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (c + NS - 1 < nch) ring_issue<CH, NS>(smem, kv, rbase, pw, lane, lo, first, c + NS - 1);
+        if (c + NS - 1 < nch) ring_issue<CH, NS>(smem, kv, rbase, max_t, pw, lane, lo, first, c + NS - 1);
     }
     __syncthreads();
     __syncthreads();
@@ -272,7 +287,7 @@ __global__ void __launch_bounds__(64 * (WS_NC + WS_NP), 1) gqa_ws1_kernel(const 
     // the consumers form it, two query heads each (and wavefront 0 the new row), and the chunks go out once the
     // consumers have issued all of their row reads (a barrier between the two), so those reads are not queued behind
     // ~25 MB of chunk transfers while the front's arithmetic runs beside the chunks' flight
-    if (wv >= WS_NC && !fused) ring_first<W1_CH, W1_NS>(smem, kv, rbase, wv - WS_NC, lane, lo, first, nch);
+    if (wv >= WS_NC && !fused) ring_first<W1_CH, W1_NS>(smem, kv, rbase, max_t, __builtin_amdgcn_readfirstlane(wv - WS_NC), lane, lo, first, nch);
     const bool app = fused && hi == Tmax && hi > lo;  // this split holds the new row pos0
     const float* qtab = reinterpret_cast<const float*>(smem + W1_QO);
     unsigned char* patch = smem + W1_PT;
@@ -292,16 +307,19 @@ __global__ void __launch_bounds__(64 * (WS_NC + WS_NP), 1) gqa_ws1_kernel(const 
         }
         asm volatile("s_barrier" ::: "memory");  // the consumers' row reads are issued
         if (wv >= WS_NC) {
-            ring_first<W1_CH, W1_NS>(smem, kv, rbase, wv - WS_NC, lane, lo, first, nch);
+            ring_first<W1_CH, W1_NS>(smem, kv, rbase, max_t, __builtin_amdgcn_readfirstlane(wv - WS_NC), lane, lo, first, nch);
         } else {
             // ---- the front (front::wave: the arithmetic of qk_norm_rope_kernel): consumer w forms query heads
             // 2w, 2w + 1; in the split that holds pos0, consumer 0 also forms the key row and the int8 codes of the
-            // new row, which go to the cache and to the patch ----
+            // new row, which go to the cache and to the patch. The RoPE angles, once for the rows, while those fly ----
+            int ln = lane;
+            asm volatile("" : "+v"(ln));  // not before the barrier, which the first chunks wait for
+            const front::wave::Rope rp = front::wave::rope_angles(ln, pos0, fr.rot, fr.theta);
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const int h = 2 * wv + j;
                 float x[4] = {qa[j].x, qa[j].y, qa[j].z, qa[j].w};
-                front::wave::norm_rope(x, wq, lane, pos0, fr.rot, fr.theta, fr.eps);
+                front::wave::norm_rope(x, wq, lane, rp, fr.rot, fr.eps);
                 const float4 y = make_float4(x[0], x[1], x[2], x[3]);
                 *reinterpret_cast<float4*>(smem + W1_QO + 4 * (h * AHD + 4 * lane)) = y;
                 if (s == 0) *reinterpret_cast<float4*>(fr.qo + (kvh * GQ + h) * AHD + 4 * lane) = y;
@@ -309,7 +327,7 @@ __global__ void __launch_bounds__(64 * (WS_NC + WS_NP), 1) gqa_ws1_kernel(const 
             if (app && wv == 0) {
                 float x[4] = {ka.x, ka.y, ka.z, ka.w};
                 const float vv[4] = {va.x, va.y, va.z, va.w};
-                front::wave::norm_rope(x, wk, lane, pos0, fr.rot, fr.theta, fr.eps);
+                front::wave::norm_rope(x, wk, lane, rp, fr.rot, fr.eps);
                 uint32_t ck, cv;
                 float sk, sv;
                 front::wave::quant_i8(x, vv, ck, cv, sk, sv);
@@ -330,7 +348,7 @@ __global__ void __launch_bounds__(64 * (WS_NC + WS_NP), 1) gqa_ws1_kernel(const 
     }
 
     if (wv >= WS_NC) {
-        ring_producer<W1_CH, W1_NS>(smem, kv, rbase, wv - WS_NC, lane, lo, first, nch, true, app ? pos0 : -1, patch);
+        ring_producer<W1_CH, W1_NS>(smem, kv, rbase, max_t, __builtin_amdgcn_readfirstlane(wv - WS_NC), lane, lo, first, nch, true, app ? pos0 : -1, patch);
     } else {
         // ---- consumers. The query digits, once per workgroup: consumer w turns heads 2w, 2w + 1 (lane l: head
         // 2w + l / 32, dims 8 (l % 32) .. + 7) into three signed base-256 digits of a 2^(22 - e) fixed point (|q| < 2^e
@@ -604,11 +622,13 @@ __global__ void __launch_bounds__(64 * (WS_NC + WS_NP), 1) gqa_wsp_kernel(const 
         }
         asm volatile("s_barrier" ::: "memory");  // the consumers' row reads are issued
         if (wv >= WS_NC) {
-            if (!late) ring_first<CH, NS>(smem, kv, rbase, wv - WS_NC, lane, lo, first, nch);
+            if (!late) ring_first<CH, NS>(smem, kv, rbase, max_t, __builtin_amdgcn_readfirstlane(wv - WS_NC), lane, lo, first, nch);
         } else {
             float* qt = reinterpret_cast<float*>(smem + (NS - 1) * STAGE);
             if (qrows) {
-                const front::wave::Rope rp = front::wave::rope_angles(lane, pos0 + t, fr.rot, fr.theta);
+                int ln = lane;
+                asm volatile("" : "+v"(ln));  // not before the barrier, which the first chunks wait for
+                const front::wave::Rope rp = front::wave::rope_angles(ln, pos0 + t, fr.rot, fr.theta);
 #pragma unroll
                 for (int j = 0; j < HP; j++) {
                     const int h = h0 + j;
@@ -628,10 +648,10 @@ __global__ void __launch_bounds__(64 * (WS_NC + WS_NP), 1) gqa_wsp_kernel(const 
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the new rows are in memory
         }
         front::sync<true>();
-        if (wv >= WS_NC && late) ring_first<CH, NS>(smem, kv, rbase, wv - WS_NC, lane, lo, first, nch);
+        if (wv >= WS_NC && late) ring_first<CH, NS>(smem, kv, rbase, max_t, __builtin_amdgcn_readfirstlane(wv - WS_NC), lane, lo, first, nch);
     }
     if (wv >= WS_NC) {
-        ring_producer<CH, NS>(smem, kv, rbase, wv - WS_NC, lane, lo, first, nch, fused);
+        ring_producer<CH, NS>(smem, kv, rbase, max_t, __builtin_amdgcn_readfirstlane(wv - WS_NC), lane, lo, first, nch, fused);
     } else {
         const int pr = wv % NPR;                                        // token pair
         const bool live = 2 * pr < ntok;
@@ -979,7 +999,13 @@ __global__ void __launch_bounds__(64 * WT_NW, 1) gqa_wst_kernel(const float* __r
     __shared__ float cm[WT_NW][GQ], cl[WT_NW][GQ];
     const int nb = gridDim.x, w_id = xcd_work_id(blockIdx.x, nb);
     const int tok = w_id % T, s = (w_id / T) % ns, kvh = w_id / (T * ns);
-    const int pos0 = *pos_d, Tmax = pos0 + T;
+    // the RoPE frequencies need only the arguments: formed while the position, which the splits follow from, is read
+    front::wave::RopeFreq rf = {0.f, 0.f};
+    if (fr.q) rf = front::wave::rope_freq(threadIdx.x & 63, fr.rot, fr.theta);
+    int pos0 = *pos_d;
+    asm volatile("" : "+v"(rf.a), "+v"(rf.b));
+    asm volatile("" : "+s"(pos0));  // used only from here on
+    const int Tmax = pos0 + T;
     const int L = (Tmax + ns - 1) / ns, lo = s * L;
     const int hi = min(pos0 + tok + 1, lo + L);  // keys [lo, hi) of this split that the token sees
     const int nch = hi > lo ? (hi - lo + WT_CH - 1) / WT_CH : 0;
@@ -1081,8 +1107,10 @@ __global__ void __launch_bounds__(64 * WT_NW, 1) gqa_wst_kernel(const float* __r
     if (fused) {
         const float4 a =
             *reinterpret_cast<const float4*>(fr.q + (size_t)tok * fr.ld + (kvh * GQ + wv) * 2 * AHD + 4 * lane);
+        const uint2 wq = *reinterpret_cast<const uint2*>(fr.qn + 4 * lane);
+        const front::wave::Rope rp = front::wave::rope_angles(rf, lane, pos0 + tok, fr.rot);  // while the row flies
         qf4[0] = a.x; qf4[1] = a.y; qf4[2] = a.z; qf4[3] = a.w;
-        front::wave::norm_rope(qf4, fr.qn, lane, pos0 + tok, fr.rot, fr.theta, fr.eps);
+        front::wave::norm_rope(qf4, wq, lane, rp, fr.rot, fr.eps);
         front::wave::wht(qf4, 0, lane);
         if (s == 0)
             *reinterpret_cast<float4*>(fr.qo + ((size_t)tok * H + kvh * GQ + wv) * AHD + 4 * lane) =
@@ -1093,7 +1121,8 @@ __global__ void __launch_bounds__(64 * WT_NW, 1) gqa_wst_kernel(const float* __r
             const float4 v4 = *reinterpret_cast<const float4*>(fr.v + o);
             float x[4] = {k4.x, k4.y, k4.z, k4.w};
             const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
-            front::wave::norm_rope(x, fr.kn, lane, na + wv, fr.rot, fr.theta, fr.eps);
+            const uint2 wk = *reinterpret_cast<const uint2*>(fr.kn + 4 * lane);
+            front::wave::norm_rope(x, wk, lane, front::wave::rope_angles(rf, lane, na + wv, fr.rot), fr.rot, fr.eps);
             front::wave::append(x, vv, kv, rbase + na + wv, lane);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
@@ -1278,10 +1307,16 @@ __global__ void __launch_bounds__(64 * WT_NW, 1) gqa_wst_kernel(const float* __r
     __syncthreads();  // every wavefront is past its last step: the rings are free
     float* Ow = reinterpret_cast<float*>(smem);  // [wavefront][head][256]
     const float un = ldexpf(1.f, -sig);
+    // lanes l, l + 32 hold the hi and lo rows: one swap folds tiles J and J + 8 (V halves 0 and 1) into one register,
+    // half 0's sums in the lower lanes and half 1's in the upper ones
 #pragma unroll
-    for (int J = 0; J < 16; J++)
+    for (int J = 0; J < 8; J++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) o[J][i] += __shfl_xor(o[J][i], 32);  // lanes l, l + 32: the hi and lo rows
+        for (int i = 0; i < 4; i++) {
+            const auto r =
+                __builtin_amdgcn_permlane32_swap(__float_as_uint(o[J][i]), __float_as_uint(o[J + 8][i]), false, false);
+            o[J][i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
     float b0[4], b1[4];  // row 4g + i is head 4 (g & 1) + i: its sums from lane 16 i (all lanes take part)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -1290,25 +1325,21 @@ __global__ void __launch_bounds__(64 * WT_NW, 1) gqa_wst_kernel(const float* __r
         b0[i] = (g & 1) ? c0 : a0;
         b1[i] = (g & 1) ? c1 : a1;
     }
-    if (g < 2) {
+    const int hf = g >> 1;  // this lane's V half
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int h = 4 * g + i;
-            float Mh = cm[0][h];
+    for (int i = 0; i < 4; i++) {
+        const int h = 4 * (g & 1) + i;
+        float Mh = cm[0][h];
 #pragma unroll
-            for (int w = 1; w < WT_NW; w++) Mh = fmaxf(Mh, cm[w][h]);
-            const float f = ex2d(cm[wv][h], Mh) * un;
+        for (int w = 1; w < WT_NW; w++) Mh = fmaxf(Mh, cm[w][h]);
+        const float f = ex2d(cm[wv][h], Mh) * un;
+        const float b = hf ? b1[i] : b0[i];
+        float* dst = Ow + (wv * GQ + h) * AHD + 128 * hf + 8 * m16;
+        float r[8];
 #pragma unroll
-            for (int hf = 0; hf < 2; hf++) {
-                const float b = hf ? b1[i] : b0[i];
-                float* dst = Ow + (wv * GQ + h) * AHD + 128 * hf + 8 * m16;
-                float r[8];
-#pragma unroll
-                for (int k = 0; k < 8; k++) r[k] = fmaf(o[8 * hf + k][i], 16777216.f, -b) * f;
-                *reinterpret_cast<float4*>(dst) = make_float4(r[0], r[1], r[2], r[3]);
-                *reinterpret_cast<float4*>(dst + 4) = make_float4(r[4], r[5], r[6], r[7]);
-            }
-        }
+        for (int k = 0; k < 8; k++) r[k] = fmaf(o[k][i], 16777216.f, -b) * f;
+        *reinterpret_cast<float4*>(dst) = make_float4(r[0], r[1], r[2], r[3]);
+        *reinterpret_cast<float4*>(dst + 4) = make_float4(r[4], r[5], r[6], r[7]);
     }
     __syncthreads();
     float* Om = reinterpret_cast<float*>(smem) + WT_NW * GQ * AHD;  // [head][256]: the merged acc, when rotating back
@@ -1344,12 +1375,18 @@ __global__ void __launch_bounds__(64 * WT_NW, 1) gqa_wst_kernel(const float* __r
         for (int b = 0; b < 2; b++) {
             float v0 = sgn(WS2, lane, Om[h * AHD + 128 * b + lane]);
             float v1 = sgn(WS2, lane + 64, Om[h * AHD + 128 * b + 64 + lane]);
-#pragma unroll
-            for (int st = 1; st < 64; st <<= 1) {
-                const float o0 = __shfl_xor(v0, st), o1 = __shfl_xor(v1, st);
-                v0 = (lane & st) ? o0 - v0 : v0 + o0;
-                v1 = (lane & st) ? o1 - v1 : v1 + o1;
-            }
+            v0 = front::wave::butterfly<1>(v0, lane);
+            v1 = front::wave::butterfly<1>(v1, lane);
+            v0 = front::wave::butterfly<2>(v0, lane);
+            v1 = front::wave::butterfly<2>(v1, lane);
+            v0 = front::wave::butterfly<4>(v0, lane);
+            v1 = front::wave::butterfly<4>(v1, lane);
+            v0 = front::wave::butterfly<8>(v0, lane);
+            v1 = front::wave::butterfly<8>(v1, lane);
+            v0 = front::wave::butterfly<16>(v0, lane);
+            v1 = front::wave::butterfly<16>(v1, lane);
+            v0 = front::wave::butterfly<32>(v0, lane);
+            v1 = front::wave::butterfly<32>(v1, lane);
             const float a0 = v0 + v1, a1 = v0 - v1;
             dst[128 * b + lane] = sgn(WS1, lane, a0 * 0.08838834764831845f);
             dst[128 * b + 64 + lane] = sgn(WS1, lane + 64, a1 * 0.08838834764831845f);

@@ -256,13 +256,53 @@ __device__ __forceinline__ void append_turbo(float x, float vv, moex_kv_cache kv
 // its xor tree pairs dims d and d ^ 16, ^ 8, ^ 4 across lanes (lane ^ 4, ^ 2, ^ 1) and d ^ 2, d ^ 1 inside the lane.
 namespace wave {
 
+// x of lane ^ M, by VALU moves: DPP inside a row of 16 lanes, the row swaps beyond. (A __shfl_xor is a ds_bpermute, a
+// round trip through LDS; a head row of the front has 12 of them in its norm and 20 more in its WHT. With the moves,
+// and the RoPE angles formed while the rows are being read, whole attn_decode steps, graph-replayed: 700 keys int8 10.8
+// -> 9.1 us, turbo 15.8 -> 13.0, 4 tokens 15.6 -> 14.2; 262144 keys turbo 43.3 -> 40.5.)
+template <int CTRL> __device__ __forceinline__ float dpp_mov(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+template <int M> __device__ __forceinline__ float lane_xor(float x) {
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a row of 16 lanes");
+    if (M == 1) return dpp_mov<0xb1>(x);                  // quad_perm [1, 0, 3, 2]
+    if (M == 2) return dpp_mov<0x4e>(x);                  // quad_perm [2, 3, 0, 1]
+    if (M == 4) return dpp_mov<0x1b>(dpp_mov<0x141>(x));  // row_half_mirror (lane ^ 7), then quad_perm [3, 2, 1, 0] (^ 3)
+    return dpp_mov<0x128>(x);                             // row_ror:8
+}
+// {x of the even one, x of the odd one} of the rows (halves) that lane and lane ^ 16 (lane ^ 32) lie in
+struct Pair {
+    float even, odd;
+};
+__device__ __forceinline__ Pair pair16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ Pair pair32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+// one butterfly stage over lanes M apart: x + partner in the lane with bit M clear, partner - x in the other
+template <int M> __device__ __forceinline__ float butterfly(float x, int lane) {
+#pragma clang fp contract(off)
+    if constexpr (M < 16) {
+        const float o = lane_xor<M>(x);
+        return o + ((lane & M) ? -x : x);
+    } else {
+        const Pair p = M == 16 ? pair16(x) : pair32(x);
+        return p.even + ((lane & M) ? -p.odd : p.odd);
+    }
+}
+
 // every dim gets its reference warp's sum (the 32-lane xor tree: offsets 16, 8, 4, 2, 1)
 __device__ __forceinline__ void sum32(float (&v)[4]) {
 #pragma clang fp contract(off)
 #pragma unroll
-    for (int o = 4; o >= 1; o >>= 1)
+    for (int i = 0; i < 4; i++) v[i] += lane_xor<4>(v[i]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] += __shfl_xor(v[i], o);
+    for (int i = 0; i < 4; i++) v[i] += lane_xor<2>(v[i]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] += lane_xor<1>(v[i]);
     float a[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) a[i] = v[i] + v[i ^ 2];
@@ -293,9 +333,14 @@ __device__ __forceinline__ float half_sum(float (&v)[4], int lane) {
 }
 __device__ __forceinline__ float row_max(const float (&v)[4]) {
     float m = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    return m;
+    Pair p = pair32(m);
+    m = fmaxf(p.even, p.odd);
+    p = pair16(m);
+    m = fmaxf(p.even, p.odd);
+    m = fmaxf(m, lane_xor<8>(m));
+    m = fmaxf(m, lane_xor<4>(m));
+    m = fmaxf(m, lane_xor<2>(m));
+    return fmaxf(m, lane_xor<1>(m));
 }
 
 // The RoPE factors of the lane's 4 dims at one position: they depend on the position and the dim only, so the rows
@@ -303,32 +348,41 @@ __device__ __forceinline__ float row_max(const float (&v)[4]) {
 struct Rope {
     float cs[4], sn[4];
 };
-__device__ __forceinline__ Rope rope_angles(int lane, int pos, int rot, float theta) {
+// the angles depend on j = d mod rot / 2 only: lane t holds the frequencies of j = t and t + 64 (the same expression as the
+// 256-thread function). They need no position: a decode kernel forms them while its position is being read
+struct RopeFreq {
+    float a, b;
+};
+__device__ __forceinline__ RopeFreq rope_freq(int lane, int rot, float theta) {
+#pragma clang fp contract(off)
+    const int h2 = rot / 2;
+    RopeFreq f = {0.f, 0.f};
+    if (lane < h2) f.a = powf(theta, -2.f * lane / rot);
+    if (h2 > 64 && lane + 64 < h2) f.b = powf(theta, -2.f * (lane + 64) / rot);
+    return f;
+}
+__device__ __forceinline__ Rope rope_angles(RopeFreq f, int lane, int pos, int rot) {
 #pragma clang fp contract(off)
     const int h2 = rot / 2, d0 = 4 * lane;
-    // the angles depend on j = d mod h2 only: lane t computes those of j = t and t + 64 (the same expression as the
-    // 256-thread function), the rotating lanes take theirs by shuffle
     float ca = 1.f, sa = 0.f, cb = 1.f, sb = 0.f;
-    if (lane < h2) {
-        const float ang = (float)pos * powf(theta, -2.f * lane / rot);
-        ca = cosf(ang);
-        sa = sinf(ang);
-    }
-    if (lane + 64 < h2) {
-        const float ang = (float)pos * powf(theta, -2.f * (lane + 64) / rot);
-        cb = cosf(ang);
-        sb = sinf(ang);
-    }
+    if (lane < h2) sincosf((float)pos * f.a, &sa, &ca);
+    if (h2 > 64 && lane + 64 < h2) sincosf((float)pos * f.b, &sb, &cb);
     Rope rp;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int d = d0 + i, j = d < h2 ? d : d - h2;
-        const float c0 = __shfl(ca, j & 63), c1 = __shfl(cb, j & 63);  // every lane takes part in every shuffle
-        const float s0 = __shfl(sa, j & 63), s1 = __shfl(sb, j & 63);
-        rp.cs[i] = j < 64 ? c0 : c1;
-        rp.sn[i] = j < 64 ? s0 : s1;
+        rp.cs[i] = __shfl(ca, j & 63);  // every lane takes part in every shuffle
+        rp.sn[i] = __shfl(sa, j & 63);
+        if (h2 > 64) {  // wave-uniform
+            const float c1 = __shfl(cb, j & 63), s1 = __shfl(sb, j & 63);
+            rp.cs[i] = j < 64 ? rp.cs[i] : c1;
+            rp.sn[i] = j < 64 ? rp.sn[i] : s1;
+        }
     }
     return rp;
+}
+__device__ __forceinline__ Rope rope_angles(int lane, int pos, int rot, float theta) {
+    return rope_angles(rope_freq(lane, rot, theta), lane, pos, rot);
 }
 // norm_rope on the lane's 4 dims (rot % 8 == 0: a RoPE partner is 4 dims per lane away, same slot); wb: the lane's 4
 // fp16 norm weights (w + 4 lane), loaded by the caller. In two steps: the RMSNorm(1 + w) and the partner values,
@@ -344,6 +398,11 @@ __device__ __forceinline__ void norm_partner(float (&x)[4], float (&px)[4], uint
 #pragma unroll
     for (int i = 0; i < 4; i++) x[i] = x[i] * r * (1.f + (float)__builtin_bit_cast(_Float16, wh[i]));
     const int h2 = rot / 2, d0 = 4 * lane;
+    if (rot == 64) {  // wave-uniform: the partners of the 16 rotating lanes are 8 lanes apart
+#pragma unroll
+        for (int i = 0; i < 4; i++) px[i] = lane_xor<8>(x[i]);
+        return;
+    }
     const int partner = d0 < h2 ? lane + h2 / 4 : lane - h2 / 4;
 #pragma unroll
     for (int i = 0; i < 4; i++) px[i] = __shfl(x[i], partner & 63);
@@ -390,13 +449,15 @@ __device__ __forceinline__ void wht(float (&x)[4], int dir, int lane) {
         for (int i = 0; i < 4; i++) v[i] = a[i];
     }
 #pragma unroll
-    for (int h = 4; h <= 64; h <<= 1) {  // stages 4 .. 64: lane ^ h / 4
+    for (int i = 0; i < 4; i++) v[i] = butterfly<1>(v[i], lane);  // stages 4 .. 64: lane ^ h / 4
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float o = __shfl_xor(v[i], h / 4);
-            v[i] = ((4 * lane) & h) ? o - v[i] : v[i] + o;
-        }
-    }
+    for (int i = 0; i < 4; i++) v[i] = butterfly<2>(v[i], lane);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = butterfly<4>(v[i], lane);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = butterfly<8>(v[i], lane);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = butterfly<16>(v[i], lane);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int j = (4 * lane + i) & 127;

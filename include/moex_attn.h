@@ -12,7 +12,7 @@
  *
  * Workspaces. moex_attn_fa widens the K/V tiles once into a tile-image workspace of KV * ceil(max_t / 32) * 37632
  * bytes (MOEX_FA_IMAGES=0: none, the kernel widens each tile itself, same results, slower). A chunk whose token
- * tiles leave the chip underfilled (KV * ceil(T / 16) < CUs) may split each token tile's keys over several
+ * tiles leave the chip underfilled (2 * KV * ceil(T / 16) <= CUs) may split each token tile's keys over several
  * workgroups, with a second workspace for their partial results, T * H * pieces * 1040 bytes (at most 32 pieces;
  * MOEX_FA_SPLIT=n caps them, 1 turns splitting off). A chunk whose token tiles fill the chip once (KV * ceil(T / 16)
  * <= CUs, not split, e.g. 2048 tokens) runs its token tiles in heavy/light pairs on two workgroups each, the heavy

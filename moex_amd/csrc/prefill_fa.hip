@@ -242,23 +242,68 @@ __device__ __forceinline__ bool map_block(int b, int KV, int NT, int& kvh, int& 
     return kvh < KV;
 }
 // Key pieces of token tile t (keys [0, pos0 + min(FT (t + 1), T))), for chunks whose token tiles leave the chip
-// underfilled (KV x tiles < CUs; the host then passes nsf > 1). Computed on the device (pos0 is a device value), the
-// same way by the FA kernel and the merge: a tile of n key tiles takes floor(n / w) pieces (1 to nsf), w = the chip's
-// average share of the work, so the pieces of all tiles fill the chip about once; w is at least
-// max(FA_MINW, 2 x token tiles), as each workgroup first loads its queries (more of them for a longer chunk) and
-// each piece adds merge traffic. Piece s is tiles [s n / ns, (s + 1) n / ns): at least w >= 8 tiles, so its first key
-// is below every row of the token tile (each row sees a key in every piece).
+// underfilled (the host then passes nsf > 1). Computed on the device (pos0 is a device value): a tile of n key tiles
+// takes ceil(n / w) pieces (1 to nsf), w the smallest length (in sixteenths of the chip's average share, FA_MINW at
+// least) for which the pieces of all tiles are at most one per CU, so the longest piece is as short as one round
+// allows. Piece s is tiles [s n / ns, (s + 1) n / ns), at least 2 of them (w >= 4), so its first key is below every row
+// of the token tile (each row sees a key in every piece). With w at least 2 x token tiles and n / w rounded down, as it
+// was, chunks of several hundred tokens left most of the chip idle: whole attn_decode calls, us, 400 tokens at position
+// 1500 76.6 -> 45.9, 600 at 3000 116 -> 70, 900 at 6000 195 -> 139, 1000 at 2000 106 -> 87, 512 at 32 000 335 -> 305.
 constexpr int FA_MINW = 8;
 constexpr int FA_NSF_MAX = 32;
 constexpr int FP_ROW = AHD + 4;  // a piece's partial row: O[256], m, l, 2 spare (16-byte aligned rows)
-__host__ __device__ inline int fa_piece_w(int pos0, int T, int KV, int NT, int ncu) {
-    const int total = (NT * ((2 * pos0 + T + FT) / 2) + NT * (BK - 1)) / BK;  // about the sum of n (split chunks: NT <= CUs)
-    const int m = FA_MINW > 2 * NT ? FA_MINW : 2 * NT, v = (KV * total + ncu - 1) / ncu;
-    return m > v ? m : v;
+constexpr int FP_W = AHD + 2;    // the spare slot of the first row holds w, for the merge
+// The first token tile with a piece p (tiles from it on have one: n grows with the tile), NT if none has
+__device__ __forceinline__ int fa_first_tile(int p, int pos0, int T, int NT, int w) {
+    const int need = BK * p * w + 1 - pos0;  // a piece p: n > p w, that is this many tokens seen
+    if (T < need) return NT;
+    return need <= FT ? 0 : (need + FT - 1) / FT - 1;
 }
-__host__ __device__ inline int fa_pieces(int t, int pos0, int T, int nsf, int w) {
-    const int n = (pos0 + (FT * (t + 1) < T ? FT * (t + 1) : T) + BK - 1) / BK, k = n / w;
-    return k < 1 ? 1 : k > nsf ? nsf : k;
+__device__ __forceinline__ int fa_pieces(int t, int pos0, int T, int nsf, int w) {
+    const int n = (pos0 + (FT * (t + 1) < T ? FT * (t + 1) : T) + BK - 1) / BK, k = (n + w - 1) / w;
+    return k > nsf ? nsf : k;
+}
+// w, and the pieces n1 of one kv head: lane l counts the pieces of its own candidate, the wavefront takes the smallest
+// that fits (uniform; every wavefront of the grid finds the same)
+__device__ __forceinline__ int fa_piece_w(int pos0, int T, int KV, int NT, int nsf, int ncu, int lane, int& n1) {
+    const int total = (NT * ((2 * pos0 + T + FT) / 2) + NT * (BK - 1)) / BK;  // about the sum of n (split chunks: NT <= CUs)
+    const int w0 = max(FA_MINW, (KV * total + ncu - 1) / ncu), wl = w0 + w0 * lane / 16;
+    int n = 0;
+    for (int p = 0; p < nsf; p++) {
+        const int c = NT - fa_first_tile(p, pos0, T, NT, wl);
+        if (!__builtin_amdgcn_ballot_w64(c > 0)) break;
+        n += c;
+    }
+    const unsigned long long fit = __builtin_amdgcn_ballot_w64(KV * n <= ncu);
+    const int nmax = (pos0 + T + BK - 1) / BK, l = fit ? __builtin_ctzll(fit) : 63;
+    if (!fit || 4 * (w0 + w0 * l / 16) > 3 * nmax) {  // the longest would hardly get shorter: no tile is split
+        n1 = NT;
+        return nmax;
+    }
+    n1 = __builtin_amdgcn_readlane(n, l);
+    return w0 + w0 * l / 16;
+}
+// Split launch: block b's (kv head, piece, token tile); false: no piece left. The pieces are listed by kv head, then by
+// piece, then by token tile, and every XCD takes a run of the list (block b runs on XCD b % 8), so the token tiles that
+// read one key range run on one XCD side by side and share its images in that L2 (listed by token tile: 300 tokens at
+// 8000 78.4 us, 74.6 so; 213 at 6144 58.5, 57.2).
+__device__ __forceinline__ bool fa_split_block(int b, int pos0, int T, int KV, int NT, int nsf, int w, int n1, int lane,
+                                               int& kvh, int& piece, int& tile) {
+    const int n = KV * n1;
+    if (b >= n) return false;
+    const int q = n >> 3, r = n & 7, x = b & 7, i = b >> 3;
+    int k = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i;
+    kvh = k / n1;
+    k -= kvh * n1;
+    const int t0 = lane < nsf ? fa_first_tile(lane, pos0, T, NT, w) : NT;  // of piece lane
+    for (piece = 0;; piece++) {
+        const int t = __builtin_amdgcn_readlane(t0, piece);
+        if (k < NT - t) {
+            tile = t + k;
+            return true;
+        }
+        k -= NT - t;
+    }
 }
 int fa_grid(int KV, int T) {
     const int NT = (T + FT - 1) / FT;
@@ -648,18 +693,12 @@ __global__ void __launch_bounds__(512, 1) fa_prefill_kernel(const float* __restr
     FaSeg sg[2];
     int kvh, nseg = 1, piece = 0, pslot = 0;
     if (MODE == FA_MODE_SPLIT) {
-        // block b takes the b-th piece, pieces listed heaviest token tile first, so the blocks left without one are
-        // the last ones dispatched (a queued block waits for a whole CU's LDS even when it has nothing to do)
-        const int w = fa_piece_w(pos0, T, KV, NT, ncu);
-        int b = blockIdx.x, tile, nsp = 1;
-        for (tile = NT - 1; tile >= 0; tile--) {
-            nsp = fa_pieces(tile, pos0, T, nsf, w);
-            if (b < KV * nsp) break;
-            b -= KV * nsp;
-        }
-        if (tile < 0) return;
-        kvh = b % KV;
-        piece = b / KV;
+        int n1;
+        const int w = fa_piece_w(pos0, T, KV, NT, nsf, ncu, threadIdx.x & 63, n1);
+        if (blockIdx.x == 0 && threadIdx.x == 0) reinterpret_cast<int*>(fpart)[FP_W] = w;
+        int tile;
+        if (!fa_split_block(blockIdx.x, pos0, T, KV, NT, nsf, w, n1, threadIdx.x & 63, kvh, piece, tile)) return;
+        const int nsp = fa_pieces(tile, pos0, T, nsf, w);
         const int nall = fa_ntiles(tile, pos0, T), ja = piece * nall / nsp;
         sg[0] = FaSeg{tile, ja, (piece + 1) * nall / nsp - ja, nsp > 1 ? FA_EPI_PIECE : FA_EPI_OUT};
     } else if (MODE == FA_MODE_PAIR) {
@@ -840,11 +879,11 @@ __global__ void __launch_bounds__(512, 1) fa_prefill_kernel(const float* __restr
 // l dims 4l .. 4l + 3 (lane s < pieces also holds piece s's m and l). Tiles with one piece were written by the FA
 // kernel.
 __global__ void __launch_bounds__(256) fa_merge_kernel(const float* __restrict__ fpart, const float* __restrict__ q_gate,
-                                                       float* __restrict__ out, int H, int KV, const int* __restrict__ pos_d,
-                                                       int ld, int T, int nsf, int ncu) {
+                                                       float* __restrict__ out, int H, const int* __restrict__ pos_d,
+                                                       int ld, int T, int nsf) {
     const int tok = 4 * blockIdx.x + (threadIdx.x >> 6), h = blockIdx.y, lane = threadIdx.x & 63, pos0 = *pos_d;
     if (tok >= T) return;
-    const int nsp = fa_pieces(tok / FT, pos0, T, nsf, fa_piece_w(pos0, T, KV, (T + FT - 1) / FT, ncu));
+    const int nsp = fa_pieces(tok / FT, pos0, T, nsf, reinterpret_cast<const int*>(fpart)[FP_W]);
     if (nsp <= 1) return;
     const float* pr = fpart + ((size_t)tok * H + h) * nsf * FP_ROW;
     const float2 ml = lane < nsp ? *reinterpret_cast<const float2*>(pr + lane * FP_ROW + AHD) : make_float2(-INFINITY, 0.f);
@@ -984,19 +1023,11 @@ FaPlan fa_plan(int H, int KV, int max_t, int T, bool turbo) {
     // underfilled. A full grid is not split: blocks queued behind a full chip were measured to start only after many
     // CUs had freed, so pieces of the heavy tiles gained little and the merge cost more. MOEX_FA_SPLIT=n caps the
     // pieces (1: no splitting).
-    int nsf = KV * NT >= ncu ? 1 : std::min(FA_NSF_MAX, (2 * ncu + KV * NT - 1) / (KV * NT));
+    // Beyond half a full grid not every tile could have two pieces, and the pairs below were faster (1500 tokens at 0 68
+    // against 77 us, at 5000 193 against 215: with every CU busy the clock drops, so shortening some blocks only is lost).
+    int nsf = 2 * KV * NT > ncu ? 1 : std::min(FA_NSF_MAX, (2 * ncu + KV * NT - 1) / (KV * NT));
     if (const char* e = std::getenv("MOEX_FA_SPLIT")) nsf = std::max(1, std::min(nsf, std::atoi(e)));
-    if (nsf > 1) {
-        // pos0 <= max_t - T: if the heaviest token tile would not split at any of these positions, launch unsplit
-        // (the split launch's extra blocks and merge cost a few microseconds even when nothing splits)
-        const int pmax = std::max(0, max_t - T);
-        bool any = false;
-        for (int i = 0; i <= 32 && !any; i++) {
-            const int p0 = (int)((long long)pmax * i / 32);
-            any = fa_pieces(NT - 1, p0, T, nsf, fa_piece_w(p0, T, KV, NT, ncu)) > 1;
-        }
-        if (!any) nsf = 1;
-    }
+    if (p.ntmax <= FA_MINW) nsf = 1;  // no token tile can have a second piece
     p.nsf = nsf;
     p.part_bytes = nsf > 1 ? (size_t)T * H * nsf * FP_ROW * sizeof(float) : 0;
     // pairs: MOEX_FA_PAIR=0 turns them off (read on every call)
@@ -1071,8 +1102,8 @@ void launch_fa_bufs(const float* qo, const float* q_gate, moex_kv_cache kv, floa
 #undef FA_LAUNCH
     MOEX_LAUNCHED();
     if (nsf > 1) {
-        hipLaunchKernelGGL(fa_merge_kernel, dim3((T + 3) / 4, H), dim3(256), 0, st, fpart, q_gate, out, H, KV, pos_d, ld,
-                           T, nsf, ncu);
+        hipLaunchKernelGGL(fa_merge_kernel, dim3((T + 3) / 4, H), dim3(256), 0, st, fpart, q_gate, out, H, pos_d, ld, T,
+                           nsf);
         MOEX_LAUNCHED();
     }
 }

@@ -184,3 +184,29 @@ def test_prefill_fallback_other_groups(Hq, KVq, pos0, T):
     e_new, e_ref = float(np.abs(got - ref).max()), float(np.abs(emu - ref).max())
     report("prefill(K7P) G", G=Hq // KVq, pos0=pos0, T=T, e_new=e_new, e_ref=e_ref, mag=mag)
     assert np.all(np.isfinite(o)) and e_new <= 2.0 * e_ref + 1e-3 * mag
+
+
+@pytest.mark.parametrize("pos0,T,cus", [
+    (0, 65, 256), (300, 129, 256), (1500, 400, 256), (6000, 1024, 256),  # half a full grid: the last size that splits
+    (6000, 1025, 256),                                                   # the first that runs in pairs
+    (20000, 213, 104), (3000, 600, 304), (33000, 1000, 8),               # other chip sizes; one too small to split on
+])
+def test_fa_piece_lengths(setup, pos0, T, cus, monkeypatch):
+    """The key pieces' length is searched on the device so that all pieces fit the chip once (planned here as for a chip
+    of `cus` CUs): every row written, and equal to the unsplit kernel up to the fp32 merge and the lazily rescaled
+    softmax's reference per piece (2e-3 of the largest output, as test_fa_key_split)."""
+    import torch
+    import moex_amd as M
+    _, dc, _, _, qo_d, qg_d = setup
+    monkeypatch.setenv("MOEX_FA_CUS", str(cus))
+    outs = []
+    for cap in ("32", "1"):
+        monkeypatch.setenv("MOEX_FA_SPLIT", cap)
+        out = torch.full((T, H, AHD), float("nan"), dtype=torch.float32, device="cuda")
+        M.attn_fa(qo_d, qg_d, dc, out, H, KV, pos_tensor(pos0), dc.max_t, LD, T)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.isfinite(outs[0]).all()
+    d, mag = float((outs[0] - outs[1]).abs().max()), float(outs[1].abs().max())
+    report("fa piece lengths", pos0=pos0, T=T, cus=cus, maxdiff=d, mag=mag)
+    assert d <= 2e-3 * mag

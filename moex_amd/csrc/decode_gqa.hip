@@ -909,23 +909,29 @@ static void launch_wsp(const float* qo, moex_kv_cache kv, int H, int KV, const i
 constexpr uint32_t spack(int a, int b, int c, int d) {
     return (uint32_t)(a & 0xff) | ((uint32_t)(b & 0xff) << 8) | ((uint32_t)(c & 0xff) << 16) | ((uint32_t)(d & 0xff) << 24);
 }
-constexpr uint32_t SK0 = spack(-127, -96, -75, -58), SK1 = spack(-44, -31, -18, -6);
-constexpr uint32_t SK2 = spack(6, 18, 31, 44), SK3 = spack(58, 75, 96, 127);
 // V codes biased by 128 (1 .. 255), read by the consumers as fp16 subnormals (bsub8)
 constexpr uint32_t SV0 = spack(1, 49, 83, 114), SV1 = spack(142, 173, 207, 255);
-// 8 nibbles of x -> the 4 signed K codes of its even nibbles (ev) and of its odd nibbles (od). The low 3 bits of a
-// nibble index a half-table (bytes 0-7 of the two v_perm sources); bit 3 moves the final pick to the upper half,
-// selector byte b + 4. 13 VALU per 8 codes.
+// 8 nibbles of x -> the 4 signed K codes of its even nibbles (ev) and of its odd nibbles (od), 11 VALU. A nibble c is a
+// v_perm selector as it is: 0-7 pick a byte of the source pair, 8-11 give the sign (0x00 / 0xff) of its byte 1, 3, 5 or 7,
+// 12 gives 0x00 and 13-15 0xff. So perm(A, c) ^ perm(B, c ^ 8) is the code when A[c] (c < 8) is I4[c] ^ what the second
+// perm gives for c + 8, and B[c - 8] (c >= 8) is I4[c] ^ what the first gives for c. (Masked to 3 bits, one perm per half
+// table and a third to choose between them took 13: whole step at 262 144 keys 41.0 us, 40.5 so.)
+constexpr uint32_t KA0 = 0x394aa081u, KA1 = 0x05111ed4u, KB0 = 0x2c1f12f9u, KB1 = 0x809fb43au;
+constexpr uint32_t perm_byte(uint32_t hi, uint32_t lo, int sel) {
+    const auto byte = [&](int i) { return (i < 4 ? lo >> (8 * i) : hi >> (8 * (i - 4))) & 0xffu; };
+    return sel < 8 ? byte(sel) : sel < 12 ? ((byte(2 * (sel - 8) + 1) & 0x80u) ? 0xffu : 0u) : sel == 12 ? 0u : 0xffu;
+}
+constexpr bool k_tables_ok() {
+    const int i4[16] = {-127, -96, -75, -58, -44, -31, -18, -6, 6, 18, 31, 44, 58, 75, 96, 127};
+    for (int c = 0; c < 16; c++)
+        if ((perm_byte(KA1, KA0, c) ^ perm_byte(KB1, KB0, c ^ 8)) != (uint32_t)(i4[c] & 0xff)) return false;
+    return true;
+}
+static_assert(k_tables_ok(), "K code tables");
 __device__ __forceinline__ void k_codes8(uint32_t x, int& ev, int& od) {
-    const uint32_t t = x >> 4;
-    const uint32_t se = x & 0x07070707u, so = t & 0x07070707u;
-    uint32_t pe, po;  // (y & 0x04040404) | 0x03020100 in one v_and_or_b32 (the constants held in registers)
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(pe) : "v"(x >> 1), "v"(0x04040404u), "v"(0x03020100u));
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(po) : "v"(t >> 1), "v"(0x04040404u), "v"(0x03020100u));
-    const uint32_t le = __builtin_amdgcn_perm(SK1, SK0, se), he = __builtin_amdgcn_perm(SK3, SK2, se);
-    const uint32_t lo = __builtin_amdgcn_perm(SK1, SK0, so), ho = __builtin_amdgcn_perm(SK3, SK2, so);
-    ev = (int)__builtin_amdgcn_perm(he, le, pe);
-    od = (int)__builtin_amdgcn_perm(ho, lo, po);
+    const uint32_t se = x & 0x0f0f0f0fu, so = (x >> 4) & 0x0f0f0f0fu;
+    ev = (int)(__builtin_amdgcn_perm(KA1, KA0, se) ^ __builtin_amdgcn_perm(KB1, KB0, se ^ 0x08080808u));
+    od = (int)(__builtin_amdgcn_perm(KA1, KA0, so) ^ __builtin_amdgcn_perm(KB1, KB0, so ^ 0x08080808u));
 }
 __device__ __forceinline__ int4_t_ k_codes(uint2 x) {  // 16 nibbles -> the MFMA operand (even, odd, even, odd)
     int a, b, c, d;

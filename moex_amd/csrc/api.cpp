@@ -302,11 +302,17 @@ void decode_step(const float* q, const float* k, const float* v, const uint16_t*
         launch_combine(part, q, out, H, ns, ld, T, st);
         return;
     }
-    launch_qk_norm_rope(q, k, v, qn, kn, qo, kv, H, KV, pos_d, max_t, rot, theta, eps, ld, T, st);
     const float* gate = kv.turbo ? nullptr : q;  // turbo: gated after the inverse rotation
-    if (T > 2 && ns == 1 && G == GQ && (moex_fa_on() || kv.turbo) && moex_fa_supported()) {
-        if (fa_scr) launch_fa_scratch(qo, gate, kv, out, H, KV, pos_d, max_t, ld, T, st, fa_scr, fa_bytes);
-        else launch_fa(qo, gate, kv, out, H, KV, pos_d, max_t, ld, T, st);
+    const bool fa = T > 2 && ns == 1 && G == GQ && (moex_fa_on() || kv.turbo) && moex_fa_supported();
+    if (fa && !fa_scr) {  // the front is part of the call
+        const FrontArgs fr{q, k, v, qn, kn, qo, skip_flag(), rot, theta, eps, ld};
+        launch_fa(qo, gate, kv, out, H, KV, pos_d, max_t, ld, T, st, &fr);
+        if (kv.turbo) launch_turbo_out(out, q, H, ld, T, st);
+        return;
+    }
+    launch_qk_norm_rope(q, k, v, qn, kn, qo, kv, H, KV, pos_d, max_t, rot, theta, eps, ld, T, st);
+    if (fa) {
+        launch_fa_scratch(qo, gate, kv, out, H, KV, pos_d, max_t, ld, T, st, fa_scr, fa_bytes);
     } else if (T > 2 && ns == 1 && 32 % G == 0 && !kv.turbo) {  // kernels.cuh:1856: any G dividing 32
         launch_prefill_k7p(qo, q, kv, out, H, KV, pos_d, max_t, ld, T, st);
     } else if (ns > 1 && G == GQ) {

@@ -110,8 +110,13 @@ void launch_gqa(const float* qo, moex_kv_cache kv, int H, int KV, const int* pos
                 int ns, hipStream_t st, bool rot_out = false, const FrontArgs* fr = nullptr);
 // this device's graph-fallback flag (g_skip, kernels.cuh:46), for kernels of other files; nullptr if unavailable
 const int* skip_flag();
+// fr: attn_decode's q/k front has not run yet (qo not formed, the rows not appended) and is part of the call
 void launch_fa(const float* qo, const float* q_gate, moex_kv_cache kv, float* out, int H, int KV, const int* pos_d,
-               int max_t, int ld, int T, hipStream_t st);
+               int max_t, int ld, int T, hipStream_t st, const FrontArgs* fr = nullptr);
+// the front's key and value rows alone (norm, RoPE, append); rows for which front_rows_aligned (the wavefront-per-row
+// kernels' condition: 16-byte aligned rows, rot % 8 == 0) holds
+void launch_front_kv(const FrontArgs& fr, moex_kv_cache kv, int KV, const int* pos_d, int max_t, int T, hipStream_t st);
+bool front_rows_aligned(const FrontArgs& fr);
 // dense int8 projections (dense.hip)
 void launch_quantize_rows_i8(const uint16_t* W, int8_t* q, float* s, int O, int I, hipStream_t st);
 void launch_gemv_i8(const int8_t* q, const float* s, const float* x, float* y, int NT, int I, int O, hipStream_t st);

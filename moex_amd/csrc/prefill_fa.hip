@@ -27,7 +27,7 @@
 #include <map>
 #include <mutex>
 #include <type_traits>
-#include "common.hpp"
+#include "front.hpp"
 
 namespace moex {
 
@@ -319,13 +319,49 @@ int fa_grid(int KV, int T) {
 // are taken by 16-byte slots (two rows a wavefront instruction). The grid is sized from the cache (the chunk's end is
 // a device value) but capped: a cache of 262 144 positions would otherwise launch 8 194 workgroups per kv head, most
 // of them for tiles past the chunk's end, and their dispatch alone took microseconds.
+// With nq > 0 (attn_decode, whose key and value rows a launch before this one has appended) the first nq workgroups form
+// the chunk's query rows, FA_QROWS of one token a wavefront (front::wave, the front kernel's bits), beside the
+// others' widening: neither needs the other, and each alone left the memory idle part of the time. The front and the
+// image pre-pass were two launches one after the other: whole attn_decode calls of 2048 tokens at position 0 int8 83.8 ->
+// 82.5 us, turbo 103.7 -> 95.9; int8 1000 at 2000 86.5 -> 83.7, 213 at 6144 56.6 -> 55.6.
+constexpr int FA_QROWS = 4;
+template <bool TB>
+__device__ __forceinline__ void fa_query_rows(const FrontArgs& fr, const int* pos_d, int T, int H, int block) {
+    if (fr.skip && *fr.skip) return;
+    const int wpt = (H + FA_QROWS - 1) / FA_QROWS;
+    const int w = block * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (w >= T * wpt) return;
+    const int tok = w / wpt, h0 = (w - tok * wpt) * FA_QROWS;
+    const float* q = fr.q + (size_t)tok * fr.ld;
+    float4 x4[FA_QROWS];
+#pragma unroll
+    for (int i = 0; i < FA_QROWS; i++)
+        if (h0 + i < H) x4[i] = *reinterpret_cast<const float4*>(q + (h0 + i) * 2 * AHD + 4 * lane);
+    const uint2 wq = *reinterpret_cast<const uint2*>(fr.qn + 4 * lane);
+    const front::wave::Rope rp = front::wave::rope_angles(lane, *pos_d + tok, fr.rot, fr.theta);
+#pragma unroll
+    for (int i = 0; i < FA_QROWS; i++) {
+        if (h0 + i >= H) break;
+        float x[4] = {x4[i].x, x4[i].y, x4[i].z, x4[i].w};
+        front::wave::norm_rope(x, wq, lane, rp, fr.rot, fr.eps);
+        if (TB) front::wave::wht(x, 0, lane);  // the keys' rotation
+        *reinterpret_cast<float4*>(fr.qo + ((size_t)tok * H + h0 + i) * AHD + 4 * lane) =
+            make_float4(x[0], x[1], x[2], x[3]);
+    }
+}
 template <bool TB>
 __global__ void __launch_bounds__(256) fa_image_kernel(moex_kv_cache kv, const int* __restrict__ pos_d, int T, int max_t,
-                                                       int ntmax, unsigned char* __restrict__ img) {
-    const int kvh = blockIdx.y, hi = *pos_d + T, tid = threadIdx.x;
+                                                       int ntmax, unsigned char* __restrict__ img, int KV, int H, int nq,
+                                                       FrontArgs fr) {
+    if ((int)blockIdx.x < nq) {
+        fa_query_rows<TB>(fr, pos_d, T, H, blockIdx.x);
+        return;
+    }
+    const int b = blockIdx.x - nq, nb = (gridDim.x - nq) / KV;  // image workgroups of a kv head
+    const int kvh = b / nb, hi = *pos_d + T, tid = threadIdx.x;
     const size_t rbase = (size_t)kvh * max_t;
     __shared__ __align__(16) unsigned char vl[VT_BYTES];  // the tile's V^T, written transposed, copied out in rows
-    for (int j = blockIdx.x; j < ntmax && j * BK < hi; j += gridDim.x) {
+    for (int j = b % nb; j < ntmax && j * BK < hi; j += nb) {
         const int k0 = j * BK;
         unsigned char* t = img + ((size_t)kvh * ntmax + j) * TILE_BYTES;
         float* sc = reinterpret_cast<float*>(t + KT_BYTES + VT_BYTES);
@@ -1060,7 +1096,7 @@ FaPlan fa_plan(int H, int KV, int max_t, int T, bool turbo) {
 template <bool TB>
 void launch_fa_bufs(const float* qo, const float* q_gate, moex_kv_cache kv, float* out, int H, int KV,
                     const int* pos_d, int max_t, int ld, int T, hipStream_t st, const FaPlan& p, unsigned char* img,
-                    float* fpart, int nsf, unsigned* pcnt) {
+                    float* fpart, int nsf, unsigned* pcnt, const FrontArgs* fr = nullptr) {
     const int ncu = fa_ncu(), ntmax = p.ntmax;
     if (nsf > 1 && !fpart) nsf = 1;
     const bool pair = nsf == 1 && p.pair && fpart && pcnt;
@@ -1070,7 +1106,9 @@ void launch_fa_bufs(const float* qo, const float* q_gate, moex_kv_cache kv, floa
         int wpc = 16;
         if (const char* e = std::getenv("MOEX_FA_IMG_WG")) wpc = std::max(1, std::atoi(e));
         const int gx = std::max(1, std::min(ntmax, wpc * ncu / KV));
-        hipLaunchKernelGGL(fa_image_kernel<TB>, dim3(gx, KV), dim3(256), 0, st, kv, pos_d, T, max_t, ntmax, img);
+        const int nq = fr ? (T * ((H + FA_QROWS - 1) / FA_QROWS) + 3) / 4 : 0;
+        hipLaunchKernelGGL(fa_image_kernel<TB>, dim3(nq + gx * KV), dim3(256), 0, st, kv, pos_d, T, max_t, ntmax, img, KV, H,
+                           nq, fr ? *fr : FrontArgs{});
         MOEX_LAUNCHED();
     }
     // a split launch has KV x tiles x nsf blocks: the pieces of every tile, the rest exit at once
@@ -1110,8 +1148,17 @@ void launch_fa_bufs(const float* qo, const float* q_gate, moex_kv_cache kv, floa
 
 template <bool TB>
 void launch_fa_t(const float* qo, const float* q_gate, moex_kv_cache kv, float* out, int H, int KV, const int* pos_d,
-                 int max_t, int ld, int T, hipStream_t st) {
+                 int max_t, int ld, int T, hipStream_t st, const FrontArgs* fr) {
     const FaPlan p = fa_plan(H, KV, max_t, T, TB);
+    // attn_decode's q/k front: a launch of its own before everything else, or, on tile images, the key and value rows
+    // in a launch and the query rows in the image pre-pass
+    unsigned char* img = !p.gns && p.img_bytes ? stream_workspace(p.img_bytes, st, 0) : nullptr;
+    const bool fuse = fr && img && front_rows_aligned(*fr);
+    if (fuse)
+        launch_front_kv(*fr, kv, KV, pos_d, max_t, T, st);
+    else if (fr)
+        launch_qk_norm_rope(fr->q, fr->k, fr->v, fr->qn, fr->kn, fr->qo, kv, H, KV, pos_d, max_t, fr->rot, fr->theta,
+                            fr->eps, fr->ld, T, st);
     if (p.gns > 0) {  // a short chunk: split-K decode kernels and the gated combine (turbo: in the rotated domain, as
                       // the FA kernel leaves it)
         float* part = reinterpret_cast<float*>(stream_workspace(p.gqa_bytes, st, 4));
@@ -1123,15 +1170,16 @@ void launch_fa_t(const float* qo, const float* q_gate, moex_kv_cache kv, float* 
     }
     float* fpart = p.part_bytes ? reinterpret_cast<float*>(stream_workspace(p.part_bytes, st, 1)) : nullptr;
     unsigned* pcnt = p.cnt_bytes ? reinterpret_cast<unsigned*>(stream_workspace(p.cnt_bytes, st, 5)) : nullptr;
-    unsigned char* img = p.img_bytes ? stream_workspace(p.img_bytes, st, 0) : nullptr;
-    launch_fa_bufs<TB>(qo, q_gate, kv, out, H, KV, pos_d, max_t, ld, T, st, p, img, fpart, fpart ? p.nsf : 1, pcnt);
+    if (!img && p.gns && p.img_bytes) img = stream_workspace(p.img_bytes, st, 0);
+    launch_fa_bufs<TB>(qo, q_gate, kv, out, H, KV, pos_d, max_t, ld, T, st, p, img, fpart, fpart ? p.nsf : 1, pcnt,
+                       fuse ? fr : nullptr);
 }
 }  // namespace
 
 void launch_fa(const float* qo, const float* q_gate, moex_kv_cache kv, float* out, int H, int KV, const int* pos_d,
-               int max_t, int ld, int T, hipStream_t st) {
-    if (kv.turbo) launch_fa_t<true>(qo, q_gate, kv, out, H, KV, pos_d, max_t, ld, T, st);
-    else launch_fa_t<false>(qo, q_gate, kv, out, H, KV, pos_d, max_t, ld, T, st);
+               int max_t, int ld, int T, hipStream_t st, const FrontArgs* fr) {
+    if (kv.turbo) launch_fa_t<true>(qo, q_gate, kv, out, H, KV, pos_d, max_t, ld, T, st, fr);
+    else launch_fa_t<false>(qo, q_gate, kv, out, H, KV, pos_d, max_t, ld, T, st, fr);
 }
 
 void launch_fa_scratch(const float* qo, const float* q_gate, moex_kv_cache kv, float* out, int H, int KV,

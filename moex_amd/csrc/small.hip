@@ -108,6 +108,24 @@ __global__ void __launch_bounds__(256) front_rows_kernel(
         }
     }
 }
+// The key and value rows of the front (a wavefront per row, r = token KV + kv head), for a prefill whose image pre-pass
+// forms the query rows
+__global__ void __launch_bounds__(256) front_kv_kernel(FrontArgs fr, moex_kv_cache kv, int KV, const int* __restrict__ pos_d,
+                                                       int max_t, int T) {
+    if (g_skip) return;
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= T * KV) return;
+    const int tok = r / KV, kvh = r - tok * KV;
+    const size_t o = (size_t)tok * fr.ld + kvh * AHD + 4 * lane;
+    const float4 k4 = *reinterpret_cast<const float4*>(fr.k + o), v4 = *reinterpret_cast<const float4*>(fr.v + o);
+    const uint2 wk = *reinterpret_cast<const uint2*>(fr.kn + 4 * lane);
+    const int pos = *pos_d + tok;
+    const front::wave::Rope rp = front::wave::rope_angles(lane, pos, fr.rot, fr.theta);
+    float x[4] = {k4.x, k4.y, k4.z, k4.w};
+    const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
+    front::wave::norm_rope(x, wk, lane, rp, fr.rot, fr.eps);
+    front::wave::append(x, vv, kv, (size_t)kvh * max_t + pos, lane);
+}
 // Quantize-append only, one wavefront per row (rows r = token KV + kv head)
 __global__ void __launch_bounds__(256) append_rows_kernel(const float* __restrict__ k, const float* __restrict__ v,
                                                           moex_kv_cache kv, int KV, const int* __restrict__ pos_d,
@@ -392,15 +410,14 @@ void launch_qk_norm_rope(const float* q, const float* k, const float* v, const u
                          float* qo, moex_kv_cache kv, int H, int KV, const int* pos_d, int max_t, int rot,
                          float theta, float eps, int ld, int T, hipStream_t st) {
     // the 16-byte row loads and the wavefront layout need 4-float aligned rows
-    const bool al = ld % 4 == 0 && ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)qo) % 16 == 0 &&
-                    ((uintptr_t)qn | (uintptr_t)kn) % 8 == 0;
+    const bool al = front_rows_aligned(FrontArgs{q, k, v, qn, kn, qo, nullptr, rot, theta, eps, ld});
     // rows per wavefront: 3 (a 2048-token chunk at 32768: int8 26.7-29.3 -> 20.1-22.0 us, turbo 33.4-34.4 -> 32.4;
     // 6 and 9 no better, turbo slower at 6); MOEX_FRONT_RPW=1, 3, 6 or 9 for comparisons (read on every call)
     int rpw = 3;
     if (const char* e = std::getenv("MOEX_FRONT_RPW")) rpw = std::atoi(e);
     const int waves = T * ((H + KV + rpw - 1) / std::max(rpw, 1));
     const dim3 grid((waves + 3) / 4);
-    if (rot % 8 == 0 && al) {
+    if (al) {
         if (rpw == 1)
             hipLaunchKernelGGL(front_rows_kernel<1>, grid, dim3(256), 0, st, q, k, v, qn, kn, qo, kv, H, KV, pos_d, max_t,
                                rot, theta, eps, ld, T);
@@ -416,6 +433,15 @@ void launch_qk_norm_rope(const float* q, const float* k, const float* v, const u
     } else
         hipLaunchKernelGGL(qk_norm_rope_kernel, dim3(H + KV, T), dim3(256), 0, st, q, k, v, qn, kn, qo, kv, H, KV,
                            pos_d, max_t, rot, theta, eps, ld);
+    MOEX_LAUNCHED();
+}
+bool front_rows_aligned(const FrontArgs& fr) {
+    return fr.rot % 8 == 0 && fr.ld % 4 == 0 &&
+           ((uintptr_t)fr.q | (uintptr_t)fr.k | (uintptr_t)fr.v | (uintptr_t)fr.qo) % 16 == 0 &&
+           ((uintptr_t)fr.qn | (uintptr_t)fr.kn) % 8 == 0;
+}
+void launch_front_kv(const FrontArgs& fr, moex_kv_cache kv, int KV, const int* pos_d, int max_t, int T, hipStream_t st) {
+    hipLaunchKernelGGL(front_kv_kernel, dim3((T * KV + 3) / 4), dim3(256), 0, st, fr, kv, KV, pos_d, max_t, T);
     MOEX_LAUNCHED();
 }
 void launch_kv_append(const float* k, const float* v, moex_kv_cache kv, int KV, const int* pos_d, int max_t, int ld,

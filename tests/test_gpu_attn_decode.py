@@ -296,3 +296,46 @@ def test_one_split_call_runs_split_k(turbo, T):
         outs.append(out.cpu().numpy())
     report("attn_decode ns=1 vs splits", turbo=turbo, T=T, maxdiff=float(np.abs(outs[0] - outs[1]).max()))
     assert np.all(np.isfinite(outs[0])) and np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("turbo,pos,T,rot,shift", [
+    (0, 0, 65, 64, 0), (1, 0, 17, 64, 0),   # the smallest chunks that take the FA kernel, nothing cached before
+    (0, 900, 131, 32, 0), (1, 900, 131, 256, 0),  # a ragged chunk inside a tile, other rotated widths
+    (0, 33, 2048, 64, 0),                   # a full grid (pairs)
+    (0, 500, 200, 64, 1),                   # rows 4 bytes off a 16-byte boundary: the front's own launch
+])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_prefill_front_matches_separate(turbo, pos, T, rot, shift, skip):
+    """attn_decode's prefill, whose query rows are formed in the image pre-pass, against qk_norm_rope, attn_fa (and
+    turbo_out) called one by one: qo, the cache and the output bit for bit, also with the skip flag set (the front
+    does nothing then, and neither does turbo_out)."""
+    import torch
+    import moex_amd as M
+    max_t = 3072
+    _, (da, db) = _caches(M, torch, turbo, max_t, 81, 2)
+    rng = np.random.default_rng(82)
+    LQ = H * 2 * AHD + 2 * KV * AHD + 4
+    buf = torch.zeros(T * LQ + 8, device="cuda")
+    qkv = buf[shift:shift + T * LQ].view(T, LQ)
+    qkv.copy_(dev(rng.standard_normal((T, LQ), dtype=np.float32)))
+    k, v = qkv[:, H * 2 * AHD:], qkv[:, H * 2 * AHD + KV * AHD:]
+    qn = dev((rng.standard_normal(AHD) * 0.1).astype(np.float16).view(np.int16))
+    kn = dev((rng.standard_normal(AHD) * 0.1).astype(np.float16).view(np.int16))
+    qa = dev(rng.standard_normal((T, H, AHD), dtype=np.float32))
+    qb = qa.clone()
+    oa, ob = (torch.full((T, H, AHD), float("nan"), device="cuda") for _ in range(2))
+    pd = pos_tensor(pos)
+    M.set_skip(skip)
+    try:
+        M.attn_decode(qkv, k, v, qn, kn, qa, da, oa, H, KV, pd, max_t, rot, 1e7, 1e-6, T, LQ)
+        M.qk_norm_rope(qkv, k, v, qn, kn, qb, db, H, KV, pd, max_t, rot, 1e7, 1e-6, LQ, T)
+        M.attn_fa(qb, None if turbo else qkv, db, ob, H, KV, pd, max_t, LQ, T)
+        if turbo:
+            M.turbo_out(ob, qkv, H, LQ, T)
+        torch.cuda.synchronize()
+    finally:
+        M.set_skip(0)
+        torch.cuda.synchronize()
+    for name in ("k", "v", "ks", "vs"):
+        assert torch.equal(getattr(da, name), getattr(db, name)), name
+    assert torch.equal(qa, qb) and torch.isfinite(oa).all() and torch.equal(oa, ob)

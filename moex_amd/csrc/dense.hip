@@ -17,6 +17,7 @@
 //   quantize_gs64_kernel   fp16 rows -> int4 / int6 codes + a scale per 64-input group (bit-exact).
 //   gemv_mat_kernel        the GEMV of the int4 / int6 / fp16 forms: a lane per 16-weight unit of R rows, each unit
 //                          summed in order and scaled, wavefront and part sums as gemv_kernel.
+//   gemv_mat_x_kernel      the same without a loop where a part of a row is one load a lane, with the input rows in LDS.
 //   gemm_tile_kernel<form> the same GEMM for every form: the staging widens int4 / int6 weights times their group
 //                          scale to fp16 (or copies fp16 weights) where int8 is widened exactly.
 #include <algorithm>
@@ -758,6 +759,22 @@ __device__ __forceinline__ void mat_unit_load(MatUnit<FMT>& u, const uint8_t* W,
         u.sc = s[row * (I / 64) + c / 4];
     }
 }
+// weight k of the unit, without its scale (k a constant after unrolling)
+template <int FMT> __device__ __forceinline__ float mat_unit_weight(const MatUnit<FMT>& u, int k) {
+    if constexpr (FMT == MF_F16) {
+        const uint4& q = u.a[k / 8];
+        const uint32_t d2 = ((k / 2) & 3) == 0 ? q.x : ((k / 2) & 3) == 1 ? q.y : ((k / 2) & 3) == 2 ? q.z : q.w;
+        return (float)u2h2(d2)[k & 1];
+    } else {
+        const uint32_t dw = k < 8 ? u.a[0].x : u.a[0].y;
+        if constexpr (FMT == MF_Q4) {
+            return (float)(int)__builtin_amdgcn_sbfe(dw, 4 * (k & 7), 4);  // the signed nibble (the builtin returns it as unsigned)
+        } else {
+            const uint32_t hb = (u.h >> (2 * k)) & 3u;
+            return (float)((int)(((dw >> (4 * (k & 7))) & 15u) | (hb << 4)) - 32);
+        }
+    }
+}
 template <int FMT>
 __device__ __forceinline__ float mat_unit_dot(const MatUnit<FMT>& u, const float4 (&x)[4]) {
     float d = 0.f;
@@ -765,24 +782,7 @@ __device__ __forceinline__ float mat_unit_dot(const MatUnit<FMT>& u, const float
     for (int j = 0; j < 4; j++) {
         const float xv[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
 #pragma unroll
-        for (int n = 0; n < 4; n++) {
-            const int k = 4 * j + n;
-            float w;
-            if constexpr (FMT == MF_F16) {
-                const uint4& q = u.a[k / 8];
-                const uint32_t d2 = ((k / 2) & 3) == 0 ? q.x : ((k / 2) & 3) == 1 ? q.y : ((k / 2) & 3) == 2 ? q.z : q.w;
-                w = (float)u2h2(d2)[k & 1];
-            } else {
-                const uint32_t dw = k < 8 ? u.a[0].x : u.a[0].y;
-                if constexpr (FMT == MF_Q4) {
-                    w = (float)(int)__builtin_amdgcn_sbfe(dw, 4 * (k & 7), 4);  // the signed nibble (the builtin returns it as unsigned)
-                } else {
-                    const uint32_t hb = (u.h >> (2 * k)) & 3u;
-                    w = (float)((int)(((dw >> (4 * (k & 7))) & 15u) | (hb << 4)) - 32);
-                }
-            }
-            d = fmaf(w, xv[n], d);
-        }
+        for (int n = 0; n < 4; n++) d = fmaf(mat_unit_weight<FMT>(u, 4 * j + n), xv[n], d);
     }
     return FMT == MF_F16 ? d : d * u.sc;
 }
@@ -801,11 +801,9 @@ __global__ void __launch_bounds__(64 * GM_WAVES) gemv_mat_kernel(const uint8_t* 
     for (int j = 0; j < rounds; j++) {
         const int g = blockIdx.x + nb * (wv / KS + j * gpr);
         if (g < ngroups) {
-            float acc[NT][R];
+            float acc[NT * R];
 #pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int r = 0; r < R; r++) acc[t][r] = 0.f;
+            for (int i = 0; i < NT * R; i++) acc[i] = 0.f;
             for (int c = cb + lane; c < ce; c += 64) {
                 MatUnit<FMT> u[R];
 #pragma unroll
@@ -817,16 +815,15 @@ __global__ void __launch_bounds__(64 * GM_WAVES) gemv_mat_kernel(const uint8_t* 
 #pragma unroll
                     for (int i = 0; i < 4; i++) xv[i] = xp[i];
 #pragma unroll
-                    for (int r = 0; r < R; r++) acc[t][r] += mat_unit_dot<FMT>(u[r], xv);
+                    for (int r = 0; r < R; r++) acc[t * R + r] += mat_unit_dot<FMT>(u[r], xv);
                 }
             }
+            wave_sums(acc);
 #pragma unroll
-            for (int t = 0; t < NT; t++)
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const float v = wave_sum(acc[t][r]);
-                    if (lane == 0) red[wv][t][r] = v;
-                }
+            for (int k = 0; k < ((NT * R + 1) / 2 + 1) / 2; k++) {
+                const int i = wave_sums_index<NT * R>(k, lane >> 4);
+                if ((lane & 15) == 0 && i < NT * R) red[wv][i / R][i % R] = acc[k];
+            }
         }
         __syncthreads();
         if (g < ngroups && part == 0 && lane < NT * R) {
@@ -836,6 +833,103 @@ __global__ void __launch_bounds__(64 * GM_WAVES) gemv_mat_kernel(const uint8_t* 
             if (o < O) y[(size_t)t * O + o] = v;
         }
         __syncthreads();  // the partial sums are read before the next round writes them
+    }
+}
+
+// The same product when a part of a row is at most 64 units (one load step a lane) and the input rows fit LDS: one row
+// group a wavefront and no loop, so a workgroup's loads all go out at once and R follows from whole rounds of the chip.
+// The input rows go into LDS once per workgroup by DMA, in gemv1_kernel's layout, instead of being read from L2 by every
+// wavefront (8 rows of inputs are ten times the bytes of 4 int6 weight rows), and a unit is widened once per group of
+// input rows. One int4 / int6 row's inputs are read straight from L2 (int4 qkv 5.0 against 5.3 us); beside the wider fp16
+// weights LDS is better for one row too (8.8 against 10.1). Same sum order as gemv_mat_kernel, so a row's bits are those
+// of its own call. Bound by the weight stream and the launch for one or two rows, by the widening and the FMAs for more.
+// Graph-replayed over rotating weights, us, before -> now (before: gemv_mat_kernel; int4 and fp16 row by row):
+//   input rows               1           2            3           4           6            8
+//   int6 qkv 9216 x 2048     7.1 -> 6.1  9.4 -> 8.1   11.1 -> 7.5 13.1 -> 9.1 23.7 -> 10.5 27.6 -> 11.8
+//   int6 o   2048 x 4096     4.7 -> 4.6  5.4 -> 5.0   7.0 -> 5.3  7.9 -> 5.7  11.1 -> 6.4  12.4 -> 7.1
+//   int4 qkv, o              6.0 -> 5.0, 4.0 -> 3.8   12.1 -> 6.3, 7.7 -> 4.2
+//   fp16 qkv, o              10.5 -> 8.8, 6.6 -> 5.5  21.0 -> 9.3, 12.9 -> 6.1
+template <int FMT, int NT> constexpr bool mat_xl = NT > 1 || FMT == MF_F16;  // input rows through LDS
+template <int FMT, int NT, int R>
+__global__ void __launch_bounds__(64 * GM_WAVES, 2) gemv_mat_x_kernel(const uint8_t* __restrict__ W,
+                                                                      const uint8_t* __restrict__ Wh,
+                                                                      const float* __restrict__ s,
+                                                                      const float* __restrict__ x, float* __restrict__ y,
+                                                                      int I, int O, int KS) {
+    constexpr bool XL = mat_xl<FMT, NT>;
+    extern __shared__ __align__(16) float xs[];  // XL: the input rows [NT][I]; then the partial sums [GM_WAVES][NT * R]
+    float* red = xs + (XL ? NT * I : 0);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gpw = GM_WAVES / KS, part = wv % KS, slice = I / 16 / KS;
+    const int g = blockIdx.x * gpw + wv / KS;
+    const bool on = lane < slice;
+    const int c = min(part * slice + lane, I / 16 - 1);
+    constexpr int TB = NT <= 4 ? NT : (NT + 1) / 2;  // input rows whose values fit the registers
+    float4 xv[TB][4];
+    if constexpr (XL) {
+        const int n = NT * I / 256;  // 1 KB transfers
+        for (int i = wv; i < n; i += GM_WAVES) {
+            const uint32_t e = 64 * i + lane;
+            dma16x(x, 16 * (e ^ ((e >> 3) & 3)), reinterpret_cast<const unsigned char*>(xs) + 1024 * i);
+        }
+    } else {
+#pragma unroll
+        for (int d = 0; d < 4; d++) xv[0][d] = reinterpret_cast<const float4*>(x)[4 * c + d];
+    }
+    MatUnit<FMT> u[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) mat_unit_load<FMT>(u[r], W, Wh, s, (size_t)min(g * R + r, O - 1), I, c);
+    if constexpr (XL) asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // the products need both anyway
+    float acc[NT * R];
+#pragma unroll
+    for (int t0 = 0; t0 < NT; t0 += TB) {
+        if constexpr (XL) {
+#pragma unroll
+            for (int t = t0; t < NT && t < t0 + TB; t++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const uint32_t e = t * (I / 4) + 4 * c + d;
+                    xv[t - t0][d] = reinterpret_cast<const float4*>(xs)[e ^ ((e >> 3) & 3)];
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            float a[TB];
+#pragma unroll
+            for (int t = 0; t < TB; t++) a[t] = 0.f;
+#pragma unroll
+            for (int d = 0; d < 4; d++) {
+                float w[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = mat_unit_weight<FMT>(u[r], 4 * d + i);
+#pragma unroll
+                for (int t = 0; t < TB && t0 + t < NT; t++) {
+                    a[t] = fmaf(w[0], xv[t][d].x, a[t]);
+                    a[t] = fmaf(w[1], xv[t][d].y, a[t]);
+                    a[t] = fmaf(w[2], xv[t][d].z, a[t]);
+                    a[t] = fmaf(w[3], xv[t][d].w, a[t]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TB && t0 + t < NT; t++)
+                acc[(t0 + t) * R + r] = on ? 0.f + (FMT == MF_F16 ? a[t] : a[t] * u[r].sc) : 0.f;  // no -0
+        }
+        if constexpr (NT > TB) asm volatile("" ::: "memory");  // the next group's values are read after these are used
+    }
+    wave_sums(acc);
+#pragma unroll
+    for (int k = 0; k < ((NT * R + 1) / 2 + 1) / 2; k++) {
+        const int i = wave_sums_index<NT * R>(k, lane >> 4);
+        if ((lane & 15) == 0 && i < NT * R) red[wv * NT * R + i] = acc[k];
+    }
+    __syncthreads();
+    const int rows = gpw * R;  // of this workgroup
+    for (int e = tid; e < NT * rows; e += 64 * GM_WAVES) {
+        const int t = e / rows, rr = e % rows, gl = rr / R, r = rr % R, o = (blockIdx.x * gpw + gl) * R + r;
+        if (o >= O) continue;
+        float v = red[gl * KS * NT * R + t * R + r];
+        for (int p = 1; p < KS; p++) v += red[(gl * KS + p) * NT * R + t * R + r];
+        y[(size_t)t * O + o] = v;
     }
 }
 
@@ -850,6 +944,20 @@ int dense_cus() {
     return cus;
 }
 
+template <int FMT, int NT, int R>
+void launch_gemv_mat_x(const uint8_t* W, const uint8_t* Wh, const float* s, const float* x, float* y, int I, int O, int ks,
+                       size_t lds, hipStream_t st) {
+    static bool once = [] {
+        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv_mat_x_kernel<FMT, NT, R>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        return true;
+    }();
+    (void)once;
+    const int gpw = GM_WAVES / ks, wgs = ((O + R - 1) / R + gpw - 1) / gpw;
+    hipLaunchKernelGGL((gemv_mat_x_kernel<FMT, NT, R>), dim3(wgs), dim3(64 * GM_WAVES), lds, st, W, Wh, s, x, y, I, O, ks);
+    MOEX_LAUNCHED();
+}
+
 template <int FMT, int NT>
 void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, const float* x, float* y, int I, int O,
                        hipStream_t st) {
@@ -860,6 +968,32 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
     int ks = 1;
     while (ks < GM_WAVES && U % (2 * ks) == 0 && U / (2 * ks) >= 64) ks *= 2;
     const int gpr = GM_WAVES / ks;
+    {
+        // the rows per wavefront with the cheapest rounds over the chip, as launch_gemv1: of 2, 3, 4 and 6 the fastest or
+        // within 6 % of it for 1 to 8 input rows on qkv (3) and o_proj (4). The transfers are of 16 bytes a lane and 1 KB
+        // each: input rows of another alignment or length take the kernel below
+        constexpr bool XL = mat_xl<FMT, NT>;
+        const size_t lds = (XL ? (size_t)NT * I * 4 : 0) + (size_t)GM_WAVES * NT * 4 * 6;
+        if (U / ks <= 64 && lds <= 160 * 1024 &&
+            (!XL || (I % 256 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0))) {
+            int best = 0;
+            long cost = 0;
+            for (int R : {2, 3, 4, 6}) {
+                const long wgs = ((O + R - 1) / R + gpr - 1) / gpr, e = (wgs + cus - 1) / cus * (R + 2);
+                if (!best || e < cost) {
+                    best = R;
+                    cost = e;
+                }
+            }
+            switch (best) {
+                case 2: launch_gemv_mat_x<FMT, NT, 2>(W, Wh, s, x, y, I, O, ks, lds, st); break;
+                case 3: launch_gemv_mat_x<FMT, NT, 3>(W, Wh, s, x, y, I, O, ks, lds, st); break;
+                case 4: launch_gemv_mat_x<FMT, NT, 4>(W, Wh, s, x, y, I, O, ks, lds, st); break;
+                default: launch_gemv_mat_x<FMT, NT, 6>(W, Wh, s, x, y, I, O, ks, lds, st); break;
+            }
+            return;
+        }
+    }
     int R = 4;
     while (R > 1 && ((O + R - 1) / R + gpr - 1) / gpr < cus) R /= 2;
     const int nb = std::min(2 * cus, ((O + R - 1) / R + gpr - 1) / gpr);

@@ -250,6 +250,31 @@ def test_gemm_odd_inputs(I):
         assert _rel(got[np.ix_(rows, cols)].astype(np.float64), orc.dense_mat_fp16x(F, hw[cols], None, None, x[rows])) < 1e-5
 
 
+@pytest.mark.parametrize("fmt", ["q4", "q6", "f16"])
+@pytest.mark.parametrize("O,I", [(1, 256), (37, 256), (2303, 2048), (513, 4096), (100, 320), (77, 8192)],
+                         ids=["one-row", "short", "qkv-like", "o-like", "part-of-a-transfer", "past-lds"])
+def test_gemv_rows_through_lds(O, I, fmt):
+    """The GEMV's input rows through LDS or, where their length, size or alignment does not allow it, straight from
+    memory: a row has the same bits alone, beside others and at any alignment, and nothing is written past the last."""
+    import torch
+    import moex_amd as M
+    rng = np.random.default_rng(O + I)
+    m, _, _, _keep = _make(fmt, (rng.standard_normal((O, I)) * 0.02).astype(np.float16))
+    x = dev(rng.standard_normal((8, I)).astype(np.float32))
+    xu = torch.empty(8 * I + 1, dtype=torch.float32, device="cuda")[1:].view(8, I)
+    xu.copy_(x)
+    Yr = torch.full((8, O), float("nan"), dtype=torch.float32, device="cuda")
+    for t in range(8):
+        M.gemv(m, x[t], Yr[t], I, O)
+    for xs in (x, xu):
+        for S in range(1, 9 if fmt == "q6" else 3):
+            Y = torch.full((9, O), 123.0, dtype=torch.float32, device="cuda")
+            M.gemm(m, xs[:S], Y, S, I, O)
+            torch.cuda.synchronize()
+            assert torch.equal(Y[:S], Yr[:S]), S
+            assert bool((Y[S:] == 123.0).all()), S
+
+
 @pytest.mark.parametrize("fmt", ["q4", "f16"])
 def test_two_rows_equal_gemv(shape, fmt):
     """int4 and fp16 with two rows (one pass over the weights): each row the bits of the one-row GEMV."""

@@ -365,8 +365,8 @@ __device__ __forceinline__ void wstage_widen(const WStage& w, bool ok, uint32_t 
 // roles, an fp16 rounding launch for every call, K split over workgroups with a reduction launch), int8:
 //   tokens              9          64         300        512        1024       2048
 //   qkv  9216 x 2048    19.2->9.0  31.0->13.6 46.7->29.1 48.4->42.7 74.8->58.0 142.9->92.0 (842 TFLOPS)
-//   o    2048 x 4096    17.2->8.5  24.1->10.5 33.8->21.9 38.8->22.7 52.9->34.5  74.3->52.3 (657 TFLOPS)
-// int4 at 300 tokens: qkv 45.9 -> 31.1, o 31.7 -> 25.3; fp16 at 2048: 142.0 -> 88.1, 82.3 -> 59.9.
+//   o    2048 x 4096    17.2->8.5  24.1->10.5 33.8->21.3 38.8->22.7 52.9->34.5  74.3->52.3 (657 TFLOPS)
+// int4 at 300 tokens: qkv 45.9 -> 31.1, o 31.7 -> 21.2; fp16 at 2048: 142.0 -> 88.1, 82.3 -> 59.9.
 template <int WM_, int WN_, int GM_, int GN_, int KW_, int BKU_, int PD_, bool XH_ = false, int WPE_ = 2>
 struct GemmTile {
     static constexpr int WM = WM_, WN = WN_, GM = GM_, GN = GN_, KW = KW_, BKU = BKU_, PD = PD_;
@@ -1008,12 +1008,15 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
 
 // ---- the GEMM's choice of tile ----
 // A call runs ceil(tiles / CUs) rounds of one tile per CU (the smallest tiles share a CU, at the same cost), and us0 +
-// us1 * I / 1024 is a tile's time, fitted over the qkv and o_proj shapes at 9 to 2048 tokens (int8; the other forms are
-// within 25 % of it, tile against tile closer). The XH tiles' rounding launch costs 8 us + 1.5 us per million
-// activations, so they pay where a call runs several rounds or the tile is large: qkv at 777 tokens 48.0 us with
-// 128 x 128 XH, 59.5 with the fp32-reading 128 x 128, 55.3 with 144 x 256; at 300 tokens (one round) 32.4 against 29.1.
-// The tile with the smallest estimate runs. Against every tile at 13 token counts on both shapes it was the fastest or
-// within 4 %.
+// us1 * I / 1024 is a tile's time, fitted to every tile at 9 to 2048 tokens on the qkv and o_proj shapes, int8 and int4
+// (int6 is within 35 %, tile against tile closer; fp16 weights cost the fp32-reading tiles 15 % more than the XH ones:
+// o_proj at 1300 tokens 58 us with 128 x 128 against 48 with 128 x 128 XH, int8 49 against 54). The XH tiles' rounding
+// launch costs 8 us + 1 us per million activations, so they pay where a call runs several rounds or the tile is large
+// (o_proj at 3000 tokens, int8: 95 -> 80). The tile with the smallest
+// estimate runs: at 12 token counts from 12 to 900 on both shapes and forms it was the fastest or within 5 %. The 48
+// token tiles fill the chip where those of 32 and 64 leave a part of it or a round short (int8 / int4, us, with the best
+// of the others against them): qkv at 40 tokens 13.0 / 14.4 -> 12.3 / 12.2, at 100 20.2 / 20.8 -> 17.3 / 20.3; o_proj
+// at 300 21.9 / 25.2 -> 21.3 / 21.2, at 600 33.7 / 37.0 -> 26.8 / 33.9. 112 x 128 was never the best by more than 1 %.
 struct GemmCost { int BM, BN; bool xh; int BK; float us0, us1; };
 using GemmA = GemmTile<9, 4, 2, 4, 1, 2, 1, true>;  // 288 x 256
 using GemmB = GemmTile<9, 2, 1, 8, 1, 2, 1, true>;  // 144 x 256
@@ -1026,11 +1029,14 @@ using GemmH = GemmTile<4, 2, 1, 1, 8, 1, 2>;        // 64 x 32
 using GemmI = GemmTile<2, 2, 1, 1, 8, 1, 1, false, 4>;       // 32 x 32
 using GemmJ = GemmTile<2, 1, 1, 1, 8, 1, 2, false, 4>;       // 32 x 16
 using GemmK = GemmTile<1, 1, 1, 1, 8, 1, 2, false, 4>;       // 16 x 16
+using GemmL = GemmTile<4, 3, 2, 1, 4, 1, 2>;        // 128 x 48
+using GemmM = GemmTile<2, 3, 2, 1, 4, 1, 2>;        // 64 x 48
 template <class C> constexpr GemmCost gemm_cost(float us0, float us1) { return {C::BM, C::BN, C::XH, C::BK, us0, us1}; }
 constexpr GemmCost GEMM_COST[] = {
-    gemm_cost<GemmA>(10.f, 33.f), gemm_cost<GemmB>(13.f, 17.f), gemm_cost<GemmC>(17.f, 10.8f), gemm_cost<GemmD>(5.5f, 11.f),
-    gemm_cost<GemmE>(2.f, 9.f),   gemm_cost<GemmF>(3.f, 7.f),   gemm_cost<GemmG>(1.2f, 4.25f), gemm_cost<GemmH>(1.5f, 2.5f),
-    gemm_cost<GemmI>(1.f, 1.75f), gemm_cost<GemmJ>(.7f, 1.15f), gemm_cost<GemmK>(.2f, 1.f)};
+    gemm_cost<GemmA>(10.f, 33.f),   gemm_cost<GemmB>(8.f, 20.7f),   gemm_cost<GemmC>(6.f, 16.6f), gemm_cost<GemmD>(6.6f, 11.f),
+    gemm_cost<GemmE>(4.f, 8.5f),    gemm_cost<GemmF>(5.6f, 7.37f),  gemm_cost<GemmG>(3.6f, 4.87f), gemm_cost<GemmH>(4.4f, 2.71f),
+    gemm_cost<GemmI>(.8f, 2.42f),   gemm_cost<GemmJ>(.4f, 1.94f),   gemm_cost<GemmK>(1.f, 1.44f), gemm_cost<GemmL>(6.f, 5.61f),
+    gemm_cost<GemmM>(2.f, 4.02f)};
 
 template <int FMT, class C>
 void launch_gemm_t(const void* W, const uint8_t* Wh, const float* s, const void* X, float* Y, int S, int I, int O,
@@ -1047,7 +1053,7 @@ void launch_gemm_t(const void* W, const uint8_t* Wh, const float* s, const void*
     MOEX_LAUNCHED();
 }
 
-int gemm_pick(int S, int I, int O, bool xh) {
+int gemm_pick(int S, int I, int O, bool xh, bool f16) {
     const int cus = dense_cus();
     int best = -1;
     float us = 0.f;
@@ -1057,8 +1063,8 @@ int gemm_pick(int S, int I, int O, bool xh) {
         // a tile's offsets stay within 32 bits (the smallest tile's are 64-bit)
         if (t.BM * t.BN > 256 && (size_t)std::max(t.BM, t.BN) * I * 4 >= (size_t)1 << 32) continue;
         const size_t tiles = (size_t)((O + t.BM - 1) / t.BM) * ((S + t.BN - 1) / t.BN);
-        const float e = (float)((tiles + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f)) +
-                        (t.xh ? 8.f + 1.5e-6f * (float)S * (float)I : 0.f);
+        const float e = (float)((tiles + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f)) *
+                            (f16 && !t.xh ? 1.15f : 1.f) + (t.xh ? 8.f + 1e-6f * (float)S * (float)I : 0.f);
         if (best < 0 || e < us) {
             best = c;
             us = e;
@@ -1070,7 +1076,7 @@ int gemm_pick(int S, int I, int O, bool xh) {
 template <int FMT>
 void launch_gemm(const void* W, const uint8_t* Wh, const float* s, const float* X, float* Y, int S, int I, int O,
                  hipStream_t st) {
-    int c = gemm_pick(S, I, O, true);
+    int c = gemm_pick(S, I, O, true, FMT == MF_F16);
     const void* Xg = X;
     if (GEMM_COST[c].xh) {
         // quiet: while the workspace cannot be had (a capture before an eager call of this size, or no memory) a tile
@@ -1083,7 +1089,7 @@ void launch_gemm(const void* W, const uint8_t* Wh, const float* s, const float* 
             MOEX_LAUNCHED();
             Xg = Xh;
         } else {
-            c = gemm_pick(S, I, O, false);
+            c = gemm_pick(S, I, O, false, FMT == MF_F16);
         }
     }
     switch (c) {
@@ -1097,7 +1103,9 @@ void launch_gemm(const void* W, const uint8_t* Wh, const float* s, const float* 
         case 7: launch_gemm_t<FMT, GemmH>(W, Wh, s, Xg, Y, S, I, O, st); break;
         case 8: launch_gemm_t<FMT, GemmI>(W, Wh, s, Xg, Y, S, I, O, st); break;
         case 9: launch_gemm_t<FMT, GemmJ>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        default: launch_gemm_t<FMT, GemmK>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 10: launch_gemm_t<FMT, GemmK>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        case 11: launch_gemm_t<FMT, GemmL>(W, Wh, s, Xg, Y, S, I, O, st); break;
+        default: launch_gemm_t<FMT, GemmM>(W, Wh, s, Xg, Y, S, I, O, st); break;
     }
 }
 

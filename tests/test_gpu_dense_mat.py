@@ -186,15 +186,19 @@ def test_int8_mat_routes_to_gemm_i8():
 @pytest.mark.parametrize("O,I,S,shift", [
     (9211, 2048, 2047, 0),   # 288 x 256 tiles, ragged in both directions, O % 4 != 0 (4-byte stores)
     (9212, 1024, 1021, 0),   # 144 x 256
-    (9217, 512, 509, 0),     # 144 x 128
+    (9215, 2048, 397, 0),    # 144 x 128
+    (9217, 512, 509, 0),     # 128 x 128, few K steps (fp16: with fp16 activations)
     (2049, 4096, 1531, 1),   # 128 x 128, output 4 bytes off a 16-byte boundary
     (9215, 2048, 770, 0),    # 128 x 128, fp16 activations
-    (2048, 1088, 650, 0),    # 128 x 64; I % 128 != 0
+    (2048, 1088, 800, 0),    # 128 x 64; I % 128 != 0
+    (2047, 4096, 611, 0),    # 128 x 48
+    (2048, 4160, 299, 1),    # 64 x 48, a ragged last K step
     (2050, 4096, 400, 0),    # 64 x 64
     (2048, 4160, 161, 1),    # 64 x 32, a ragged last K step (I % 256 = 64)
     (2047, 320, 65, 0),      # 32 x 32, K steps 1.25
     (9216, 192, 17, 0),      # 32 x 16, I below one K step
-    (33, 64, 11, 0),         # 16 x 16, the smallest I of the group-scaled forms
+    (2047, 4096, 25, 0),     # 16 x 16
+    (33, 64, 11, 0),         # 32 x 16, the smallest I of the group-scaled forms
 ])
 def test_gemm_tiles(fmt, O, I, S, shift):
     """Every tile of the GEMM at its edges (the tile is chosen by size; the comments name it): ragged O and S, a last K

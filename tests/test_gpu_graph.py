@@ -133,7 +133,7 @@ def test_fa_images_and_dense_graph_replays():
 
 def test_dense_forms_graph_replays():
     """The int4 / int6 / fp16 matrix forms captured on a stream after one eager call (which allocates the GEMM's
-    workspaces): int4 GEMV, int6 four-row GEMV pass, fp16 GEMM with a K split and int4 GEMM, every replay bit-identical
+    workspaces): int4 GEMV, int6 four-row GEMV pass, fp16 GEMM and int4 GEMM, every replay bit-identical
     to the eager outputs, with eager work in between."""
     import torch
     import moex_amd as M
@@ -154,7 +154,7 @@ def test_dense_forms_graph_replays():
     def run(ys):
         M.gemv(m4, x[0], ys[0], I, O, st)
         M.gemm(m6, x[:4], ys[1], 4, I, O, st)
-        M.gemm(mf, x[:16], ys[2], 16, I, O, st)   # 16 tiles: K split over workgroups, summed by a second kernel
+        M.gemm(mf, x[:16], ys[2], 16, I, O, st)
         M.gemm(m4, x, ys[3], 64, I, O, st)
 
     shapes = [(O,), (4, O), (16, O), (64, O)]

@@ -198,21 +198,22 @@ __global__ void __launch_bounds__(64 * GV_WAVES) gemv_kernel(const int8_t* __res
 // 4 input rows) for many. One or two input rows are read by each lane straight from L2; more are copied into LDS once
 // per workgroup by DMA (float4 e of the rows in slot e ^ (e / 8) % 4: the lanes of a read, 64 bytes apart, then hit
 // different banks), as eight wavefronts each reading 4 or 8 rows from L2 took longer than the weights, and their
-// values left no registers for the weights in flight. Graph-replayed over rotating weights, us, before -> now (before:
+// values left no registers for the weights in flight. The wait for the transfers counts on the R weight loads being
+// issued after them: q is no __restrict__ pointer, since loads through a noalias, read-only kernel argument count as
+// loads of constant memory, which the compiler may move across the transfers' asm statements. Graph-replayed over rotating weights, us, before -> now (before:
 // every input row from L2, 8 rows a wavefront, qkv's rows not split, six cross-lane steps per sum):
 //   input rows          1           2           3            4            6            8
 //   qkv  9216 x 2048    7.0 -> 5.2  8.7 -> 6.0  12.3 -> 6.6  21.0 -> 7.7  16.3 -> 9.2  20.9 -> 10.6
 //   o    2048 x 4096    4.2 -> 3.9  4.8 -> 4.9  5.4 -> 4.8   6.2 -> 5.1   7.7 -> 6.1   9.3 -> 6.7
 template <int NT, int R>
-__global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* __restrict__ q, const float* __restrict__ s,
+__global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q, const float* __restrict__ s,
                                                                  const float* __restrict__ x, float* __restrict__ y,
                                                                  int I, int O, int KS) {
     constexpr bool XL = NT > 2;
     extern __shared__ __align__(16) float xs[];  // XL: the input rows [NT][I]; then the partial sums [GV_WAVES][NT * R]
     float* red = xs + (XL ? NT * I : 0);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ngroups = (O + R - 1) / R, gpw = GV_WAVES / KS;
-    const int part = wv % KS, slice = I / 16 / KS, cb = part * slice;
+    const int gpw = GV_WAVES / KS, part = wv % KS, slice = I / 16 / KS, cb = part * slice;
     const int g = blockIdx.x * gpw + wv / KS;
     const bool on = lane < slice;
     const int c = min(cb + lane, I / 16 - 1);
@@ -325,6 +326,15 @@ __device__ __forceinline__ void wstage_load_at(WStage& w, const void* W, const u
         w.sc = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(s + base / 64) + off / 64 * 4);
     }
 }
+// a use of everything that wstage_load_at has loaded
+template <int FMT>
+__device__ __forceinline__ void wstage_use(const WStage& w) {
+    if constexpr (FMT == MF_I8) asm volatile("" ::"v"(w.a.x), "v"(w.a.y), "v"(w.a.z), "v"(w.a.w));
+    else if constexpr (FMT == MF_F16)
+        asm volatile("" ::"v"(w.a.x), "v"(w.a.y), "v"(w.a.z), "v"(w.a.w), "v"(w.b.x), "v"(w.b.y), "v"(w.b.z), "v"(w.b.w));
+    else asm volatile("" ::"v"(w.a.x), "v"(w.a.y), "v"(w.sc));
+    if constexpr (FMT == MF_Q6) asm volatile("" ::"v"(w.h));
+}
 template <int FMT>
 __device__ __forceinline__ void wstage_widen(const WStage& w, bool ok, uint32_t (&h)[8]) {
     if constexpr (FMT == MF_I8) {
@@ -384,9 +394,14 @@ struct GemmTile {
     static_assert(!XH || BK <= 512, "a transfer holds whole rows of a K step");
 };
 template <int N> __device__ __forceinline__ void gemm_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// The XH wait counts on a K step's weight loads being issued between its transfers and the wait: W, Wh and s are no
+// __restrict__ pointers there (see gemv1_kernel), and every load has a use, the last ones after the loop. The other tiles
+// wait for nothing by count and leave the order to the compiler.
+template <class C, class T>
+using weight_ptr = std::conditional_t<C::XH, const T*, const T* __restrict__>;
 template <int FMT, class C>
-__global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(const void* __restrict__ W, const uint8_t* __restrict__ Wh,
-                                                           const float* __restrict__ s, const void* __restrict__ Xv,
+__global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, void> W, weight_ptr<C, uint8_t> Wh,
+                                                           weight_ptr<C, float> s, const void* __restrict__ Xv,
                                                            float* __restrict__ Y, int S, int I, int O, int vec) {
     extern __shared__ __align__(16) _Float16 gl[];
     const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
@@ -546,7 +561,12 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(const void* __re
     };
     if (wv < 4) steps(std::true_type{});
     else steps(std::false_type{});
-    if constexpr (!C::XH) {
+    if constexpr (C::XH) {
+#pragma unroll
+        for (int p = 0; p < C::PD; p++)
+#pragma unroll
+            for (int u = 0; u < C::NW; u++) wstage_use<FMT>(wst[p][u]);
+    } else {
         if (nk * C::BK < I) {  // the ragged last step: inputs past I are zero in both operands
             load(wst[0], xst[0], nk, std::true_type{});
             store(wst[0], xst[0], nk, std::true_type{});

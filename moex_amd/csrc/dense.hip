@@ -220,10 +220,20 @@ __global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q
     constexpr int TB = NT < 4 ? NT : 4;
     float4 xv[TB][4];
     if constexpr (XL) {
-        const int n = NT * I / 256;  // 1 KB transfers
-        for (int i = wv; i < n; i += GV_WAVES) {
-            const uint32_t e = 64 * i + lane;
-            dma16x(x, 16 * (e ^ ((e >> 3) & 3)), reinterpret_cast<const unsigned char*>(xs) + 1024 * i);
+        if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+            const int n = NT * I / 256;  // 1 KB transfers
+            for (int i = wv; i < n; i += GV_WAVES) {
+                const uint32_t e = 64 * i + lane;
+                dma16x(x, 16 * (e ^ ((e >> 3) & 3)), reinterpret_cast<const unsigned char*>(xs) + 1024 * i);
+            }
+        } else {
+            // rows off a 16-byte boundary: the same slots by loads and LDS writes (8 rows: qkv 10.8 us against 10.6 with
+            // transfers, o 6.9 against 6.7; gemv_kernel, which ran them before, 26.2 and 14.2)
+#pragma unroll 4
+            for (uint32_t e = tid; e < (uint32_t)NT * I / 4; e += 64 * GV_WAVES) {
+                const float* p = x + 4 * (e ^ ((e >> 3) & 3));
+                reinterpret_cast<float4*>(xs)[e] = make_float4(p[0], p[1], p[2], p[3]);
+            }
         }
     } else {
 #pragma unroll
@@ -236,7 +246,7 @@ __global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q
     for (int r = 0; r < R; r++)  // rows past the last repeat it
         w[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q + (size_t)min(g * R + r, O - 1) * I) + c);
     // XL: this wavefront's transfers have landed when only its R weight loads are in flight
-    if constexpr (XL) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(R) : "memory");
+    if constexpr (XL) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(R) : "memory");
     float acc[NT * R];
 #pragma unroll
     for (int t0 = 0; t0 < NT; t0 += TB) {  // input rows in groups whose values fit the registers
@@ -649,7 +659,7 @@ __global__ void __launch_bounds__(256) round_f16_kernel(const float4* __restrict
 template <int NT, int R>
 bool launch_gemv1_r(const int8_t* q, const float* s, const float* x, float* y, int I, int O, int ks, hipStream_t st) {
     const size_t lds = (NT > 2 ? (size_t)NT * I * 4 : 0) + (size_t)GV_WAVES * NT * R * 4;
-    if (lds > 160 * 1024 || (NT > 2 && (reinterpret_cast<uintptr_t>(x) & 15))) return false;  // 16-byte transfers
+    if (lds > 160 * 1024) return false;
     static bool once = [] {
         MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv1_kernel<NT, R>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));

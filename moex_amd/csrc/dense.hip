@@ -6,10 +6,10 @@
 //   quantize_rows_kernel   fp16 [O][I] -> int8 [O][I] + scale absmax/127 per row (bit-exact: IEEE divide, rint).
 //   gemv1_kernel<NT, R>    y[t][o] = s[o] * sum_i q[o][i] x[t][i] for NT <= 8 rows of x, fp32 sums. HBM-bound on the
 //                          weights, which are read once for all NT rows. A wavefront takes R weight rows over 1/KS of
-//                          I, a lane 16 weights of each, sums them in order and over the wavefront, and the KS parts
-//                          of a row are added in LDS. KS and the sum order depend on O and I only, so any row of a
-//                          multi-row call is bit-identical to the same row alone.
-//   gemv_kernel<NT>        The same for parts of more than 64 16-weight chunks, which a lane walks in steps.
+//                          I, a lane 16 weights of each (32 where I is 16384), sums them in order and over
+//                          the wavefront, and the KS parts of a row are added in LDS. KS and the sum order depend on
+//                          O and I only, so any row of a multi-row call is bit-identical to the same row alone.
+//   gemv_kernel<NT>        The same for longer parts, which a lane walks in steps.
 //   gemm_tile_kernel       S > 8 rows (prefill): Y = X . W^T * s on v_mfma_f32_16x16x32_f16. Weights are widened to
 //                          fp16 exactly (integers), activations rounded to fp16 as the reference does
 //                          (kernels.cuh:306-307), fp32 accumulation, the row scale applied last. One workgroup per
@@ -192,8 +192,9 @@ __global__ void __launch_bounds__(64 * GV_WAVES) gemv_kernel(const int8_t* __res
 #undef GV_LOAD
 }
 
-// The same product when a part of a row is at most 64 chunks, one load a lane (the attention's qkv and o shapes): a
-// wavefront takes R rows, sends all of its loads before any product and needs no loop. Same sum order as gemv_kernel.
+// The same product when a part of a row is at most 64 U chunks, U loads a lane (U = 1: I up to 8192, the attention's qkv and
+// o shapes among them; U = 2: 16384, where at most two input rows come at once): a wavefront takes R rows, sends all
+// of its loads before any product and needs no loop. Same sum order as gemv_kernel.
 // It is bound by the weight stream and the launch for few input rows, by the FMAs (and the widening, once per group of
 // 4 input rows) for many. One or two input rows are read by each lane straight from L2; more are copied into LDS once
 // per workgroup by DMA (float4 e of the rows in slot e ^ (e / 8) % 4: the lanes of a read, 64 bytes apart, then hit
@@ -205,7 +206,7 @@ __global__ void __launch_bounds__(64 * GV_WAVES) gemv_kernel(const int8_t* __res
 //   input rows          1           2           3            4            6            8
 //   qkv  9216 x 2048    7.0 -> 5.2  8.7 -> 6.0  12.3 -> 6.6  21.0 -> 7.7  16.3 -> 9.2  20.9 -> 10.6
 //   o    2048 x 4096    4.2 -> 3.9  4.8 -> 4.9  5.4 -> 4.8   6.2 -> 5.1   7.7 -> 6.1   9.3 -> 6.7
-template <int NT, int R>
+template <int NT, int R, int U>
 __global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q, const float* __restrict__ s,
                                                                  const float* __restrict__ x, float* __restrict__ y,
                                                                  int I, int O, int KS) {
@@ -215,10 +216,12 @@ __global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int gpw = GV_WAVES / KS, part = wv % KS, slice = I / 16 / KS, cb = part * slice;
     const int g = blockIdx.x * gpw + wv / KS;
-    const bool on = lane < slice;
-    const int c = min(cb + lane, I / 16 - 1);
+    static_assert(U == 1 || !XL, "two loads a lane: input rows from L2");
+    int c[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) c[u] = min(cb + 64 * u + lane, I / 16 - 1);
     constexpr int TB = NT < 4 ? NT : 4;
-    float4 xv[TB][4];
+    float4 xv[U][TB][4];
     if constexpr (XL) {
         if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
             const int n = NT * I / 256;  // 1 KB transfers
@@ -237,14 +240,18 @@ __global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q
         }
     } else {
 #pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int d = 0; d < 4; d++) xv[t][d] = reinterpret_cast<const float4*>(x + (size_t)t * I)[4 * c + d];
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) xv[u][t][d] = reinterpret_cast<const float4*>(x + (size_t)t * I)[4 * c[u] + d];
     }
-    u32x4 w[R];
+    u32x4 w[U][R];
 #pragma unroll
-    for (int r = 0; r < R; r++)  // rows past the last repeat it
-        w[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q + (size_t)min(g * R + r, O - 1) * I) + c);
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int r = 0; r < R; r++)  // rows past the last repeat it
+            w[u][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q + (size_t)min(g * R + r, O - 1) * I) + c[u]);
     // XL: this wavefront's transfers have landed when only its R weight loads are in flight
     if constexpr (XL) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(R) : "memory");
     float acc[NT * R];
@@ -255,30 +262,36 @@ __global__ void __launch_bounds__(64 * GV_WAVES, 2) gemv1_kernel(const int8_t* q
             for (int t = t0; t < NT && t < t0 + TB; t++)
 #pragma unroll
                 for (int d = 0; d < 4; d++) {
-                    const uint32_t e = t * (I / 4) + 4 * c + d;
-                    xv[t - t0][d] = reinterpret_cast<const float4*>(xs)[e ^ ((e >> 3) & 3)];
+                    const uint32_t e = t * (I / 4) + 4 * c[0] + d;
+                    xv[0][t - t0][d] = reinterpret_cast<const float4*>(xs)[e ^ ((e >> 3) & 3)];
                 }
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
             float a[TB];
 #pragma unroll
-            for (int t = 0; t < TB; t++) a[t] = 0.f;
+            for (int u = 0; u < U; u++) {
 #pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const uint32_t wd = w[r][d];
-                const float w0 = (float)(int8_t)wd, w1 = (float)(int8_t)(wd >> 8), w2 = (float)(int8_t)(wd >> 16),
-                            w3 = (float)(int8_t)(wd >> 24);
+                for (int t = 0; t < TB; t++) a[t] = u ? acc[(t0 + t) * R + r] : 0.f;
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const uint32_t wd = w[u][r][d];
+                    const float w0 = (float)(int8_t)wd, w1 = (float)(int8_t)(wd >> 8), w2 = (float)(int8_t)(wd >> 16),
+                                w3 = (float)(int8_t)(wd >> 24);
+#pragma unroll
+                    for (int t = 0; t < TB && t0 + t < NT; t++) {
+                        a[t] = fmaf(w0, xv[u][t][d].x, a[t]);
+                        a[t] = fmaf(w1, xv[u][t][d].y, a[t]);
+                        a[t] = fmaf(w2, xv[u][t][d].z, a[t]);
+                        a[t] = fmaf(w3, xv[u][t][d].w, a[t]);
+                    }
+                }
 #pragma unroll
                 for (int t = 0; t < TB && t0 + t < NT; t++) {
-                    a[t] = fmaf(w0, xv[t][d].x, a[t]);
-                    a[t] = fmaf(w1, xv[t][d].y, a[t]);
-                    a[t] = fmaf(w2, xv[t][d].z, a[t]);
-                    a[t] = fmaf(w3, xv[t][d].w, a[t]);
+                    float& s_ = acc[(t0 + t) * R + r];
+                    s_ = 64 * u + lane < slice ? a[t] : u ? s_ : 0.f;  // lanes past the part add nothing
                 }
             }
-#pragma unroll
-            for (int t = 0; t < TB && t0 + t < NT; t++) acc[(t0 + t) * R + r] = on ? a[t] : 0.f;
         }
         if constexpr (NT > TB) asm volatile("" ::: "memory");  // the next group's values are read after these are used
     }
@@ -656,42 +669,51 @@ __global__ void __launch_bounds__(256) round_f16_kernel(const float4* __restrict
     }
 }
 
-template <int NT, int R>
+template <int NT, int R, int U>
 bool launch_gemv1_r(const int8_t* q, const float* s, const float* x, float* y, int I, int O, int ks, hipStream_t st) {
     const size_t lds = (NT > 2 ? (size_t)NT * I * 4 : 0) + (size_t)GV_WAVES * NT * R * 4;
     if (lds > 160 * 1024) return false;
     static bool once = [] {
-        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv1_kernel<NT, R>),
+        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemv1_kernel<NT, R, U>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         return true;
     }();
     (void)once;
     const int gpw = GV_WAVES / ks, wgs = ((O + R - 1) / R + gpw - 1) / gpw;
-    hipLaunchKernelGGL((gemv1_kernel<NT, R>), dim3(wgs), dim3(64 * GV_WAVES), lds, st, q, s, x, y, I, O, ks);
+    hipLaunchKernelGGL((gemv1_kernel<NT, R, U>), dim3(wgs), dim3(64 * GV_WAVES), lds, st, q, s, x, y, I, O, ks);
     MOEX_LAUNCHED();
     return true;
 }
-template <int NT>
+template <int NT, int U>
 bool launch_gemv1(const int8_t* q, const float* s, const float* x, float* y, int I, int O, int ks, int cus,
                   hipStream_t st) {
     // the rows per wavefront with the cheapest rounds over the chip: R rows and a fixed part of about two rows' time each.
-    // Of 2, 3, 4, 6, 9 and 12 it was the fastest or within 12 % of it for 1 to 8 input rows on qkv (9) and o_proj (4)
+    // Of 2, 3, 4, 6, 9 and 12 it was the fastest or within 12 % of it for 1 to 8 input rows on qkv (9) and o_proj (4).
+    // Two loads a lane (16384 inputs) leave registers for 4 and pay for one round only, where the looped kernel has too few
+    // workgroups (us, looped -> so, 1 / 2 input rows: 512 x 16384 7.7 / 11.5 -> 5.1 / 5.7; 2 rounds, 2048 x 16384, 1 row 10.0 ->
+    // 10.7)
     int best = 0;
     long cost = 0;
     for (int R : {2, 3, 4, 6, 9, 12}) {
+        if (U > 1 && R > 4) break;
         const long gpw = GV_WAVES / ks, wgs = ((O + R - 1) / R + gpw - 1) / gpw, e = (wgs + cus - 1) / cus * (R + 2);
         if (!best || e < cost) {
             best = R;
             cost = e;
         }
     }
+    if (U > 1 && cost > best + 2) return false;
+    if constexpr (U == 1) {
+        switch (best) {
+            case 6: return launch_gemv1_r<NT, 6, U>(q, s, x, y, I, O, ks, st);
+            case 9: return launch_gemv1_r<NT, 9, U>(q, s, x, y, I, O, ks, st);
+            case 12: return launch_gemv1_r<NT, 12, U>(q, s, x, y, I, O, ks, st);
+        }
+    }
     switch (best) {
-        case 2: return launch_gemv1_r<NT, 2>(q, s, x, y, I, O, ks, st);
-        case 3: return launch_gemv1_r<NT, 3>(q, s, x, y, I, O, ks, st);
-        case 4: return launch_gemv1_r<NT, 4>(q, s, x, y, I, O, ks, st);
-        case 6: return launch_gemv1_r<NT, 6>(q, s, x, y, I, O, ks, st);
-        case 9: return launch_gemv1_r<NT, 9>(q, s, x, y, I, O, ks, st);
-        default: return launch_gemv1_r<NT, 12>(q, s, x, y, I, O, ks, st);
+        case 2: return launch_gemv1_r<NT, 2, U>(q, s, x, y, I, O, ks, st);
+        case 3: return launch_gemv1_r<NT, 3, U>(q, s, x, y, I, O, ks, st);
+        default: return launch_gemv1_r<NT, 4, U>(q, s, x, y, I, O, ks, st);
     }
 }
 
@@ -704,8 +726,12 @@ void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, in
     }();
     (void)once;
     const int groups = (O + GV_R - 1) / GV_R;
-    int ks = 1;  // split each row over up to 8 wavefronts until 8 wavefronts per CU have 8 rows each
-    while (ks < GV_WAVES && groups * ks < 2048 && (I / 16) % (128 * ks) == 0) ks *= 2;
+    // split each row over up to 8 wavefronts until 8 wavefronts per CU have 8 rows each, and where I allows it until a part
+    // is one load a lane (I % 512 == 0, so the parts are equal). With longer parts left to the looped kernel, us, then -> now,
+    // 1 / 2 / 4 / 8 input rows: 9216 x 1536 7.0 / 8.7 / 12.3 / 19.1 -> 4.7 / 5.5 / 7.1 / 10.0; 16384 x 2048 9.3 / 11.8 / 17.8 /
+    // 27.5 -> 7.7 / 9.0 / 10.9 / 19.3; 12288 x 4096 13.8 / 18.4 / 28.3 / 44.1 -> 10.3 / 12.8 / 14.1 / 25.5
+    int ks = 1;
+    while (ks < GV_WAVES && ((groups * ks < 2048 && (I / 16) % (128 * ks) == 0) || (I <= 8192 && I / 16 / ks > 64))) ks *= 2;
     static const int cus = [] {
         int dev = 0, v = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
@@ -713,7 +739,10 @@ void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, in
             return v;
         return 256;
     }();
-    if (I / 16 / ks <= 64 && launch_gemv1<NT>(q, s, x, y, I, O, ks, cus, st)) return;
+    if (I / 16 / ks <= 64 && launch_gemv1<NT, 1>(q, s, x, y, I, O, ks, cus, st)) return;
+    if constexpr (NT <= 2) {
+        if (I / 16 / ks <= 128 && launch_gemv1<NT, 2>(q, s, x, y, I, O, ks, cus, st)) return;
+    }
     const int nb = std::min(cus, groups * ks);
     const size_t lds = (size_t)NT * I * 4 + GV_WAVES * NT * GV_R * 4;
     hipLaunchKernelGGL(gemv_kernel<NT>, dim3(nb), dim3(64 * GV_WAVES), lds, st, q, s, x, y, I, O, ks);

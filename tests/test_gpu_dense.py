@@ -162,7 +162,7 @@ def test_gemm_both_kernels_ragged():
 
 
 def test_many_row_groups():
-    """O large enough that a wavefront takes several row groups (the looped GEMV: lm_head-like shapes), 1 and 3 rows."""
+    """More row groups than one round of workgroups (lm_head-like shapes), 1 and 3 rows."""
     import torch
     import moex_amd as M
     O, I = 40000, 1024
@@ -184,7 +184,7 @@ def test_many_row_groups():
 @pytest.mark.parametrize("O,I,shift", [
     (1001, 512, 0),    # half of a part's lanes idle, O not a multiple of any row group
     (12301, 2048, 0),  # more row groups than one round of workgroups
-    (700, 1536, 0),    # parts of more than 64 chunks: the looped kernel
+    (700, 1536, 0),    # parts of 48 chunks
     (9216, 1024, 1),   # input rows 4 bytes off a 16-byte boundary: no transfers into LDS
     (130, 8192, 0),    # the most parts a row is split in
 ])
@@ -245,3 +245,49 @@ def test_gemv_unaligned_rows_time(O, I, S):
     t = [_graph_us(lambda st, x=buf[sh:sh + S * I]: M.gemm_i8(q, s, x, Y, S, I, O, st)) for sh in (0, 1)]
     print(f"gemv {O}x{I} {S} rows: aligned {t[0]:.2f} us, unaligned {t[1]:.2f} us", flush=True)
     assert t[1] <= 1.5 * t[0]
+
+
+@pytest.mark.parametrize("O,I,than,S,most", [
+    (9216, 1536, (9216, 2048), 1, 1.2), (9216, 1536, (9216, 2048), 4, 1.2), (9216, 1536, (9216, 2048), 8, 1.2),  # 96 chunks
+    (16384, 2048, (16000, 2048), 4, 1.2),                                  # 128 chunks, 2048 groups of 8 rows
+    (512, 16384, (1024, 8192), 1, 1.6), (512, 16384, (1024, 8192), 2, 1.6),  # 1024 chunks: two loads a lane
+])
+def test_gemv_long_parts_time(O, I, than, S, most):
+    """Rows whose parts were more than one load a lane take about as long as a matrix of as many weights whose parts were
+    not (measured 0.9 to 1.05, with two loads a lane 1.2; the looped kernel took 1.4 to 2.5 times as long)."""
+    import torch
+    import moex_amd as M
+    us = []
+    for o, i in ((O, I), than):
+        rng = np.random.default_rng(o + i)
+        q, s = _quantize((rng.standard_normal((o, i)) * 0.02).astype(np.float16))
+        x, Y = torch.randn((S, i), device="cuda"), torch.empty((S, o), device="cuda")
+        us.append(_graph_us(lambda st: M.gemm_i8(q, s, x, Y, S, i, o, st)))
+    print(f"gemv {S} rows: {O}x{I} {us[0]:.2f} us, {than} {us[1]:.2f} us", flush=True)
+    assert us[0] <= most * us[1]
+
+
+@pytest.mark.parametrize("O,I", [(4000, 512), (6001, 512), (8001, 512), (12001, 512), (18001, 512), (24001, 512),
+                                 (8001, 2048), (500, 16384), (767, 16384), (1021, 16384), (130, 12288), (2000, 10240)])
+def test_gemv_every_row_group(O, I):
+    """Every number of rows a wavefront takes (2, 3, 4, 6, 9 and 12, chosen by O; at 16384 inputs 2 to 4 with two loads a
+    lane; 12288 and 10240 inputs take the looped kernel) at every number of input rows: a row has the bits of the one-row call and is within
+    1e-5 of the exact product (fp32 sums of at most 16384 products)."""
+    import torch
+    import moex_amd as M
+    n = min(8, 40448 // I)
+    g = torch.Generator(device="cuda").manual_seed(O + I)
+    q = torch.randint(-127, 128, (O, I), dtype=torch.int8, device="cuda", generator=g)
+    s = torch.rand(O, device="cuda", generator=g) * 0.01 + 1e-3
+    x = torch.randn((n, I), device="cuda", generator=g)
+    one = torch.full((n, O), float("nan"), device="cuda")
+    for t in range(n):
+        M.gemv_i8(q, s, x[t], one[t], I, O)
+    for S in range(2, n + 1):
+        Y = torch.full((S + 1, O), 123.0, device="cuda")
+        M.gemm_i8(q, s, x, Y, S, I, O)
+        torch.cuda.synchronize()
+        assert torch.equal(Y[:S], one[:S]), S
+        assert bool((Y[S] == 123.0).all()), S
+    assert _rel(one.cpu().numpy().astype(np.float64),
+                orc.dense_i8_f64(q.cpu().numpy(), s.cpu().numpy(), x.cpu().numpy())) < 1e-5

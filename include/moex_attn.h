@@ -23,13 +23,14 @@
  * combine instead, with a workspace of T * H * ns * 1032 bytes for their partials (ns = moex_gqa_splits(T, KV,
  * moex_decode_splits(max_t), turbo)). moex_attn_decode with ns == 1 and T <= 2 (the reference's one-split call) runs
  * the split-K kernels too, with its partials in a workspace of T * H * n2 * 1032 bytes (n2 = moex_gqa_splits(T, KV,
- * moex_decode_splits(max_t), turbo); none when n2 == 1). The dense GEMM (moex_dense.h) keeps one more. Each is one per (device, stream), allocated on first use with hipMalloc and grown
- * when a larger call comes. An outgrown buffer is not freed before the process ends, because a HIP graph captured
+ * moex_decode_splits(max_t), turbo); none when n2 == 1). The dense GEMM (moex_dense.h) keeps up to two more. Each is one
+ * per (device, stream), allocated on first use with hipMalloc and grown when a larger call comes. An outgrown buffer is not freed before the process ends, because a HIP graph captured
  * earlier may still replay into it. No workspace is allocated while the stream is being captured: a call that would
  * need to grow one reports hipErrorStreamCaptureUnsupported. So after one eager call of a given max_t and T on a
- * stream, the same call can be captured into a HIP graph. The one exception is the one-split decode step above: while
- * its workspace does not exist yet it is captured with the per-head kernel of the reference (no partials, no
- * allocation, no error), so it can be captured first time as the reference's can. A graph's replays use the capturing stream's workspaces:
+ * stream, the same call can be captured into a HIP graph. The exceptions are the one-split decode step above, which while
+ * its workspace does not exist yet is captured with the per-head kernel of the reference (no partials, no allocation,
+ * no error), so it can be captured first time as the reference's can, and the dense GEMM, which is captured with a tile
+ * that needs none. A graph's replays use the capturing stream's workspaces:
  * replays and eager calls that overlap in time on different streams race on them. moex_attn_workspace_bytes gives
  * the bytes one call needs, moex_workspace_held the bytes held now (for a VRAM audit next to moex_kv_bytes).
  *

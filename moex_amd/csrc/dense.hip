@@ -422,11 +422,16 @@ template <int N> __device__ __forceinline__ void gemm_vm_wait() { asm volatile("
 // wait for nothing by count and leave the order to the compiler.
 template <class C, class T>
 using weight_ptr = std::conditional_t<C::XH, const T*, const T* __restrict__>;
-template <int FMT, class C>
+// SPLIT: workgroup (x, y) takes spp K steps of tile x from spp y on and writes their sums, without the row scales, to the
+// y-th [S][O] of Y. An instance of its own, as the parts' bounds would cost every call 0.2 to 0.4 us. vec_spp: bit 0 says that
+// outputs can be stored 16 bytes at a time, the others are spp; in one word, since with two the grid's size lay past the
+// first 64 bytes of the arguments, another 0.2 us.
+template <int FMT, class C, bool SPLIT>
 __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, void> W, weight_ptr<C, uint8_t> Wh,
                                                            weight_ptr<C, float> s, const void* __restrict__ Xv,
-                                                           float* __restrict__ Y, int S, int I, int O, int vec) {
+                                                           float* __restrict__ Y, int S, int I, int O, int vec_spp) {
     extern __shared__ __align__(16) _Float16 gl[];
+    const int vec = vec_spp & 1, spp = vec_spp >> 1;
     const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nO = (O + C::BM - 1) / C::BM, nt = gridDim.x;
@@ -435,7 +440,8 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
     const int q8 = nt >> 3, r8 = nt & 7, xc = blockIdx.x & 7, xi = blockIdx.x >> 3;
     const int tile = (xc < r8 ? xc * (q8 + 1) : r8 * (q8 + 1) + (xc - r8) * q8) + xi;
     const int o0 = (tile % nO) * C::BM, s0 = (tile / nO) * C::BN;
-    const int nk = I / C::BK;  // whole K steps; a ragged one follows them
+    // the whole K steps [kb, kb + nk); a ragged one follows the last
+    const int kb = SPLIT ? spp * (int)blockIdx.y : 0, nk = SPLIT ? min(spp, I / C::BK - kb) : I / C::BK;
     WStage wst[C::PD][C::NW];
     float4 xst[C::PD][C::NX];
     constexpr int WU = C::BK / 16, XU = C::BK / 4;  // units of a row
@@ -452,7 +458,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
     }
     auto dma = [&](int kt, int buf) {
         if constexpr (C::XH) {
-            const _Float16* base = reinterpret_cast<const _Float16*>(Xv) + (size_t)s0 * I + kt * C::BK;
+            const _Float16* base = reinterpret_cast<const _Float16*>(Xv) + (size_t)s0 * I + (kb + kt) * C::BK;
             const unsigned char* dst = reinterpret_cast<const unsigned char*>(gl + buf * C::STAGE + C::BM * C::LD);
 #pragma unroll
             for (int d = 0; d < C::ND; d++) dma16x(base, xd[d], dst + (wv * C::ND + d) * 1024);
@@ -473,12 +479,12 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
     }
     auto load = [&](WStage(&w)[C::NW], float4(&x)[C::NX], int kt, auto rag) {
         constexpr bool RAG = decltype(rag)::value;
-        const size_t wbase = (size_t)o0 * I + (size_t)kt * C::BK;
-        const char* xb = reinterpret_cast<const char*>(Xv) + ((size_t)s0 * I + (size_t)kt * C::BK) * 4;
+        const size_t wbase = (size_t)o0 * I + (size_t)(kb + kt) * C::BK;
+        const char* xb = reinterpret_cast<const char*>(Xv) + ((size_t)s0 * I + (size_t)(kb + kt) * C::BK) * 4;
 #pragma unroll
         for (int u = 0; u < C::NW; u++) {
             typename C::off_t off = wro[u];  // RAG: inputs past the row's end are read inside it, zeroed when stored
-            if (RAG) off -= max(0, kt * C::BK + 16 * ((tid + 512 * u) % WU) - (I - 16));
+            if (RAG) off -= max(0, (kb + kt) * C::BK + 16 * ((tid + 512 * u) % WU) - (I - 16));
             wstage_load_at<FMT>(w[u], W, Wh, s, wbase, off);
         }
         if constexpr (C::XH) return;
@@ -486,7 +492,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
         for (int u = 0; u < C::NX; u++) {
             if ((C::BN * XU) % 512 != 0 && tid + 512 * u >= C::BN * XU) break;
             typename C::off_t off = xro[u];
-            if (RAG) off -= 4 * max(0, kt * C::BK + 4 * ((tid + 512 * u) % XU) - (I - 4));
+            if (RAG) off -= 4 * max(0, (kb + kt) * C::BK + 4 * ((tid + 512 * u) % XU) - (I - 4));
             x[u] = *reinterpret_cast<const float4*>(xb + off);
         }
     };
@@ -498,7 +504,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
             const int e = tid + 512 * u, r = e / WU, k = 16 * (e % WU);
             if ((C::BM * WU) % 512 != 0 && e >= C::BM * WU) break;
             uint32_t h[8];
-            wstage_widen<FMT>(w[u], !RAG || kt * C::BK + k < I, h);
+            wstage_widen<FMT>(w[u], !RAG || (kb + kt) * C::BK + k < I, h);
             uint4* d = reinterpret_cast<uint4*>(b + r * C::LD + k);
             d[0] = make_uint4(h[0], h[1], h[2], h[3]);
             d[1] = make_uint4(h[4], h[5], h[6], h[7]);
@@ -509,7 +515,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
         for (int u = 0; u < C::NX; u++) {
             const int e = tid + 512 * u, r = e / XU, k = 4 * (e % XU);
             if ((C::BN * XU) % 512 != 0 && e >= C::BN * XU) break;
-            const bool ok = !RAG || kt * C::BK + k < I;
+            const bool ok = !RAG || (kb + kt) * C::BK + k < I;
             const float4 v = x[u];
             *reinterpret_cast<uint2*>(b + r * C::LD + k) =
                 make_uint2(ok ? h22u(half2_t{(_Float16)v.x, (_Float16)v.y}) : 0u, ok ? h22u(half2_t{(_Float16)v.z, (_Float16)v.w}) : 0u);
@@ -590,7 +596,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
 #pragma unroll
             for (int u = 0; u < C::NW; u++) wstage_use<FMT>(wst[p][u]);
     } else {
-        if (nk * C::BK < I) {  // the ragged last step: inputs past I are zero in both operands
+        if ((!SPLIT || nk < spp) && (kb + nk) * C::BK < I) {  // the ragged last step: inputs past I are zero in both operands
             load(wst[0], xst[0], nk, std::true_type{});
             store(wst[0], xst[0], nk, std::true_type{});
             bar();
@@ -598,6 +604,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
             bar();
         }
     }
+    if (SPLIT) Y += (size_t)blockIdx.y * S * O;
     // acc[i][j] element e: weight row wr + 16 i + 4 g + e, token wt + 16 j + m16
     if constexpr (C::KW == 1) {
 #pragma unroll
@@ -605,7 +612,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
             const int o = o0 + wr + 16 * i + 4 * g;
             if (o >= O) continue;
             float sc[4] = {1.f, 1.f, 1.f, 1.f};
-            if constexpr (FMT == MF_I8) {
+            if constexpr (FMT == MF_I8 && !SPLIT) {
 #pragma unroll
                 for (int e = 0; e < 4; e++) sc[e] = s[min(o + e, O - 1)];
             }
@@ -646,7 +653,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
                 a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
             }
             float v[4] = {a.x, a.y, a.z, a.w};
-            if constexpr (FMT == MF_I8) {
+            if constexpr (FMT == MF_I8 && !SPLIT) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) v[i] *= s[min(o + i, O - 1)];
             }
@@ -658,6 +665,15 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
                     if (o + i < O) y[i] = v[i];
             }
         }
+    }
+}
+// The parts of a K split summed in part order (deterministic), times the row scale (int8; s = nullptr: none)
+__global__ void __launch_bounds__(256) gemm_reduce_kernel(const float* __restrict__ part, const float* __restrict__ s,
+                                                          float* __restrict__ Y, size_t n, int O, int nks) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        float a = part[i];
+        for (int k = 1; k < nks; k++) a += part[k * n + i];
+        Y[i] = s ? a * s[i % O] : a;
     }
 }
 // Activations rounded to fp16 once (round to nearest even, as kernels.cuh:306-307 rounds them inside gemm_i8_k): the
@@ -1076,7 +1092,7 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
 // token tiles fill the chip where those of 32 and 64 leave a part of it or a round short (int8 / int4, us, with the best
 // of the others against them): qkv at 40 tokens 13.0 / 14.4 -> 12.3 / 12.2, at 100 20.2 / 20.8 -> 17.3 / 20.3; o_proj
 // at 300 21.9 / 25.2 -> 21.3 / 21.2, at 600 33.7 / 37.0 -> 26.8 / 33.9. 112 x 128 was never the best by more than 1 %.
-struct GemmCost { int BM, BN; bool xh; int BK; float us0, us1; };
+struct GemmCost { int BM, BN; bool xh; int BK; float us0, us1; bool split; };
 using GemmA = GemmTile<9, 4, 2, 4, 1, 2, 1, true>;  // 288 x 256
 using GemmB = GemmTile<9, 2, 1, 8, 1, 2, 1, true>;  // 144 x 256
 using GemmC = GemmTile<9, 2, 1, 4, 2, 1, 2>;        // 144 x 128
@@ -1090,31 +1106,57 @@ using GemmJ = GemmTile<2, 1, 1, 1, 8, 1, 2, false, 4>;       // 32 x 16
 using GemmK = GemmTile<1, 1, 1, 1, 8, 1, 2, false, 4>;       // 16 x 16
 using GemmL = GemmTile<4, 3, 2, 1, 4, 1, 2>;        // 128 x 48
 using GemmM = GemmTile<2, 3, 2, 1, 4, 1, 2>;        // 64 x 48
-template <class C> constexpr GemmCost gemm_cost(float us0, float us1) { return {C::BM, C::BN, C::XH, C::BK, us0, us1}; }
+// the tiles that are built with a K split too
+template <class C>
+constexpr bool gemm_splits = std::is_same_v<C, GemmE> || std::is_same_v<C, GemmF> || std::is_same_v<C, GemmH> ||
+                             std::is_same_v<C, GemmI> || std::is_same_v<C, GemmK> || std::is_same_v<C, GemmG>;
+template <class C> constexpr GemmCost gemm_cost(float us0, float us1) {
+    return {C::BM, C::BN, C::XH, C::BK, us0, us1, gemm_splits<C>};
+}
 constexpr GemmCost GEMM_COST[] = {
     gemm_cost<GemmA>(10.f, 33.f),   gemm_cost<GemmB>(8.f, 20.7f),   gemm_cost<GemmC>(6.f, 16.6f), gemm_cost<GemmD>(6.6f, 11.f),
     gemm_cost<GemmE>(4.f, 8.5f),    gemm_cost<GemmF>(5.6f, 7.37f),  gemm_cost<GemmG>(3.6f, 4.87f), gemm_cost<GemmH>(4.4f, 2.71f),
     gemm_cost<GemmI>(.8f, 2.42f),   gemm_cost<GemmJ>(.4f, 1.94f),   gemm_cost<GemmK>(1.f, 1.44f), gemm_cost<GemmL>(6.f, 5.61f),
     gemm_cost<GemmM>(2.f, 4.02f)};
 
-template <int FMT, class C>
-void launch_gemm_t(const void* W, const uint8_t* Wh, const float* s, const void* X, float* Y, int S, int I, int O,
-                   hipStream_t st) {
+// nks parts of K (at most: no empty one is left) where the tile has a split instance
+template <int FMT, class C, bool SPLIT>
+int launch_gemm_s(const void* W, const uint8_t* Wh, const float* s, const void* X, float* Y, int S, int I, int O, int nks,
+                  hipStream_t st) {
     static bool once = [] {
-        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tile_kernel<FMT, C>),
+        MOEX_CK(hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tile_kernel<FMT, C, SPLIT>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         return true;
     }();
     (void)once;
     const int tiles = ((O + C::BM - 1) / C::BM) * ((S + C::BN - 1) / C::BN);
     const int vec = O % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;  // 16-byte output stores
-    hipLaunchKernelGGL((gemm_tile_kernel<FMT, C>), dim3(tiles), dim3(512), C::LDS, st, W, Wh, s, X, Y, S, I, O, vec);
+    const int ns = (I + C::BK - 1) / C::BK, spp = (ns + nks - 1) / nks, parts = (ns + spp - 1) / spp;
+    hipLaunchKernelGGL((gemm_tile_kernel<FMT, C, SPLIT>), dim3(tiles, parts), dim3(512), C::LDS, st, W, Wh, s, X, Y, S, I, O,
+                       vec + 2 * spp);
     MOEX_LAUNCHED();
+    return parts;
+}
+template <int FMT, class C>
+void launch_gemm_t(const void* W, const uint8_t* Wh, const float* s, const void* X, float* Y, int S, int I, int O,
+                   hipStream_t st, int& nks) {
+    if constexpr (gemm_splits<C>) {
+        if (nks > 1) {
+            nks = launch_gemm_s<FMT, C, true>(W, Wh, s, X, Y, S, I, O, nks, st);
+            return;
+        }
+    }
+    launch_gemm_s<FMT, C, false>(W, Wh, s, X, Y, S, I, O, 1, st);
 }
 
-int gemm_pick(int S, int I, int O, bool xh, bool f16) {
+// A long K and few tiles: K is split over nks workgroups a tile, parts of 4096 inputs at least (so the attention's shapes never
+// split), where the shorter tiles save more than the second launch (4 us) and the parts' traffic cost, and 5 %. us, whole K in one
+// workgroup -> split, int8 / fp16: 64 x 40448, 9 tokens 57 / 54 -> 13 / 12; 128 x 16384, 100 tokens 24 / 24 -> 12 / 12;
+// 2048 x 16384, 300 tokens 68 / 80 -> 47 / 62, 1100 tokens 179 / 194 -> 121 / 126; 1024 x 8192, 17 tokens 14 / 14 -> 11 / 11.
+struct GemmPick { int tile, nks; };
+GemmPick gemm_pick(int S, int I, int O, bool xh, bool split, bool f16) {
     const int cus = dense_cus();
-    int best = -1;
+    GemmPick best = {-1, 1};
     float us = 0.f;
     for (int c = 0; c < (int)(sizeof(GEMM_COST) / sizeof(GEMM_COST[0])); c++) {
         const GemmCost& t = GEMM_COST[c];
@@ -1122,11 +1164,14 @@ int gemm_pick(int S, int I, int O, bool xh, bool f16) {
         // a tile's offsets stay within 32 bits (the smallest tile's are 64-bit)
         if (t.BM * t.BN > 256 && (size_t)std::max(t.BM, t.BN) * I * 4 >= (size_t)1 << 32) continue;
         const size_t tiles = (size_t)((O + t.BM - 1) / t.BM) * ((S + t.BN - 1) / t.BN);
-        const float e = (float)((tiles + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f)) *
-                            (f16 && !t.xh ? 1.15f : 1.f) + (t.xh ? 8.f + 1e-6f * (float)S * (float)I : 0.f);
-        if (best < 0 || e < us) {
-            best = c;
-            us = e;
+        for (int nks = 1; nks == 1 || (split && t.split && nks <= I / 4096 && tiles * nks <= (size_t)2 * cus); nks++) {
+            float e = (float)((tiles * nks + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f) / (float)nks) *
+                          (f16 && !t.xh ? 1.15f : 1.f) + (t.xh ? 8.f + 1e-6f * (float)S * (float)I : 0.f);
+            if (nks > 1) e = 1.05f * e + 4.f + 2e-6f * (float)nks * (float)S * (float)O;
+            if (best.tile < 0 || e < us) {
+                best = {c, nks};
+                us = e;
+            }
         }
     }
     return best;
@@ -1135,36 +1180,47 @@ int gemm_pick(int S, int I, int O, bool xh, bool f16) {
 template <int FMT>
 void launch_gemm(const void* W, const uint8_t* Wh, const float* s, const float* X, float* Y, int S, int I, int O,
                  hipStream_t st) {
-    int c = gemm_pick(S, I, O, true, FMT == MF_F16);
-    const void* Xg = X;
-    if (GEMM_COST[c].xh) {
-        // quiet: while the workspace cannot be had (a capture before an eager call of this size, or no memory) a tile
-        // that rounds the activations itself runs
-        const size_t n4 = (size_t)S * I / 4;
-        uint2* Xh = reinterpret_cast<uint2*>(stream_workspace(n4 * 8, st, 2, true));
-        if (Xh) {
-            hipLaunchKernelGGL(round_f16_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, st,
-                               reinterpret_cast<const float4*>(X), Xh, n4);
-            MOEX_LAUNCHED();
-            Xg = Xh;
-        } else {
-            c = gemm_pick(S, I, O, false, FMT == MF_F16);
-        }
+    // quiet: while a workspace cannot be had (a capture before an eager call of this size, or no memory) the best tile that
+    // needs none runs: one that rounds the activations itself, over the whole of K
+    const size_t n4 = (size_t)S * I / 4;
+    uint2* Xh = nullptr;
+    float* part = nullptr;
+    GemmPick p;
+    for (bool xh = true, split = true;;) {
+        p = gemm_pick(S, I, O, xh, split, FMT == MF_F16);
+        if (p.nks > 1 && !(part = reinterpret_cast<float*>(stream_workspace((size_t)p.nks * S * O * 4, st, 3, true)))) split = false;
+        else if (GEMM_COST[p.tile].xh && !(Xh = reinterpret_cast<uint2*>(stream_workspace(n4 * 8, st, 2, true)))) xh = false;
+        else break;
     }
-    switch (c) {
-        case 0: launch_gemm_t<FMT, GemmA>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 1: launch_gemm_t<FMT, GemmB>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 2: launch_gemm_t<FMT, GemmC>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 3: launch_gemm_t<FMT, GemmD>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 4: launch_gemm_t<FMT, GemmE>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 5: launch_gemm_t<FMT, GemmF>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 6: launch_gemm_t<FMT, GemmG>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 7: launch_gemm_t<FMT, GemmH>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 8: launch_gemm_t<FMT, GemmI>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 9: launch_gemm_t<FMT, GemmJ>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 10: launch_gemm_t<FMT, GemmK>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        case 11: launch_gemm_t<FMT, GemmL>(W, Wh, s, Xg, Y, S, I, O, st); break;
-        default: launch_gemm_t<FMT, GemmM>(W, Wh, s, Xg, Y, S, I, O, st); break;
+    const void* Xg = X;
+    if (GEMM_COST[p.tile].xh) {
+        hipLaunchKernelGGL(round_f16_kernel, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 4096)), dim3(256), 0, st,
+                           reinterpret_cast<const float4*>(X), Xh, n4);
+        MOEX_LAUNCHED();
+        Xg = Xh;
+    }
+    float* const out = Y;
+    if (p.nks > 1) Y = part;
+    switch (p.tile) {
+        case 0: launch_gemm_t<FMT, GemmA>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 1: launch_gemm_t<FMT, GemmB>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 2: launch_gemm_t<FMT, GemmC>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 3: launch_gemm_t<FMT, GemmD>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 4: launch_gemm_t<FMT, GemmE>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 5: launch_gemm_t<FMT, GemmF>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 6: launch_gemm_t<FMT, GemmG>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 7: launch_gemm_t<FMT, GemmH>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 8: launch_gemm_t<FMT, GemmI>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 9: launch_gemm_t<FMT, GemmJ>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 10: launch_gemm_t<FMT, GemmK>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 11: launch_gemm_t<FMT, GemmL>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        default: launch_gemm_t<FMT, GemmM>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+    }
+    if (p.nks > 1) {
+        const size_t n = (size_t)S * O;
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 2048)), dim3(256), 0, st, part,
+                           FMT == MF_I8 ? s : nullptr, out, n, O, p.nks);
+        MOEX_LAUNCHED();
     }
 }
 

@@ -958,7 +958,7 @@ struct WsKey {
     int dev;
     hipStream_t st;
     int kind;  // 0: FA tile images, 1: FA partials of split token tiles, 2: fp16 GEMM activations,
-               // 4: decode-kernel partials of short FA chunks, 5: FA pair arrival
+               // 3: partial sums of a K-split GEMM, 4: decode-kernel partials of short FA chunks, 5: FA pair arrival
                // counters (zeroed when allocated)
     bool operator<(const WsKey& o) const {
         return dev != o.dev ? dev < o.dev : st != o.st ? st < o.st : kind < o.kind;

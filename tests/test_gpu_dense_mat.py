@@ -295,3 +295,70 @@ def test_two_rows_equal_gemv(shape, fmt):
         M.gemv(m, xd[t], Yr[t], I, O)
     torch.cuda.synchronize()
     assert torch.equal(Y, Yr)
+
+
+@pytest.mark.parametrize("fmt", ["i8", "q4", "q6", "f16"])
+@pytest.mark.parametrize("O,I,S,shift", [
+    (64, 40448, 9, 0),       # 9 parts of 16 x 16 tiles
+    (130, 16448, 40, 1),     # a ragged last K step in the last part, 4-byte stores
+    (2047, 16384, 300, 0),   # 128 x 64 tiles
+    (2048, 12352, 1100, 0),  # 128-row tiles
+    (96, 8192, 33, 0),       # two parts, the shortest K that is split
+])
+def test_gemm_k_split(fmt, O, I, S, shift):
+    """K split over workgroups (few tiles, a long K), the parts summed by a second kernel: against the precision model, whose
+    exact sums the fp32 ones of up to 40448 products of random sign miss by ~2e-6 of the largest output; the same bits on
+    every call; nothing outside [S][O] written."""
+    import torch
+    import moex_amd as M
+    rng = np.random.default_rng(O + I + S)
+    w = (rng.standard_normal((O, I)) * 0.02).astype(np.float16)
+    if fmt == "i8":
+        q = torch.empty((O, I), dtype=torch.int8, device="cuda")
+        s = torch.empty(O, dtype=torch.float32, device="cuda")
+        M.quantize_rows_i8(dev(w.view(np.int16)), q, s, O, I)
+        torch.cuda.synchronize()
+        m, hq, hs, _keep = M.Mat(q=q, s=s), q.cpu().numpy(), s.cpu().numpy(), (q, s)
+    else:
+        m, (hw, hh, hs), F, _keep = _make(fmt, w)
+    x = rng.standard_normal((S, I)).astype(np.float32)
+    xd = dev(x)
+    got = []
+    for _ in range(2):
+        buf = torch.full((shift + S * O + 64,), float("nan"), dtype=torch.float32, device="cuda")
+        M.gemm(m, xd, buf[shift:shift + S * O], S, I, O)
+        torch.cuda.synchronize()
+        assert torch.isnan(buf[shift + S * O:]).all() and torch.isnan(buf[:shift]).all()
+        got.append(buf[shift:shift + S * O].cpu().numpy().reshape(S, O))
+    rows = sorted({0, 15, S // 2, S - 1} & set(range(S)))
+    cols = np.unique(np.r_[0:O:max(1, O // 32), max(0, O - 4):O])
+    if fmt == "i8":
+        model = orc.dense_i8_fp16x(hq[cols], hs[cols], x[rows])
+    else:
+        model = orc.dense_mat_fp16x(F, hw[cols], None if hh is None else hh[cols], None if hs is None else hs[cols], x[rows])
+    rel = _rel(got[0][np.ix_(rows, cols)].astype(np.float64), model)
+    report("gemm k split", fmt=fmt, O=O, I=I, S=S, rel=rel)
+    assert np.all(np.isfinite(got[0])) and np.array_equal(got[0], got[1]) and rel < 1e-5
+
+
+@pytest.mark.parametrize("fmt,O,I,S,than", [("i8", 64, 40448, 9, (64, 4096, 9)), ("q6", 64, 40448, 40, (64, 4096, 40)),
+                                            ("f16", 2048, 16384, 300, (2048, 4096, 300))])
+def test_gemm_long_k_time(fmt, O, I, S, than):
+    """A long K costs a matrix of few tiles a second launch and its share of the chip, not a K step after the other (measured
+    1.6 to 2.6 times the product of 4096 inputs, 3.2 to 8.4 times with all of K in one workgroup), so at most 2.9 times."""
+    import torch
+    import moex_amd as M
+    from tests.test_gpu_dense import _graph_us
+    us = []
+    for o, i, n in ((O, I, S), than):
+        w = np.random.default_rng(o + i).standard_normal((o, i), dtype=np.float32).astype(np.float16)
+        if fmt == "i8":
+            q, s = torch.empty((o, i), dtype=torch.int8, device="cuda"), torch.empty(o, device="cuda")
+            M.quantize_rows_i8(dev(w.view(np.int16)), q, s, o, i)
+            m = M.Mat(q=q, s=s)
+        else:
+            m, _, _, _keep = _make(fmt, w)
+        x, Y = torch.randn((n, i), device="cuda"), torch.empty((n, o), device="cuda")
+        us.append(_graph_us(lambda st: M.gemm(m, x, Y, n, i, o, st)))
+    print(f"gemm {fmt} {S} tokens: {O}x{I} {us[0]:.2f} us, {than} {us[1]:.2f} us", flush=True)
+    assert us[0] <= 2.9 * us[1]

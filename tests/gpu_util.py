@@ -95,3 +95,12 @@ def append_threaded(cache, k, v, ld, T, pos0, chunk=8192):
     jobs = [(t, min(chunk, T - t)) for t in range(0, T, chunk)]
     with ThreadPoolExecutor(_threads()) as ex:
         list(ex.map(lambda j: orc.kv_append(cache, k[j[0]:j[0] + j[1]], v[j[0]:j[0] + j[1]], ld, j[1], pos0 + j[0]), jobs))
+
+
+def new_stream():
+    """A HIP stream that nothing has used before (torch.cuda.Stream hands out the streams of a pool in turn), default priority"""
+    import ctypes
+    import moex_amd as M
+    st = ctypes.c_void_p()
+    assert M.lib().hipStreamCreate(ctypes.byref(st)) == 0  # the runtime that the library is linked to
+    return torch_dev().cuda.ExternalStream(st.value)

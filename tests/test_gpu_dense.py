@@ -210,10 +210,14 @@ def test_gemv_rows_split(O, I, shift):
     assert _rel(one.cpu().numpy().astype(np.float64), orc.dense_i8_f64(q.cpu().numpy(), s.cpu().numpy(), x)) < 1e-5
 
 
+_timing_stream = None  # one for all of them: torch's pool has 32, which the tests of fresh streams need
+
+
 def _graph_us(call, replays=5, n=40):
     """Time of one call in us, graph-replayed, the best of several replays of n calls"""
     import torch
-    st = torch.cuda.Stream()
+    global _timing_stream
+    st = _timing_stream = _timing_stream or torch.cuda.Stream()
     call(st)
     st.synchronize()
     graph = torch.cuda.CUDAGraph()

@@ -115,7 +115,7 @@ def test_fa_images_and_dense_graph_replays():
                           torch.empty((64, O), device="cuda"))
     torch.cuda.synchronize()
     with torch.cuda.stream(st):
-        run(out_e, y2_e, y64_e)  # eager: allocates the stream's workspace, sets the kernels' attributes
+        run(out_e, y2_e, y64_e)  # eager: allocates attn_fa's workspaces, sets the kernels' attributes
     st.synchronize()
     out_g, y2_g, y64_g = torch.zeros_like(out_e), torch.zeros_like(y2_e), torch.zeros_like(y64_e)
     graph = torch.cuda.CUDAGraph()
@@ -132,9 +132,9 @@ def test_fa_images_and_dense_graph_replays():
 
 
 def test_dense_forms_graph_replays():
-    """The int4 / int6 / fp16 matrix forms captured on a stream after one eager call (which allocates the GEMM's
-    workspaces): int4 GEMV, int6 four-row GEMV pass, fp16 GEMM and int4 GEMM, every replay bit-identical
-    to the eager outputs, with eager work in between."""
+    """The int4 / int6 / fp16 matrix forms captured on a stream after one eager call (these sizes take no workspace): int4
+    GEMV, int6 four-row GEMV pass, fp16 GEMM and int4 GEMM, every replay bit-identical to the eager outputs, with eager
+    work in between."""
     import torch
     import moex_amd as M
     rng = np.random.default_rng(19)
@@ -176,6 +176,93 @@ def test_dense_forms_graph_replays():
         assert all(torch.equal(a, b) for a, b in zip(yg, ye)), i
         x.mul_(1.0)
         torch.cuda.synchronize()
+
+
+# products that take the GEMM's workspaces: fp16 activations (128 x 128 and 288 x 256 tiles), partial sums of a split K, both
+GEMM_WS = [("f16", 4608, 2048, 700), ("i8", 9216, 2048, 1500), ("i8", 130, 16384, 40), ("f16", 2048, 12288, 1100)]
+
+
+def _gemm_ws_case(M, torch, fmt, O, I, S):
+    """(Mat, x, the product of x rounded to fp16 in 64 bits, tensors to keep)"""
+    g = torch.Generator(device="cuda").manual_seed(O + I + S)
+    x = torch.randn((S, I), generator=g, device="cuda")
+    if fmt == "f16":
+        w = (torch.randn((O, I), generator=g, device="cuda") * 0.02).half()
+        m, keep, wd = M.Mat(f16=w), w, w.double()
+    else:
+        q = torch.randint(-127, 128, (O, I), generator=g, device="cuda", dtype=torch.int8)
+        s = torch.rand(O, generator=g, device="cuda") * 0.01 + 1e-3
+        m, keep, wd = M.Mat(q=q, s=s), (q, s), q.double() * s.double()[:, None]
+    return m, x, x.half().double() @ wd.t().contiguous(), keep
+
+
+@pytest.mark.parametrize("fmt,O,I,S", GEMM_WS)
+def test_gemm_workspaces_graph_replays(fmt, O, I, S):
+    """A GEMM that takes a workspace, captured after an eager call on the stream: every replay has the eager call's bits, also
+    after eager calls that use the same workspaces, and then one that outgrows them."""
+    import torch
+    import moex_amd as M
+    from tests.gpu_util import new_stream
+    m, x, ref, _keep = _gemm_ws_case(M, torch, fmt, O, I, S)
+    st = new_stream()
+    eager, out = torch.empty((S, O), device="cuda"), torch.empty((S, O), device="cuda")
+    big = torch.randn((S + S // 2, I), device="cuda")
+    other = torch.empty((S + S // 2, O), device="cuda")
+    torch.cuda.synchronize()
+    held = M.lib().moex_workspace_held()
+    M.gemm(m, x, eager, S, I, O, st)
+    st.synchronize()
+    assert M.lib().moex_workspace_held() > held, "this product was to take a workspace"
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        M.gemm(m, x, out, S, I, O, st)
+    torch.cuda.synchronize()
+    assert float((eager.double() - ref).norm() / ref.norm()) < 1e-5
+    for n in (S, S, S + S // 2):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), n
+        M.gemm(m, big, other, n, I, O, st)
+        torch.cuda.synchronize()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("fmt,O,I,S", GEMM_WS)
+def test_gemm_captured_first(fmt, O, I, S):
+    """A GEMM that would take a workspace, captured as the first call on a fresh stream with no soft-error slot: it allocates
+    nothing, reports nothing and runs a tile that needs none. Every replay (new activations in between) is within 1e-5 of
+    the exact product of the rounded activations, as is the eager call that makes the workspace later, whose sums are in
+    another order; the graph keeps its own bits after it."""
+    import torch
+    import moex_amd as M
+    from tests.gpu_util import new_stream
+    m, x, ref, _keep = _gemm_ws_case(M, torch, fmt, O, I, S)
+    out, eager = torch.empty((S, O), device="cuda"), torch.empty((S, O), device="cuda")
+    M.gemm(m, x, out, S, I, O)  # elsewhere: the kernels' attributes
+    torch.cuda.synchronize()
+    held = M.lib().moex_workspace_held()
+    st = new_stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        M.gemm(m, x, out, S, I, O, st)
+    torch.cuda.synchronize()
+    assert M.lib().moex_workspace_held() == held
+    first = None
+    for i in range(4):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((out.double() - ref).norm() / ref.norm()) < 1e-5, i
+        first = out.clone() if first is None else first
+        assert torch.equal(out, first), i
+        if i == 1:
+            M.gemm(m, x, eager, S, I, O, st)
+            st.synchronize()
+            assert M.lib().moex_workspace_held() > held
+            assert float((eager.double() - ref).norm() / ref.norm()) < 1e-5
 
 
 @pytest.mark.parametrize("gqa_maxt", ["0", "64"])

@@ -1063,7 +1063,13 @@ FaPlan fa_plan(int H, int KV, int max_t, int T, bool turbo) {
     // against 77 us, at 5000 193 against 215: with every CU busy the clock drops, so shortening some blocks only is lost).
     int nsf = 2 * KV * NT > ncu ? 1 : std::min(FA_NSF_MAX, (2 * ncu + KV * NT - 1) / (KV * NT));
     if (const char* e = std::getenv("MOEX_FA_SPLIT")) nsf = std::max(1, std::min(nsf, std::atoi(e)));
-    if (p.ntmax <= FA_MINW) nsf = 1;  // no token tile can have a second piece
+    // A cache so small that pieces never pay, wherever the chunk lies in it, keeps the pairs: no position where the device would
+    // split (fa_piece_w's last condition), or only some token tiles get a second piece there, the others staying as long as
+    // the whole of them (65 tokens at 200 of 320 positions 30.9 -> 28.9 us, 150 at 200 of 384 34.6 -> 31.0, 213 at 200 of 448
+    // 37.5 -> 33.0, 300 at 200 of 512 39.2 -> 36.7; from 576 positions on, pieces win near the cache's end: 300 at 276 36.1
+    // against 39.1)
+    const int nlight = (std::max(0, max_t - T) + FT + BK - 1) / BK;  // key tiles of the first token tile, at most
+    if (4 * FA_MINW > 3 * p.ntmax || (p.ntmax <= 2 * FA_MINW && nlight <= FA_MINW)) nsf = 1;
     p.nsf = nsf;
     p.part_bytes = nsf > 1 ? (size_t)T * H * nsf * FP_ROW * sizeof(float) : 0;
     // pairs: MOEX_FA_PAIR=0 turns them off (read on every call)

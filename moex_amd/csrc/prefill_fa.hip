@@ -1117,7 +1117,6 @@ void launch_fa_bufs(const float* qo, const float* q_gate, moex_kv_cache kv, floa
                            nq, fr ? *fr : FrontArgs{});
         MOEX_LAUNCHED();
     }
-    // a split launch has KV x tiles x nsf blocks: the pieces of every tile, the rest exit at once
     const int mode = nsf > 1 ? FA_MODE_SPLIT : pair ? FA_MODE_PAIR : FA_MODE_ONE;
     int pmin = FA_PAIR_MIN;  // MOEX_FA_PAIR_MIN=n: split a pair's heavy tile only when its second half has n tiles
     if (const char* e = std::getenv("MOEX_FA_PAIR_MIN")) pmin = std::max(1, std::min(255, std::atoi(e)));
@@ -1126,7 +1125,10 @@ void launch_fa_bufs(const float* qo, const float* q_gate, moex_kv_cache kv, floa
     int pextra = FA_PAIR_EXTRA;
     if (const char* e = std::getenv("MOEX_FA_PAIR_EXTRA")) pextra = std::max(0, std::min(255, std::atoi(e)));
     const int pk = pmin | (pextra << 8);
-    const dim3 grid(mode == FA_MODE_SPLIT ? KV * p.NT * nsf : mode == FA_MODE_PAIR ? fa_pair_grid(KV, T) : fa_grid(KV, T));
+    // a split launch: fa_piece_w never lists more pieces than CUs (its KV * n <= ncu, or one a token tile). A surplus block
+    // takes a whole CU's LDS before it finds nothing to do
+    const int nsplit = std::min(KV * p.NT * nsf, std::max(ncu, KV * p.NT));
+    const dim3 grid(mode == FA_MODE_SPLIT ? nsplit : mode == FA_MODE_PAIR ? fa_pair_grid(KV, T) : fa_grid(KV, T));
     const size_t lds = (img ? 4 : 2) * TILE_BYTES;
 #define FA_LAUNCH(IMG_, MODE_)                                                                                         \
     do {                                                                                                               \

@@ -249,7 +249,16 @@ __device__ __forceinline__ bool map_block(int b, int KV, int NT, int& kvh, int& 
 // of the token tile (each row sees a key in every piece). With w at least 2 x token tiles and n / w rounded down, as it
 // was, chunks of several hundred tokens left most of the chip idle: whole attn_decode calls, us, 400 tokens at position
 // 1500 76.6 -> 45.9, 600 at 3000 116 -> 70, 900 at 6000 195 -> 139, 1000 at 2000 106 -> 87, 512 at 32 000 335 -> 305.
+// Two exceptions. No tile is split where the longest piece would be fewer than FA_SAVE_ALL key tiles shorter than the
+// whole, FA_SAVE_SOME where some tiles keep their keys in one piece: the partial results cost as much (us, split -> not:
+// 125 tokens at 200 34.0 -> 32.2, 300 at 100 38.0 -> 36.9, 180 at 150 36.3 -> 33.5; 400 at 0 38.0 -> 39.0 the other way).
+// And a longer w is taken where it needs fewer CUs for about the same longest piece, weighed by FA_BUSY: the clock drops
+// with the CUs that are busy. A third piece for most tiles, the rest keeping two, had made 700 tokens at 32 768 497 us with
+// 256 workgroups, two each with 176 445; 529 at 32 768 355 -> 337, 768 at 10 000 183 -> 174 (FA_BUSY from six such pairs:
+// 0.2 to 0.7; the worst case of it, 698 at 7000, 137 -> 140).
 constexpr int FA_MINW = 8;
+constexpr int FA_SAVE_ALL = 5, FA_SAVE_SOME = 7;
+constexpr float FA_BUSY = 0.5f;
 constexpr int FA_NSF_MAX = 32;
 constexpr int FP_ROW = AHD + 4;  // a piece's partial row: O[256], m, l, 2 spare (16-byte aligned rows)
 constexpr int FP_W = AHD + 2;    // the spare slot of the first row holds w, for the merge
@@ -274,11 +283,28 @@ __device__ __forceinline__ int fa_piece_w(int pos0, int T, int KV, int NT, int n
         if (!__builtin_amdgcn_ballot_w64(c > 0)) break;
         n += c;
     }
+    // the first token tile, the shortest, has kmin pieces: 1 + floor((n - 1) / wl), half a tile off an exact quotient
+    const int nmax = (pos0 + T + BK - 1) / BK, nmin = (pos0 + min(FT, T) + BK - 1) / BK;
+    const int kmin = min(nsf, 1 + (int)(((float)nmin - 0.5f) * __builtin_amdgcn_rcpf((float)wl)));
     const unsigned long long fit = __builtin_amdgcn_ballot_w64(KV * n <= ncu);
-    const int nmax = (pos0 + T + BK - 1) / BK, l = fit ? __builtin_ctzll(fit) : 63;
-    if (!fit || 4 * (w0 + w0 * l / 16) > 3 * nmax) {  // the longest would hardly get shorter: no tile is split
-        n1 = NT;
+    int l = fit ? __builtin_ctzll(fit) : 63;
+    // the longest piece: nmax / kmin where every token tile has kmin pieces, about wl where some have one more
+    const float len = (float)nmax * __builtin_amdgcn_rcpf((float)(kmin * wl >= nmax ? kmin : nsf));
+    const float longest = kmin * wl >= nmax ? len : fmaxf((float)wl, len);
+    const bool one = kmin == 1;
+    const unsigned long long pays =
+        __builtin_amdgcn_ballot_w64((float)nmax - longest >= (one ? (float)FA_SAVE_SOME : (float)FA_SAVE_ALL));
+    if (!fit || 4 * (w0 + w0 * l / 16) > 3 * nmax || !(pays >> l & 1)) {  // the longest would hardly get shorter
+        n1 = NT;  // no token tile is split
         return nmax;
+    }
+    // Not the shortest longest piece, if it takes many more CUs for little: the clock drops with the CUs that are busy
+    const float cost = longest * ((float)ncu + FA_BUSY * (float)(KV * n));
+    for (;;) {
+        const float c = 0.99f * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(cost), l));
+        const unsigned long long better = fit & __builtin_amdgcn_ballot_w64(cost < c);
+        if (!better) break;
+        l = __builtin_ctzll(better);
     }
     n1 = __builtin_amdgcn_readlane(n, l);
     return w0 + w0 * l / 16;

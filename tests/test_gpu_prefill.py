@@ -186,22 +186,50 @@ def test_prefill_fallback_other_groups(Hq, KVq, pos0, T):
     assert np.all(np.isfinite(o)) and e_new <= 2.0 * e_ref + 1e-3 * mag
 
 
+def _pieces(pos0, T, cus):
+    """The kernel's rule in plain Python: pieces of each token tile's keys, or None where the plan takes pairs or tiles"""
+    NT = -(-T // 16)
+    if 2 * KV * NT > cus:
+        return None
+    nsf = min(32, (2 * cus + KV * NT - 1) // (KV * NT))
+    n = [-(-(pos0 + min(16 * (t + 1), T)) // 32) for t in range(NT)]  # key tiles of every token tile
+    w0 = max(8, -(-KV * ((NT * ((2 * pos0 + T + 16) // 2) + NT * 31) // 32) // cus))
+    fit = []
+    for w in (w0 + w0 * i // 16 for i in range(64)):
+        k = [min(nsf, -(-x // w)) for x in n]
+        if KV * sum(k) <= cus:
+            fit.append((w, k, n[-1] / k[0] if k[0] * w >= n[-1] else max(w, n[-1] / nsf)))
+    if not fit or 4 * fit[0][0] > 3 * n[-1] or n[-1] - fit[0][2] < (7 if fit[0][1][0] == 1 else 5):
+        return [1] * NT
+    cost = [length * (cus + 0.5 * KV * sum(k)) for _, k, length in fit]
+    best = 0
+    while True:
+        better = [i for i in range(len(fit)) if cost[i] < 0.99 * cost[best]]
+        if not better:
+            return fit[best][1]
+        best = better[0]
+
+
 @pytest.mark.parametrize("pos0,T,cus", [
     (0, 65, 256), (300, 129, 256), (1500, 400, 256), (6000, 1024, 256),  # half a full grid: the last size that splits
     (6000, 1025, 256),                                                   # the first that runs in pairs
     (20000, 213, 104), (3000, 600, 304), (33000, 1000, 8),               # other chip sizes; one too small to split on
+    (100, 300, 256), (150, 400, 256), (200, 213, 256),                   # pieces of the heavier tiles only: worth it in one
+    (32768, 700, 256), (7000, 768, 256), (32768, 529, 256),              # fewer pieces than CUs, as long within a few percent
 ])
 def test_fa_piece_lengths(setup, pos0, T, cus, monkeypatch):
     """The key pieces' length is searched on the device so that all pieces fit the chip once (planned here as for a chip
-    of `cus` CUs): every row written, and equal to the unsplit kernel up to the fp32 merge and the lazily rescaled
-    softmax's reference per piece (2e-3 of the largest output, as test_fa_key_split)."""
+    of `cus` CUs): every row written, the test_fa.cu gate, and equal to the kernel without pieces or pairs up to the fp32
+    merge and the lazily rescaled softmax's reference per piece (2e-3 of the largest output, as test_fa_key_split). A token
+    tile of one piece has that kernel's bits, one of several has not: the pieces are where the rule puts them."""
     import torch
     import moex_amd as M
-    _, dc, _, _, qo_d, qg_d = setup
+    hc, dc, qo, qg, qo_d, qg_d = setup
     monkeypatch.setenv("MOEX_FA_CUS", str(cus))
     outs = []
     for cap in ("32", "1"):
         monkeypatch.setenv("MOEX_FA_SPLIT", cap)
+        monkeypatch.setenv("MOEX_FA_PAIR", cap if cap == "32" else "0")
         out = torch.full((T, H, AHD), float("nan"), dtype=torch.float32, device="cuda")
         M.attn_fa(qo_d, qg_d, dc, out, H, KV, pos_tensor(pos0), dc.max_t, LD, T)
         torch.cuda.synchronize()
@@ -210,3 +238,31 @@ def test_fa_piece_lengths(setup, pos0, T, cus, monkeypatch):
     d, mag = float((outs[0] - outs[1]).abs().max()), float(outs[1].abs().max())
     report("fa piece lengths", pos0=pos0, T=T, cus=cus, maxdiff=d, mag=mag)
     assert d <= 2e-3 * mag
+    _gate("fa piece lengths", outs[0].cpu().numpy(), qo, qg, hc, pos0, T)
+    k = _pieces(pos0, T, cus)
+    same = [torch.equal(outs[0][16 * t:16 * t + 16], outs[1][16 * t:16 * t + 16]) for t in range(-(-T // 16))]
+    if k is not None:
+        assert same == [x == 1 for x in k], (k, same)
+    elif KV * len(same) <= cus:
+        assert not all(same)  # pairs: the heavy tiles in two halves
+    else:
+        assert all(same)  # whole token tiles in both runs
+
+
+@pytest.mark.parametrize("pos0,T", [(32768, 700), (10000, 695)])
+def test_fa_even_pieces(setup, pos0, T, monkeypatch):
+    """Where a third piece for most token tiles would shorten the longest by a few percent and take every CU, all tiles keep
+    two: the same bits as with at most two pieces allowed (three each for most took 497 us here, two 445)."""
+    import torch
+    import moex_amd as M
+    _, dc, _, _, qo_d, qg_d = setup
+    monkeypatch.setenv("MOEX_FA_CUS", "256")
+    outs = []
+    for cap in ("32", "2"):
+        monkeypatch.setenv("MOEX_FA_SPLIT", cap)
+        out = torch.full((T, H, AHD), float("nan"), dtype=torch.float32, device="cuda")
+        M.attn_fa(qo_d, qg_d, dc, out, H, KV, pos_tensor(pos0), dc.max_t, LD, T)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert set(_pieces(pos0, T, 256)) == {2}
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])

@@ -128,10 +128,12 @@ constexpr float WS_SLACK = 8.f;
 // one) in a ring of NS LDS stages, NS - 1 chunks in flight. A stage holds the K rows, the V rows, then ks[CH] and
 // vs[CH]. Producers 0, 1 move the K rows, 2, 3 the V rows (CH / 8 instructions of 4 rows each); with 128-key chunks
 // each producer also moves 64 scales (ks for 0, 1, vs for 2, 3), with 64-key chunks producers 0 and 2 move all 64
-// (4 bytes a lane). Rows past the chunk repeat its last row: their P is 0. Chunk c + NS - 1 is issued at the barrier
-// that hands chunk c to the consumers (its stage held chunk c - 1, now consumed); the producers end each chunk with a
-// bare s_barrier, as __syncthreads would also wait for the chunks still in flight. Takes part in the nch + 2
-// barriers of the chunk loop and the consumer merge.
+// (4 bytes a lane). The K and V codes of a stage past its chunk's end are arbitrary bytes: the rows that follow (another
+// chunk's, unwritten ones or one just being appended) or, near the cache's end, the chunk's last row again. The scales
+// there repeat the chunk's last one, so they are finite, and the consumers mask those scores before the maximum: their
+// P is 0. Chunk c + NS - 1 is issued at the barrier that hands chunk c to the consumers (its stage held chunk c - 1, now
+// consumed); the producers end each chunk with a bare s_barrier, as __syncthreads would also wait for the chunks still
+// in flight. Takes part in the nch + 2 barriers of the chunk loop and the consumer merge.
 // LDS transfers of 16 (4) bytes per active lane, lane l to lds + 16 l (4 l), written in inline asm: the compiler cannot
 // tell which LDS bytes a transfer writes and would make the wavefront's next LDS read wait for every transfer in
 // flight; the kernel waits for its own transfers with vm_wait. dma16s: wave-uniform base + per-lane 32-bit offset.

@@ -421,15 +421,6 @@ __device__ __forceinline__ void norm_rope(float (&x)[4], uint2 wb, int lane, con
     norm_partner(x, px, wb, lane, rot, eps);
     rotate(x, px, rp, lane, rot);
 }
-__device__ __forceinline__ void norm_rope(float (&x)[4], uint2 wb, int lane, int pos, int rot, float theta, float eps) {
-    float px[4];
-    norm_partner(x, px, wb, lane, rot, eps);
-    rotate(x, px, rope_angles(lane, pos, rot, theta), lane, rot);
-}
-__device__ __forceinline__ void norm_rope(float (&x)[4], const uint16_t* w, int lane, int pos, int rot, float theta,
-                                          float eps) {
-    norm_rope(x, *reinterpret_cast<const uint2*>(w + 4 * lane), lane, pos, rot, theta, eps);
-}
 
 // wht of both 128-value halves of the row (dir 0 forward, 1 inverse)
 __device__ __forceinline__ void wht(float (&x)[4], int dir, int lane) {

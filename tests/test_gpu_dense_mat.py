@@ -235,23 +235,34 @@ def test_gemm_tiles(fmt, O, I, S, shift):
     assert torch.isnan(buf[shift + S * O:]).all() and torch.isnan(buf[:shift]).all()
 
 
+@pytest.mark.parametrize("fmt", ["i8", "f16"])
 @pytest.mark.parametrize("I", [32, 96, 2080])
-def test_gemm_odd_inputs(I):
-    """I a multiple of 32 but not of 64 (int8 and fp16 only), below, above and at a K step's remainder."""
+def test_gemm_odd_inputs(I, fmt):
+    """I a multiple of 32 but not of 64 (int8 and fp16 only), below, above and at a K step's remainder; the last rows of
+    tokens and weights among those compared."""
     import torch
     import moex_amd as M
     rng = np.random.default_rng(I)
     for O, S in ((130, 9), (2048, 300), (4608, 1100)):
         w = (rng.standard_normal((O, I)) * 0.02).astype(np.float16)
-        m, (hw, _, _), F, _keep = _make("f16", w)
+        if fmt == "i8":
+            q, s = torch.empty((O, I), dtype=torch.int8, device="cuda"), torch.empty(O, device="cuda")
+            M.quantize_rows_i8(dev(w.view(np.int16)), q, s, O, I)
+            torch.cuda.synchronize()
+            m, hq, hs = M.Mat(q=q, s=s), q.cpu().numpy(), s.cpu().numpy()
+        else:
+            m, (hw, _, _), F, _keep = _make("f16", w)
         x = rng.standard_normal((S, I)).astype(np.float32)
-        Y = torch.full((S, O), float("nan"), dtype=torch.float32, device="cuda")
+        Y = torch.full((S + 1, O), float("nan"), dtype=torch.float32, device="cuda")
         M.gemm(m, dev(x), Y, S, I, O)
         torch.cuda.synchronize()
-        got = Y.cpu().numpy()
-        rows, cols = [0, S // 2, S - 1], np.arange(0, O, max(1, O // 100))
+        assert torch.isnan(Y[S]).all()
+        got = Y[:S].cpu().numpy()
+        rows, cols = [0, S // 2, S - 2, S - 1], np.unique(np.r_[0:O:max(1, O // 100), O - 20:O])
+        model = (orc.dense_i8_fp16x(hq[cols], hs[cols], x[rows]) if fmt == "i8" else
+                 orc.dense_mat_fp16x(F, hw[cols], None, None, x[rows]))
         assert np.all(np.isfinite(got))
-        assert _rel(got[np.ix_(rows, cols)].astype(np.float64), orc.dense_mat_fp16x(F, hw[cols], None, None, x[rows])) < 1e-5
+        assert _rel(got[np.ix_(rows, cols)].astype(np.float64), model) < 1e-5
 
 
 @pytest.mark.parametrize("fmt", ["q4", "q6", "f16"])
@@ -295,6 +306,33 @@ def test_two_rows_equal_gemv(shape, fmt):
         M.gemv(m, xd[t], Yr[t], I, O)
     torch.cuda.synchronize()
     assert torch.equal(Y, Yr)
+
+
+@pytest.mark.parametrize("fmt", ["q4", "q6", "f16"])
+@pytest.mark.parametrize("O,I", [(1999, 2048), (2305, 2048), (3999, 2048), (4501, 2048), (18439, 256), (1023, 4096),
+                                 (1101, 4096), (1601, 4096), (2303, 4096), (700, 8192)])
+def test_gemv_mat_every_row_group(O, I, fmt):
+    """Every number of rows a wavefront takes (2, 3, 4 and 6, chosen by O), at every number of parts a row is split in (1, 2,
+    4, 8) and every number of input rows: a row has the bits of its own call and is within 1e-5 of the exact product (fp32
+    sums of at most 8192 products); nothing is written past the last row."""
+    import torch
+    import moex_amd as M
+    rng = np.random.default_rng(O + I)
+    m, (hw, hh, hs), F, _keep = _make(fmt, (rng.standard_normal((O, I)) * 0.02).astype(np.float16))
+    n = 8 if fmt == "q6" else 2
+    x = rng.standard_normal((n, I)).astype(np.float32)
+    xd = dev(x)
+    one = torch.full((n, O), float("nan"), dtype=torch.float32, device="cuda")
+    for t in range(n):
+        M.gemv(m, xd[t], one[t], I, O)
+    for S in range(2, n + 1):
+        Y = torch.full((S + 1, O), 123.0, device="cuda")
+        M.gemm(m, xd, Y, S, I, O)
+        torch.cuda.synchronize()
+        assert torch.equal(Y[:S], one[:S]), S
+        assert bool((Y[S] == 123.0).all()), S
+    ref = orc.dense_mat_f64(F, hw, hh, hs, x)
+    assert _rel(one.cpu().numpy().astype(np.float64), ref) < 1e-5
 
 
 @pytest.mark.parametrize("fmt", ["i8", "q4", "q6", "f16"])

@@ -1092,7 +1092,10 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
 // token tiles fill the chip where those of 32 and 64 leave a part of it or a round short (int8 / int4, us, with the best
 // of the others against them): qkv at 40 tokens 13.0 / 14.4 -> 12.3 / 12.2, at 100 20.2 / 20.8 -> 17.3 / 20.3; o_proj
 // at 300 21.9 / 25.2 -> 21.3 / 21.2, at 600 33.7 / 37.0 -> 26.8 / 33.9. 112 x 128 was never the best by more than 1 %.
-struct GemmCost { int BM, BN; bool xh; int BK; float us0, us1; bool split; };
+// 128 x 96 runs where it fills the chip in one round only (`one`): o_proj of 1025 to 1536 tokens, which 128 x 128 tiles leave
+// half idle (int8 / fp16, us, with the best of the others against it: 1100 tokens 53 / 49 -> 44 / 45, 1500 49 / 50 ->
+// 46 / 47; 9216 x 3072, 288 tokens, 44 / 41 -> 35 / 37); over several rounds 128 x 128 was up to 15 % faster.
+struct GemmCost { int BM, BN; bool xh; int BK; float us0, us1; bool split, one; };
 using GemmA = GemmTile<9, 4, 2, 4, 1, 2, 1, true>;  // 288 x 256
 using GemmB = GemmTile<9, 2, 1, 8, 1, 2, 1, true>;  // 144 x 256
 using GemmC = GemmTile<9, 2, 1, 4, 2, 1, 2>;        // 144 x 128
@@ -1106,18 +1109,19 @@ using GemmJ = GemmTile<2, 1, 1, 1, 8, 1, 2, false, 4>;       // 32 x 16
 using GemmK = GemmTile<1, 1, 1, 1, 8, 1, 2, false, 4>;       // 16 x 16
 using GemmL = GemmTile<4, 3, 2, 1, 4, 1, 2>;        // 128 x 48
 using GemmM = GemmTile<2, 3, 2, 1, 4, 1, 2>;        // 64 x 48
+using GemmN = GemmTile<4, 3, 2, 2, 2, 2, 2, true>;  // 128 x 96
 // the tiles that are built with a K split too
 template <class C>
 constexpr bool gemm_splits = std::is_same_v<C, GemmE> || std::is_same_v<C, GemmF> || std::is_same_v<C, GemmH> ||
                              std::is_same_v<C, GemmI> || std::is_same_v<C, GemmK> || std::is_same_v<C, GemmG>;
-template <class C> constexpr GemmCost gemm_cost(float us0, float us1) {
-    return {C::BM, C::BN, C::XH, C::BK, us0, us1, gemm_splits<C>};
+template <class C> constexpr GemmCost gemm_cost(float us0, float us1, bool one = false) {
+    return {C::BM, C::BN, C::XH, C::BK, us0, us1, gemm_splits<C>, one};
 }
 constexpr GemmCost GEMM_COST[] = {
     gemm_cost<GemmA>(10.f, 33.f),   gemm_cost<GemmB>(8.f, 20.7f),   gemm_cost<GemmC>(6.f, 16.6f), gemm_cost<GemmD>(6.6f, 11.f),
     gemm_cost<GemmE>(4.f, 8.5f),    gemm_cost<GemmF>(5.6f, 7.37f),  gemm_cost<GemmG>(3.6f, 4.87f), gemm_cost<GemmH>(4.4f, 2.71f),
     gemm_cost<GemmI>(.8f, 2.42f),   gemm_cost<GemmJ>(.4f, 1.94f),   gemm_cost<GemmK>(1.f, 1.44f), gemm_cost<GemmL>(6.f, 5.61f),
-    gemm_cost<GemmM>(2.f, 4.02f)};
+    gemm_cost<GemmM>(2.f, 4.02f),   gemm_cost<GemmN>(7.f, 7.2f, true)};
 
 // nks parts of K (at most: no empty one is left) where the tile has a split instance
 template <int FMT, class C, bool SPLIT>
@@ -1164,6 +1168,7 @@ GemmPick gemm_pick(int S, int I, int O, bool xh, bool split, bool f16) {
         // a tile's offsets stay within 32 bits (the smallest tile's are 64-bit)
         if (t.BM * t.BN > 256 && (size_t)std::max(t.BM, t.BN) * I * 4 >= (size_t)1 << 32) continue;
         const size_t tiles = (size_t)((O + t.BM - 1) / t.BM) * ((S + t.BN - 1) / t.BN);
+        if (t.one && tiles > (size_t)cus) continue;
         for (int nks = 1; nks == 1 || (split && t.split && nks <= I / 4096 && tiles * nks <= (size_t)2 * cus); nks++) {
             float e = (float)((tiles * nks + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f) / (float)nks) *
                           (f16 && !t.xh ? 1.15f : 1.f) + (t.xh ? 8.f + 1e-6f * (float)S * (float)I : 0.f);
@@ -1214,7 +1219,8 @@ void launch_gemm(const void* W, const uint8_t* Wh, const float* s, const float* 
         case 9: launch_gemm_t<FMT, GemmJ>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
         case 10: launch_gemm_t<FMT, GemmK>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
         case 11: launch_gemm_t<FMT, GemmL>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
-        default: launch_gemm_t<FMT, GemmM>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        case 12: launch_gemm_t<FMT, GemmM>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
+        default: launch_gemm_t<FMT, GemmN>(W, Wh, s, Xg, Y, S, I, O, st, p.nks); break;
     }
     if (p.nks > 1) {
         const size_t n = (size_t)S * O;

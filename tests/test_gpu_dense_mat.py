@@ -189,6 +189,9 @@ def test_int8_mat_routes_to_gemm_i8():
     (9215, 2048, 397, 0),    # 144 x 128
     (9217, 512, 509, 0),     # 128 x 128, few K steps (fp16: with fp16 activations)
     (2049, 4096, 1531, 1),   # 128 x 128, output 4 bytes off a 16-byte boundary
+    (2047, 4096, 1531, 0),   # 128 x 96, one tile a CU, ragged in both directions
+    (2048, 4096, 1025, 1),   # 128 x 96, one token past a tile, output 4 bytes off a 16-byte boundary
+    (5500, 3072, 385, 0),    # 128 x 96
     (9215, 2048, 770, 0),    # 128 x 128, fp16 activations
     (2048, 1088, 800, 0),    # 128 x 64; I % 128 != 0
     (2047, 4096, 611, 0),    # 128 x 48
@@ -377,6 +380,22 @@ def test_gemm_k_split(fmt, O, I, S, shift):
     rel = _rel(got[0][np.ix_(rows, cols)].astype(np.float64), model)
     report("gemm k split", fmt=fmt, O=O, I=I, S=S, rel=rel)
     assert np.all(np.isfinite(got[0])) and np.array_equal(got[0], got[1]) and rel < 1e-5
+
+
+def test_gemm_half_full_grid_time():
+    """o_proj of 1100 tokens takes no longer than of 1536, a full round of the same tile (measured 0.96 of it; with 128 x 128
+    tiles on half of the chip 1.05 to 1.10)."""
+    import torch
+    import moex_amd as M
+    from tests.test_gpu_dense import _graph_us
+    O, I = 2048, 4096
+    q = torch.randint(-127, 128, (O, I), dtype=torch.int8, device="cuda")
+    m, us = M.Mat(q=q, s=torch.rand(O, device="cuda")), []
+    for S in (1100, 1536):
+        x, y = torch.randn((S, I), device="cuda"), torch.empty((S, O), device="cuda")
+        us.append(_graph_us(lambda st: M.gemm(m, x, y, S, I, O, st), n=20))
+    print(f"o_proj 1100 tokens {us[0]:.2f} us, 1536 {us[1]:.2f} us", flush=True)
+    assert us[0] <= 1.02 * us[1]
 
 
 @pytest.mark.parametrize("fmt,O,I,S,than", [("i8", 64, 40448, 9, (64, 4096, 9)), ("q6", 64, 40448, 40, (64, 4096, 40)),

@@ -394,12 +394,12 @@ __device__ __forceinline__ void wstage_widen(const WStage& w, bool ok, uint32_t 
 // outputs are what 256 VGPRs and 160 KB of LDS hold, and at 2048 tokens the qkv matrix is 256 such tiles, one a CU.
 // The small tiles: the latency of a K step's loads; a tile that one CU runs alone has all of its K parts inside one
 // workgroup, so no partial sum goes through memory and no second launch adds them.
-// Measured (graph-replayed calls over rotating weights, us; before: 128 x 128 tiles on 4 wavefronts or 4 + 4 split
-// roles, an fp16 rounding launch for every call, K split over workgroups with a reduction launch), int8:
+// Measured (graph-replayed calls over 300 MB of rotating weights, us; before: 128 x 128 tiles on 4 wavefronts or 4 + 4
+// split roles, an fp16 rounding launch for every call, K split over workgroups with a reduction launch), int8:
 //   tokens              9          64         300        512        1024       2048
-//   qkv  9216 x 2048    19.2->9.0  31.0->13.6 46.7->29.1 48.4->42.7 74.8->58.0 142.9->92.0 (842 TFLOPS)
-//   o    2048 x 4096    17.2->8.5  24.1->10.5 33.8->21.3 38.8->22.7 52.9->34.5  74.3->52.3 (657 TFLOPS)
-// int4 at 300 tokens: qkv 45.9 -> 31.1, o 31.7 -> 21.2; fp16 at 2048: 142.0 -> 88.1, 82.3 -> 59.9.
+//   qkv  9216 x 2048    21.0->10.4 32.7->17.1 47.1->31.2 50.3->43.6 73.8->57.9 139->90.2 (857 TFLOPS)
+//   o    2048 x 4096    17.9->10.1 24.9->12.1 34.4->23.8 39.0->26.8 53.3->38.2 79.6->53.8 (638 TFLOPS)
+// int4 at 300 tokens: qkv 45.3 -> 32.3, o 31.8 -> 23.6; fp16 at 2048: 136 -> 84.4, 81.6 -> 59.2.
 template <int WM_, int WN_, int GM_, int GN_, int KW_, int BKU_, int PD_, bool XH_ = false, int WPE_ = 2>
 struct GemmTile {
     static constexpr int WM = WM_, WN = WN_, GM = GM_, GN = GN_, KW = KW_, BKU = BKU_, PD = PD_;

@@ -420,18 +420,38 @@ template <int N> __device__ __forceinline__ void gemm_vm_wait() { asm volatile("
 // The XH wait counts on a K step's weight loads being issued between its transfers and the wait: W, Wh and s are no
 // __restrict__ pointers there (see gemv1_kernel), and every load has a use, the last ones after the loop. The other tiles
 // wait for nothing by count and leave the order to the compiler.
+// Four outputs (row scales) of a lane from p on, n of them inside the row: 16-byte accesses at any 4-byte alignment, which the
+// hardware takes as they are. With 4-byte stores wherever O or Y was not a multiple of 16 bytes, a line was written in four
+// passes, and four scale loads a lane cost an int8 tile with a short K as much as its outputs (us, 4-byte accesses -> so:
+// 11925 x 320, 1625 tokens int8 59.0 -> 42.7, fp16 65.2 -> 40.0; 11971 x 1088, 389 tokens fp16 37.9 -> 29.9; 6722 x 128, 1005
+// tokens int8 26.1 -> 16.5)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f32x4u load4(const float* p, int n) {
+    if (n >= 4) return *reinterpret_cast<const f32x4u*>(p);
+    f32x4u v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 3; e++)
+        if (e < n) v[e] = p[e];
+    return v;
+}
+__device__ __forceinline__ void store4(float* p, float4_t v, int n) {
+    if (n >= 4) {
+        *reinterpret_cast<f32x4u*>(p) = v;
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 3; e++)
+        if (e < n) p[e] = v[e];
+}
 template <class C, class T>
 using weight_ptr = std::conditional_t<C::XH, const T*, const T* __restrict__>;
 // SPLIT: workgroup (x, y) takes spp K steps of tile x from spp y on and writes their sums, without the row scales, to the
-// y-th [S][O] of Y. An instance of its own, as the parts' bounds would cost every call 0.2 to 0.4 us. vec_spp: bit 0 says that
-// outputs can be stored 16 bytes at a time, the others are spp; in one word, since with two the grid's size lay past the
-// first 64 bytes of the arguments, another 0.2 us.
+// y-th [S][O] of Y. An instance of its own, as the parts' bounds would cost every call 0.2 to 0.4 us.
 template <int FMT, class C, bool SPLIT>
 __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, void> W, weight_ptr<C, uint8_t> Wh,
                                                            weight_ptr<C, float> s, const void* __restrict__ Xv,
-                                                           float* __restrict__ Y, int S, int I, int O, int vec_spp) {
+                                                           float* __restrict__ Y, int S, int I, int O, int spp) {
     extern __shared__ __align__(16) _Float16 gl[];
-    const int vec = vec_spp & 1, spp = vec_spp >> 1;
     const int tid = threadIdx.x, lane = tid & 63, m16 = lane & 15, g = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nO = (O + C::BM - 1) / C::BM, nt = gridDim.x;
@@ -611,24 +631,13 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
         for (int i = 0; i < C::WM; i++) {
             const int o = o0 + wr + 16 * i + 4 * g;
             if (o >= O) continue;
-            float sc[4] = {1.f, 1.f, 1.f, 1.f};
-            if constexpr (FMT == MF_I8 && !SPLIT) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) sc[e] = s[min(o + e, O - 1)];
-            }
+            f32x4u sc = {1.f, 1.f, 1.f, 1.f};
+            if constexpr (FMT == MF_I8 && !SPLIT) sc = load4(s + o, O - o);
 #pragma unroll
             for (int j = 0; j < C::WN; j++) {
                 const int t = s0 + wt + 16 * j + m16;
                 if (t >= S) continue;
-                float* y = Y + (size_t)t * O + o;
-                const float4_t v = acc[i][j];
-                if (vec) {
-                    *reinterpret_cast<float4*>(y) = make_float4(v[0] * sc[0], v[1] * sc[1], v[2] * sc[2], v[3] * sc[3]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (o + e < O) y[e] = v[e] * sc[e];
-                }
+                store4(Y + (size_t)t * O + o, acc[i][j] * sc, O - o);
             }
         }
     } else {
@@ -652,18 +661,9 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
                 const float4 b = *reinterpret_cast<const float4*>(red + ((size_t)p * C::BN + tl) * RL + rl);
                 a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
             }
-            float v[4] = {a.x, a.y, a.z, a.w};
-            if constexpr (FMT == MF_I8 && !SPLIT) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[i] *= s[min(o + i, O - 1)];
-            }
-            float* y = Y + (size_t)t * O + o;
-            if (vec) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
-            else {
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (o + i < O) y[i] = v[i];
-            }
+            f32x4u v = {a.x, a.y, a.z, a.w};
+            if constexpr (FMT == MF_I8 && !SPLIT) v *= load4(s + o, O - o);
+            store4(Y + (size_t)t * O + o, v, O - o);
         }
     }
 }
@@ -1088,7 +1088,7 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
 // o_proj at 1300 tokens 58 us with 128 x 128 against 48 with 128 x 128 XH, int8 49 against 54). The XH tiles' rounding
 // launch costs 8 us + 1 us per million activations, so they pay where a call runs several rounds or the tile is large
 // (o_proj at 3000 tokens, int8: 95 -> 80). The tile with the smallest
-// estimate runs: at 12 token counts from 12 to 900 on both shapes and forms it was the fastest or within 5 %. The 48
+// estimate runs: at 12 token counts from 12 to 900 on both shapes and forms it was the fastest or within 5 %.
 // token tiles fill the chip where those of 32 and 64 leave a part of it or a round short (int8 / int4, us, with the best
 // of the others against them): qkv at 40 tokens 13.0 / 14.4 -> 12.3 / 12.2, at 100 20.2 / 20.8 -> 17.3 / 20.3; o_proj
 // at 300 21.9 / 25.2 -> 21.3 / 21.2, at 600 33.7 / 37.0 -> 26.8 / 33.9. 112 x 128 was never the best by more than 1 %.
@@ -1134,10 +1134,9 @@ int launch_gemm_s(const void* W, const uint8_t* Wh, const float* s, const void* 
     }();
     (void)once;
     const int tiles = ((O + C::BM - 1) / C::BM) * ((S + C::BN - 1) / C::BN);
-    const int vec = O % 4 == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;  // 16-byte output stores
     const int ns = (I + C::BK - 1) / C::BK, spp = (ns + nks - 1) / nks, parts = (ns + spp - 1) / spp;
     hipLaunchKernelGGL((gemm_tile_kernel<FMT, C, SPLIT>), dim3(tiles, parts), dim3(512), C::LDS, st, W, Wh, s, X, Y, S, I, O,
-                       vec + 2 * spp);
+                       spp);
     MOEX_LAUNCHED();
     return parts;
 }

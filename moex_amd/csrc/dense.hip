@@ -1088,7 +1088,8 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
 // o_proj at 1300 tokens 58 us with 128 x 128 against 48 with 128 x 128 XH, int8 49 against 54). The XH tiles' rounding
 // launch costs 8 us + 1 us per million activations, so they pay where a call runs several rounds or the tile is large
 // (o_proj at 3000 tokens, int8: 95 -> 80). The tile with the smallest
-// estimate runs: at 12 token counts from 12 to 900 on both shapes and forms it was the fastest or within 5 %.
+// estimate runs: at 12 token counts from 12 to 900 on both shapes and forms it was the fastest or within 5 %, and 3 % off the
+// fastest in the mean over 100 other matrices of 64 to 2048 inputs, which us0 of 128 x 128 XH, 32 x 32 and 32 x 16 was set by. The 48
 // token tiles fill the chip where those of 32 and 64 leave a part of it or a round short (int8 / int4, us, with the best
 // of the others against them): qkv at 40 tokens 13.0 / 14.4 -> 12.3 / 12.2, at 100 20.2 / 20.8 -> 17.3 / 20.3; o_proj
 // at 300 21.9 / 25.2 -> 21.3 / 21.2, at 600 33.7 / 37.0 -> 26.8 / 33.9. 112 x 128 was never the best by more than 1 %.
@@ -1119,8 +1120,8 @@ template <class C> constexpr GemmCost gemm_cost(float us0, float us1, bool one =
 }
 constexpr GemmCost GEMM_COST[] = {
     gemm_cost<GemmA>(10.f, 33.f),   gemm_cost<GemmB>(8.f, 20.7f),   gemm_cost<GemmC>(6.f, 16.6f), gemm_cost<GemmD>(6.6f, 11.f),
-    gemm_cost<GemmE>(4.f, 8.5f),    gemm_cost<GemmF>(5.6f, 7.37f),  gemm_cost<GemmG>(3.6f, 4.87f), gemm_cost<GemmH>(4.4f, 2.71f),
-    gemm_cost<GemmI>(.8f, 2.42f),   gemm_cost<GemmJ>(.4f, 1.94f),   gemm_cost<GemmK>(1.f, 1.44f), gemm_cost<GemmL>(6.f, 5.61f),
+    gemm_cost<GemmE>(3.f, 8.8f),    gemm_cost<GemmF>(5.6f, 7.37f),  gemm_cost<GemmG>(3.6f, 4.87f), gemm_cost<GemmH>(4.4f, 2.71f),
+    gemm_cost<GemmI>(1.1f, 2.42f),  gemm_cost<GemmJ>(.7f, 1.94f),   gemm_cost<GemmK>(1.f, 1.44f), gemm_cost<GemmL>(6.f, 5.61f),
     gemm_cost<GemmM>(2.f, 4.02f),   gemm_cost<GemmN>(7.f, 7.2f, true)};
 
 // nks parts of K (at most: no empty one is left) where the tile has a split instance

@@ -187,7 +187,7 @@ def test_int8_mat_routes_to_gemm_i8():
     (9211, 2048, 2047, 0),   # 288 x 256 tiles, ragged in both directions, O % 4 != 0 (4-byte stores)
     (9212, 1024, 1021, 0),   # 144 x 256
     (9215, 2048, 397, 0),    # 144 x 128
-    (9217, 512, 509, 0),     # 128 x 128, few K steps (fp16: with fp16 activations)
+    (9217, 512, 509, 0),     # 128 x 128, fp16 activations, few K steps
     (2049, 4096, 1531, 1),   # 128 x 128, output 4 bytes off a 16-byte boundary
     (2047, 4096, 1531, 0),   # 128 x 96, one tile a CU, ragged in both directions
     (2048, 4096, 1025, 1),   # 128 x 96, one token past a tile, output 4 bytes off a 16-byte boundary
@@ -199,7 +199,8 @@ def test_int8_mat_routes_to_gemm_i8():
     (2050, 4096, 400, 0),    # 64 x 64
     (2048, 4160, 161, 1),    # 64 x 32, a ragged last K step (I % 256 = 64)
     (2047, 320, 65, 0),      # 32 x 32, K steps 1.25
-    (9216, 192, 17, 0),      # 32 x 16, I below one K step
+    (9216, 192, 17, 0),      # 64 x 48, I of one K step and a half
+    (9217, 2048, 13, 0),     # 32 x 16
     (2047, 4096, 25, 0),     # 16 x 16
     (33, 64, 11, 0),         # 32 x 16, the smallest I of the group-scaled forms
 ])

@@ -705,26 +705,29 @@ bool launch_gemv1(const int8_t* q, const float* s, const float* x, float* y, int
                   hipStream_t st) {
     // the rows per wavefront with the cheapest rounds over the chip: R rows and a fixed part of about two rows' time each.
     // Of 2, 3, 4, 6, 9 and 12 it was the fastest or within 12 % of it for 1 to 8 input rows on qkv (9) and o_proj (4).
-    // Two loads a lane (16384 inputs) leave registers for 4 and pay for one round only, where the looped kernel has too few
-    // workgroups (us, looped -> so, 1 / 2 input rows: 512 x 16384 7.7 / 11.5 -> 5.1 / 5.7; 2 rounds, 2048 x 16384, 1 row 10.0 ->
-    // 10.7)
+    // Two loads a lane (16384 inputs) leave registers for 8 and pay for one round only, where the looped kernel has too few
+    // workgroups (us, looped -> so, 1 / 2 input rows: 512 x 16384 7.7 / 11.5 -> 5.1 / 5.7, 2048 x 16384 13.3 / 17.1 -> 9.5 /
+    // 10.9)
     int best = 0;
     long cost = 0;
-    for (int R : {2, 3, 4, 6, 9, 12}) {
-        if (U > 1 && R > 4) break;
+    for (int R : {2, 3, 4, 6, U > 1 ? 8 : 9, 12}) {
+        if (U > 1 && R > 8) break;
         const long gpw = GV_WAVES / ks, wgs = ((O + R - 1) / R + gpw - 1) / gpw, e = (wgs + cus - 1) / cus * (R + 2);
         if (!best || e < cost) {
             best = R;
             cost = e;
         }
     }
-    if (U > 1 && cost > best + 2) return false;
     if constexpr (U == 1) {
         switch (best) {
             case 6: return launch_gemv1_r<NT, 6, U>(q, s, x, y, I, O, ks, st);
             case 9: return launch_gemv1_r<NT, 9, U>(q, s, x, y, I, O, ks, st);
             case 12: return launch_gemv1_r<NT, 12, U>(q, s, x, y, I, O, ks, st);
         }
+    }
+    if constexpr (U == 2) {
+        if (best == 6) return launch_gemv1_r<NT, 6, U>(q, s, x, y, I, O, ks, st);
+        if (best == 8) return launch_gemv1_r<NT, 8, U>(q, s, x, y, I, O, ks, st);
     }
     switch (best) {
         case 2: return launch_gemv1_r<NT, 2, U>(q, s, x, y, I, O, ks, st);
@@ -756,8 +759,15 @@ void launch_gemv_t(const int8_t* q, const float* s, const float* x, float* y, in
         return 256;
     }();
     if (I / 16 / ks <= 64 && launch_gemv1<NT, 1>(q, s, x, y, I, O, ks, cus, st)) return;
+    // longer parts: two chunks a lane where one round of workgroups holds the matrix, else the looped kernel, with 4
+    // wavefronts per CU (8: 4476 x 12288, 2 rows, 24.7 us, 4: 20.7)
+    const bool two = I / 16 / ks <= 128 && (O + 7) / 8 <= cus * (GV_WAVES / ks);
     if constexpr (NT <= 2) {
-        if (I / 16 / ks <= 128 && launch_gemv1<NT, 2>(q, s, x, y, I, O, ks, cus, st)) return;
+        if (two && launch_gemv1<NT, 2>(q, s, x, y, I, O, ks, cus, st)) return;
+    }
+    if (I / 16 / ks > 64 && !two) {
+        ks = 1;
+        while (ks < GV_WAVES && groups * ks < 1024 && (I / 16) % (128 * ks) == 0) ks *= 2;
     }
     const int nb = std::min(cus, groups * ks);
     const size_t lds = (size_t)NT * I * 4 + GV_WAVES * NT * GV_R * 4;
@@ -862,8 +872,9 @@ __device__ __forceinline__ float mat_unit_dot(const MatUnit<FMT>& u, const float
     return FMT == MF_F16 ? d : d * u.sc;
 }
 constexpr int GM_WAVES = 8;
+// (wavefronts a SIMD: 5 int6 rows in 4 took 130 registers left alone, 2 too many for 4 of them: 9814 x 1536 19.6 -> 16.2 us)
 template <int FMT, int NT, int R>
-__global__ void __launch_bounds__(64 * GM_WAVES) gemv_mat_kernel(const uint8_t* __restrict__ W,
+__global__ void __launch_bounds__(64 * GM_WAVES, NT == 5 ? 4 : 2) gemv_mat_kernel(const uint8_t* __restrict__ W,
                                                                  const uint8_t* __restrict__ Wh,
                                                                  const float* __restrict__ s,
                                                                  const float* __restrict__ x, float* __restrict__ y,
@@ -1049,7 +1060,10 @@ void launch_gemv_mat_t(const uint8_t* W, const uint8_t* Wh, const float* s, cons
         // each: input rows of another alignment or length take the kernel below
         constexpr bool XL = mat_xl<FMT, NT>;
         const size_t lds = (XL ? (size_t)NT * I * 4 : 0) + (size_t)GM_WAVES * NT * 4 * 6;
-        if (U / ks <= 64 && lds <= 160 * 1024 &&
+        // (one fp16 row of a matrix that leaves half the chip idle gains nothing from LDS either, and pays for the
+        // copy: 579 x 2048 3.75 us, 3.50 without)
+        const bool few = FMT == MF_F16 && NT == 1 && 2 * (((O + 1) / 2 + gpr - 1) / gpr) <= cus;
+        if (U / ks <= 64 && lds <= 160 * 1024 && !few &&
             (!XL || (I % 256 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0))) {
             int best = 0;
             long cost = 0;

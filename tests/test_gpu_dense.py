@@ -255,6 +255,7 @@ def test_gemv_unaligned_rows_time(O, I, S):
     (9216, 1536, (9216, 2048), 1, 1.2), (9216, 1536, (9216, 2048), 4, 1.2), (9216, 1536, (9216, 2048), 8, 1.2),  # 96 chunks
     (16384, 2048, (16000, 2048), 4, 1.2),                                  # 128 chunks, 2048 groups of 8 rows
     (512, 16384, (1024, 8192), 1, 1.6), (512, 16384, (1024, 8192), 2, 1.6),  # 1024 chunks: two loads a lane
+    (1856, 16384, (3712, 8192), 2, 1.3),
 ])
 def test_gemv_long_parts_time(O, I, than, S, most):
     """Rows whose parts were more than one load a lane take about as long as a matrix of as many weights whose parts were
@@ -272,10 +273,11 @@ def test_gemv_long_parts_time(O, I, than, S, most):
 
 
 @pytest.mark.parametrize("O,I", [(4000, 512), (6001, 512), (8001, 512), (12001, 512), (18001, 512), (24001, 512),
-                                 (8001, 2048), (500, 16384), (767, 16384), (1021, 16384), (130, 12288), (2000, 10240)])
+                                 (8001, 2048), (500, 16384), (767, 16384), (1021, 16384), (1300, 16384), (1801, 16384),
+                                 (2100, 16384), (130, 12288), (2000, 10240)])
 def test_gemv_every_row_group(O, I):
-    """Every number of rows a wavefront takes (2, 3, 4, 6, 9 and 12, chosen by O; at 16384 inputs 2 to 4 with two loads a
-    lane; 12288 and 10240 inputs take the looped kernel) at every number of input rows: a row has the bits of the one-row call and is within
+    """Every number of rows a wavefront takes (2, 3, 4, 6, 9 and 12, chosen by O; at 16384 inputs 2, 3, 4, 6 and 8 with two
+    loads a lane; more rows of them, 12288 and 10240 inputs take the looped kernel) at every number of input rows: a row has the bits of the one-row call and is within
     1e-5 of the exact product (fp32 sums of at most 16384 products)."""
     import torch
     import moex_amd as M

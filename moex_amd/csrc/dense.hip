@@ -1167,10 +1167,12 @@ void launch_gemm_t(const void* W, const uint8_t* Wh, const float* s, const void*
     launch_gemm_s<FMT, C, false>(W, Wh, s, X, Y, S, I, O, 1, st);
 }
 
-// A long K and few tiles: K is split over nks workgroups a tile, parts of 4096 inputs at least (so the attention's shapes never
-// split), where the shorter tiles save more than the second launch (4 us) and the parts' traffic cost, and 5 %. us, whole K in one
+// A long K and few tiles: K of more than 4096 inputs (so not the attention's shapes) is split over nks workgroups a tile, parts
+// of 2048 inputs at least, where the shorter tiles save more than the second launch (4 us) and the parts' traffic cost, and 5 %. us, whole K in one
 // workgroup -> split, int8 / fp16: 64 x 40448, 9 tokens 57 / 54 -> 13 / 12; 128 x 16384, 100 tokens 24 / 24 -> 12 / 12;
 // 2048 x 16384, 300 tokens 68 / 80 -> 47 / 62, 1100 tokens 179 / 194 -> 121 / 126; 1024 x 8192, 17 tokens 14 / 14 -> 11 / 11.
+// With parts of 4096 at least, 4936 x 10240 with 100 tokens took 51 / 54 (40 / 44 so), 64 x 6144 with 11 11 / 11 (7 / 8), 1920 x 10240
+// with 300 48 / 54 (37 / 41).
 struct GemmPick { int tile, nks; };
 GemmPick gemm_pick(int S, int I, int O, bool xh, bool split, bool f16) {
     const int cus = dense_cus();
@@ -1183,7 +1185,7 @@ GemmPick gemm_pick(int S, int I, int O, bool xh, bool split, bool f16) {
         if (t.BM * t.BN > 256 && (size_t)std::max(t.BM, t.BN) * I * 4 >= (size_t)1 << 32) continue;
         const size_t tiles = (size_t)((O + t.BM - 1) / t.BM) * ((S + t.BN - 1) / t.BN);
         if (t.one && tiles > (size_t)cus) continue;
-        for (int nks = 1; nks == 1 || (split && t.split && nks <= I / 4096 && tiles * nks <= (size_t)2 * cus); nks++) {
+        for (int nks = 1; nks == 1 || (split && t.split && I > 4096 && nks <= I / 2048 && tiles * nks <= (size_t)2 * cus); nks++) {
             float e = (float)((tiles * nks + cus - 1) / cus) * (t.us0 + t.us1 * (float)I * (1.f / 1024.f) / (float)nks) *
                           (f16 && !t.xh ? 1.15f : 1.f) + (t.xh ? 8.f + 1e-6f * (float)S * (float)I : 0.f);
             if (nks > 1) e = 1.05f * e + 4.f + 2e-6f * (float)nks * (float)S * (float)O;

@@ -345,7 +345,8 @@ def test_gemv_mat_every_row_group(O, I, fmt):
     (130, 16448, 40, 1),     # a ragged last K step in the last part, 4-byte stores
     (2047, 16384, 300, 0),   # 128 x 64 tiles
     (2048, 12352, 1100, 0),  # 128-row tiles
-    (96, 8192, 33, 0),       # two parts, the shortest K that is split
+    (96, 8192, 33, 0),       # 4 parts of 16 x 16 tiles
+    (64, 6144, 9, 1),        # 3 parts, the shortest
 ])
 def test_gemm_k_split(fmt, O, I, S, shift):
     """K split over workgroups (few tiles, a long K), the parts summed by a second kernel: against the precision model, whose

@@ -273,19 +273,27 @@ __device__ __forceinline__ int fa_pieces(int t, int pos0, int T, int nsf, int w)
     return k > nsf ? nsf : k;
 }
 // w, and the pieces n1 of one kv head: lane l counts the pieces of its own candidate, the wavefront takes the smallest
-// that fits (uniform; every wavefront of the grid finds the same)
+// that fits (uniform; every wavefront of the grid finds the same). Every workgroup does this before its first load: with up to 32
+// steps here and in fa_split_block, 65 tokens at 6000 took 46.0 us, 44.2 with as few as the chunk allows; turbo 17 at 20 000
+// 69.0, 66.2.
 __device__ __forceinline__ int fa_piece_w(int pos0, int T, int KV, int NT, int nsf, int ncu, int lane, int& n1) {
     const int total = (NT * ((2 * pos0 + T + FT) / 2) + NT * (BK - 1)) / BK;  // about the sum of n (split chunks: NT <= CUs)
     const int w0 = max(FA_MINW, (KV * total + ncu - 1) / ncu), wl = w0 + w0 * lane / 16;
+    // ceil(n / wl) as 1 + floor((n - 1 / 2) / wl), half a key tile off an exact quotient
+    const float rw = __builtin_amdgcn_rcpf((float)wl);
+    const auto pieces = [&](int x) { return min(nsf, 1 + (int)(((float)x - 0.5f) * rw)); };
+    const int nmax = (pos0 + T + BK - 1) / BK;
     int n = 0;
-    for (int p = 0; p < nsf; p++) {
-        const int c = NT - fa_first_tile(p, pos0, T, NT, wl);
-        if (!__builtin_amdgcn_ballot_w64(c > 0)) break;
-        n += c;
+    if (NT < __builtin_amdgcn_readfirstlane(pieces(nmax))) {  // by token tiles or by pieces, whichever are fewer
+        for (int t = 0; t < NT; t++) n += pieces((pos0 + min(FT * (t + 1), T) + BK - 1) / BK);
+    } else {
+        for (int p = 0; p < nsf; p++) {
+            const int c = NT - fa_first_tile(p, pos0, T, NT, wl);
+            if (!__builtin_amdgcn_ballot_w64(c > 0)) break;
+            n += c;
+        }
     }
-    // the first token tile, the shortest, has kmin pieces: 1 + floor((n - 1) / wl), half a tile off an exact quotient
-    const int nmax = (pos0 + T + BK - 1) / BK, nmin = (pos0 + min(FT, T) + BK - 1) / BK;
-    const int kmin = min(nsf, 1 + (int)(((float)nmin - 0.5f) * __builtin_amdgcn_rcpf((float)wl)));
+    const int kmin = pieces((pos0 + min(FT, T) + BK - 1) / BK);  // of the first token tile, the shortest
     const unsigned long long fit = __builtin_amdgcn_ballot_w64(KV * n <= ncu);
     int l = fit ? __builtin_ctzll(fit) : 63;
     // the longest piece: nmax / kmin where every token tile has kmin pieces, about wl where some have one more
@@ -322,7 +330,14 @@ __device__ __forceinline__ bool fa_split_block(int b, int pos0, int T, int KV, i
     kvh = k / n1;
     k -= kvh * n1;
     const int t0 = lane < nsf ? fa_first_tile(lane, pos0, T, NT, w) : NT;  // of piece lane
-    for (piece = 0;; piece++) {
+    const int all = __builtin_popcountll(__builtin_amdgcn_ballot_w64(t0 == 0));  // pieces that every token tile has
+    if (k < all * NT) {
+        piece = __builtin_amdgcn_readfirstlane((int)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)NT)));
+        tile = k - piece * NT;
+        return true;
+    }
+    k -= all * NT;
+    for (piece = all;; piece++) {
         const int t = __builtin_amdgcn_readlane(t0, piece);
         if (k < NT - t) {
             tile = t + k;

@@ -214,6 +214,7 @@ def _pieces(pos0, T, cus):
     (0, 65, 256), (300, 129, 256), (1500, 400, 256), (6000, 1024, 256),  # half a full grid: the last size that splits
     (6000, 1025, 256),                                                   # the first that runs in pairs
     (20000, 213, 104), (3000, 600, 304), (33000, 1000, 8),               # other chip sizes; one too small to split on
+    (33000, 70, 256), (32000, 129, 256), (33000, 65, 40),                # fewer token tiles than pieces a tile
     (100, 300, 256), (150, 400, 256), (200, 213, 256),                   # pieces of the heavier tiles only: worth it in one
     (32768, 700, 256), (7000, 768, 256), (32768, 529, 256),              # fewer pieces than CUs, as long within a few percent
 ])

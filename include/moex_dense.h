@@ -11,7 +11,8 @@
  * GEMM (moex_gemm_i8 with S > 8, moex_gemm when it takes the GEMM), which takes up to two per-(device, stream)
  * workspaces: the larger tiles read X rounded to fp16 from one of S * I * 2 bytes (on 256 CUs the attention's qkv from 513
  * rows on, fp16 also 193 to 384, and o from 1025 rows on but for 1537 to 2304, fp16 2049 to 2176), and a product of I > 4096
- * whose tiles leave the chip idle splits K and keeps fp32 partial sums in one of parts * S * O * 4 bytes (parts <= I / 2048, tiles * parts <= 2 * CUs).
+ * whose tiles leave the chip idle splits K and keeps fp32 partial sums in one of parts * S * O * 4 bytes (parts <= I /
+ * 2048, tiles * parts <= 2 * CUs).
  * Both are allocated on first use, grown for larger sizes and kept until the process ends. While one cannot be had (the
  * stream is being captured before an eager call of that size, or there is no memory) the call runs without it: another
  * tile, slower, with the same rounding of X and the K sums in another fp32 order, so the results agree with the eager

@@ -424,24 +424,29 @@ template <int N> __device__ __forceinline__ void gemm_vm_wait() { asm volatile("
 // hardware takes as they are. With 4-byte stores wherever O or Y was not a multiple of 16 bytes, a line was written in four
 // passes, and four scale loads a lane cost an int8 tile with a short K as much as its outputs (us, 4-byte accesses -> so:
 // 11925 x 320, 1625 tokens int8 59.0 -> 42.7, fp16 65.2 -> 40.0; 11971 x 1088, 389 tokens fp16 37.9 -> 29.9; 6722 x 128, 1005
-// tokens int8 26.1 -> 16.5)
+// tokens int8 26.1 -> 16.5). inside (uniform): the whole tile is.
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ f32x4u load4(const float* p, int n) {
-    if (n >= 4) return *reinterpret_cast<const f32x4u*>(p);
+__device__ __forceinline__ f32x4u load4(const float* p, int n, bool inside) {
+    if (inside || n >= 4) return *reinterpret_cast<const f32x4u*>(p);
     f32x4u v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int e = 0; e < 3; e++)
         if (e < n) v[e] = p[e];
     return v;
 }
-__device__ __forceinline__ void store4(float* p, float4_t v, int n) {
-    if (n >= 4) {
+__device__ __forceinline__ void store4(float* p, float4_t v, int n, bool inside) {
+    if (inside) {
         *reinterpret_cast<f32x4u*>(p) = v;
-        return;
-    }
+    } else {
+        asm volatile("");  // keeps the two stores apart: merged, the branch is taken lane by lane, 1 to 2 % of a small call
+        if (n >= 4) {
+            *reinterpret_cast<f32x4u*>(p) = v;
+        } else {
 #pragma unroll
-    for (int e = 0; e < 3; e++)
-        if (e < n) p[e] = v[e];
+            for (int e = 0; e < 3; e++)
+                if (e < n) p[e] = v[e];
+        }
+    }
 }
 template <class C, class T>
 using weight_ptr = std::conditional_t<C::XH, const T*, const T* __restrict__>;
@@ -625,6 +630,7 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
         }
     }
     if (SPLIT) Y += (size_t)blockIdx.y * S * O;
+    const bool inside = o0 + C::BM <= O;  // uniform
     // acc[i][j] element e: weight row wr + 16 i + 4 g + e, token wt + 16 j + m16
     if constexpr (C::KW == 1) {
 #pragma unroll
@@ -632,12 +638,12 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
             const int o = o0 + wr + 16 * i + 4 * g;
             if (o >= O) continue;
             f32x4u sc = {1.f, 1.f, 1.f, 1.f};
-            if constexpr (FMT == MF_I8 && !SPLIT) sc = load4(s + o, O - o);
+            if constexpr (FMT == MF_I8 && !SPLIT) sc = load4(s + o, O - o, inside);
 #pragma unroll
             for (int j = 0; j < C::WN; j++) {
                 const int t = s0 + wt + 16 * j + m16;
                 if (t >= S) continue;
-                store4(Y + (size_t)t * O + o, acc[i][j] * sc, O - o);
+                store4(Y + (size_t)t * O + o, acc[i][j] * sc, O - o, inside);
             }
         }
     } else {
@@ -662,8 +668,8 @@ __global__ void __launch_bounds__(512, C::WPE) gemm_tile_kernel(weight_ptr<C, vo
                 a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
             }
             f32x4u v = {a.x, a.y, a.z, a.w};
-            if constexpr (FMT == MF_I8 && !SPLIT) v *= load4(s + o, O - o);
-            store4(Y + (size_t)t * O + o, v, O - o);
+            if constexpr (FMT == MF_I8 && !SPLIT) v *= load4(s + o, O - o, inside);
+            store4(Y + (size_t)t * O + o, v, O - o, inside);
         }
     }
 }

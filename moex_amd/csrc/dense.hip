@@ -397,9 +397,9 @@ __device__ __forceinline__ void wstage_widen(const WStage& w, bool ok, uint32_t 
 // Measured (graph-replayed calls over 300 MB of rotating weights, us; before: 128 x 128 tiles on 4 wavefronts or 4 + 4
 // split roles, an fp16 rounding launch for every call, K split over workgroups with a reduction launch), int8:
 //   tokens              9          64         300        512        1024       2048
-//   qkv  9216 x 2048    21.0->10.4 32.7->17.1 47.1->31.2 50.3->43.6 73.8->57.9 139->90.2 (857 TFLOPS)
-//   o    2048 x 4096    17.9->10.1 24.9->12.1 34.4->23.8 39.0->26.8 53.3->38.2 79.6->53.8 (638 TFLOPS)
-// int4 at 300 tokens: qkv 45.3 -> 32.3, o 31.8 -> 23.6; fp16 at 2048: 136 -> 84.4, 81.6 -> 59.2.
+//   qkv  9216 x 2048    21.1->10.4 33.0->16.1 47.9->31.7 50.8->39.2 74.0->58.7 140->90.6 (853 TFLOPS)
+//   o    2048 x 4096    17.9->10.1 25.0->11.9 34.6->23.3 38.9->25.6 53.4->36.1 79.5->53.8 (639 TFLOPS)
+// int4 at 300 tokens: qkv 45.4 -> 32.2, o 31.9 -> 23.5; fp16 at 2048: 137 -> 85.8, 81.8 -> 58.9.
 template <int WM_, int WN_, int GM_, int GN_, int KW_, int BKU_, int PD_, bool XH_ = false, int WPE_ = 2>
 struct GemmTile {
     static constexpr int WM = WM_, WN = WN_, GM = GM_, GN = GN_, KW = KW_, BKU = BKU_, PD = PD_;

@@ -417,14 +417,14 @@ def test_gemm_half_full_grid_time():
         x, y = torch.randn((S, I), device="cuda"), torch.empty((S, O), device="cuda")
         us.append(_graph_us(lambda st: M.gemm(m, x, y, S, I, O, st), n=20))
     print(f"o_proj 1100 tokens {us[0]:.2f} us, 1536 {us[1]:.2f} us", flush=True)
-    assert us[0] <= 1.02 * us[1]
+    assert us[0] <= 1.03 * us[1]
 
 
 @pytest.mark.parametrize("fmt,O,I,S,than", [("i8", 64, 40448, 9, (64, 4096, 9)), ("q6", 64, 40448, 40, (64, 4096, 40)),
                                             ("f16", 2048, 16384, 300, (2048, 4096, 300))])
 def test_gemm_long_k_time(fmt, O, I, S, than):
     """A long K costs a matrix of few tiles a second launch and its share of the chip, not a K step after the other (measured
-    1.6 to 2.6 times the product of 4096 inputs, 3.2 to 8.4 times with all of K in one workgroup), so at most 2.9 times."""
+    1.4 to 2.3 times the product of 4096 inputs, 3.2 to 8.4 times with all of K in one workgroup), so at most 2.9 times."""
     import torch
     import moex_amd as M
     from tests.test_gpu_dense import _graph_us
